@@ -288,6 +288,8 @@ void launch_force(const Geo& g, const DevTables& t, const double* Psi, const dou
                   int mode, double jxwChild, const double* jxwParent, double* force, int colour,
                   hipStream_t s);
 void launch_zero_rows(int64_t N, int B, double* X, const unsigned char* mask, hipStream_t s);
+// X = 0 on the rows of the mesh's boundary nodes
+void launch_zero_boundary(const Geo& g, int B, double* X, hipStream_t s);
 // MINRES
 // nq = 2: partial also holds (D r)^2 partials at row offset nblk (into Q2)
 void launch_minres_start(int B, int nblk, const double* partial, const double* negEig,

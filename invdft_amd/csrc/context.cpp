@@ -271,7 +271,7 @@ struct idft_ctx {
     }
     launch_right_mult(t.N, b, a, small2.p, out, ns, beta, s);
   }
-  void zero_boundary(double* v, int b) { launch_zero_rows(t.N, b, v, bnd.p, s); }
+  void zero_boundary(double* v, int b) { launch_zero_boundary(g, b, v, s); }
 
   // ------------------------------------------------------ Hamiltonian
   // Operator of the current v_eff: the quadrature weights w = v_eff JxW
