@@ -262,10 +262,21 @@ void launch_loss(int64_t nQ, int nq, const double* rho, const double* rhoT, cons
                  const double* veff, const double* jxw, double* u, double* partial,
                  hipStream_t s);
 constexpr int kLossBlocks = 256;
-// out[cell][k] = sum_q wq[cell][q] A_{i_k}(q) B_{j_k}(q), pairs (i_k, j_k)
-void launch_pair_quad(const Geo& g, const DevTables& t, const double* A, const double* Bv, int B,
-                      const int* pairs, int np, const double* wq, int64_t wstride, double* out,
-                      hipStream_t s);
+// Quadrature operator T = N^T diag(W) N Bv over the wb columns of Bv (row length
+// ldb) by sum-factorised cell products into Yc (cell_scratch_elems(g, wb)
+// elements) and a node gather; W per cell wstride apart (0: one cell's weights
+// for all).  T2 != nullptr stores T (row length ldt); np pairs (<= 256) give
+// out[k] = sum_n asc[n] A[n][i_k] T[n][j_k] (A of row length lda; asc may be null).
+void launch_quad_pairs(const Geo& g, const double* W, int64_t wstride, const double* Bv, int ldb,
+                       int wb, double* Yc, const double* A, int lda, const double* asc, double* T2,
+                       int ldt, const int* pairs, int np, DevBuf<double>& partial, double* out,
+                       hipStream_t s);
+// Y = S T (+ column scale cc, and psi's node scale q, with rhs) + psi C for a C
+// with few entries: coef[e] of column i at e in [list[i], list[i + 1]), its row
+// (psi's column) list[B + 1 + e].
+void launch_pair_combine(int64_t N, int B, bool rhs, const double* T, const double* S,
+                         const double* q, const double* psi, const double* cc, const double* coef,
+                         const int* list, int nnz, double* Y, hipStream_t s);
 void launch_copy_cols(int64_t N, int Bs, int off, int Bd, const double* src, double* dst,
                       hipStream_t s);
 // dst[n][k] = src[n][idx[k]], k < Bd (gather) / dst[n][idx[k]] = src[n][k], k < Bs (scatter)
@@ -279,9 +290,6 @@ void launch_mul_q(int64_t nQ, int nq, const double* u, const double* jxw, double
 // partial[blk][k] = sum_n w[n] X[n][i_k] Y[n][j_k] (w may be null)
 int launch_pairdot_partial(int64_t N, int B, const double* X, const double* Y, const double* w,
                            const int* pairs, int np, double* partial, hipStream_t s);
-// Y += N^T diag(wq) N X over the cells of one colour
-void launch_quad_operator(const Geo& g, const DevTables& t, const double* X, int B,
-                          const double* wq, double* Y, int colour, hipStream_t s);
 // force[child node] += int N^child sum_j Psi_j P_j over one colour; mode 0 = child
 // Gauss points (weight jxwChild), mode 1 = parent Gauss points (weights jxwParent[q])
 void launch_force(const Geo& g, const DevTables& t, const double* Psi, const double* P, int B,

@@ -112,8 +112,8 @@ struct idft_ctx {
   idft_stats st{};
   AdjointState adj;
   MinresWork<double> mw64;
-  DevBuf<double> mst, mx, mtmp, mnegc, mcell;
-  DevBuf<int> mflags, msel;
+  DevBuf<double> mst, mx, mtmp, mnegc, mcell, pairCoef;
+  DevBuf<int> mflags, msel, pairList;
   idft_mv mvPsi, mvX;
 
   // rocBLAS handle on s (created on first use), for the Gram and X Q products
@@ -714,16 +714,39 @@ struct idft_ctx {
   }
 
   // ----------------------------------------------------- adjoint problem
-  std::vector<double> pair_quad_sum(const double* A, const double* Bv, int b, const double* wq,
-                                    int64_t wstride) {
+  // v_k = sum_n asc[n] A[n][i_k] (R Bv)[n][j_k] over the adjoint's pairs, with
+  // R = N^T diag(wq) N the quadrature operator (wstride 0: the same weights in
+  // every cell): the pairs' quadrature sums sum_q wq A_i B_j.  T2 (optional)
+  // receives R Bv.
+  std::vector<double> quad_pairs(const double* A, const double* asc, const double* Bv, int b,
+                                 const double* wq, int64_t wstride, double* T2) {
     const int np = (int)adj.pairs.size() / 2;
-    if (np == 0) return {};
-    partial.resize((size_t)t.ncell * np);
+    if (np == 0 && !T2) return {};
+    // columns per pass: all, unless the cell kernel's width or the 32-bit index
+    // of the cell scratch bounds them
+    const int64_t fit = ((int64_t)0xffffffffLL - 1) / cell_scratch_elems(g, 1);
+    const int w = (int)std::min<int64_t>(std::min(b, kMaxCols), std::max<int64_t>(fit, 1));
+    const bool fused = w == b && np <= 256;
+    if (!fused && !T2 && np) {
+      T2buf.resize(NB(b));
+      T2 = T2buf.p;
+    }
     small.resize(std::max(np, 16));
-    launch_pair_quad(g, dt, A, Bv, b, adj.dpairs.p, np, wq, wstride, partial.p, s);
-    launch_sum_partials((int)t.ncell, np, partial.p, small.p, s);
+    Yc64.resize(cell_scratch_elems(g, w));
+    for (int j = 0; j < b; j += w) {
+      const int wj = std::min(w, b - j);
+      launch_quad_pairs(g, wq, wstride, Bv + j, b, wj, Yc64.p, A, b, asc, T2 ? T2 + j : nullptr, b,
+                        adj.dpairs.p, fused ? np : 0, partial, small.p, s);
+    }
+    if (!fused)  // pairs in runs of the node-dot kernel's 256
+      for (int k = 0; k < np; k += 256) {
+        const int m = std::min(256, np - k);
+        partial.resize((size_t)1024 * m);
+        const int nb = launch_pairdot_partial(t.N, b, A, T2, asc, adj.dpairs.p + 2 * k, m, partial.p, s);
+        launch_sum_partials(nb, m, partial.p, small.p + k, s);
+      }
     std::vector<double> out(np);
-    small.download(out.data(), np, s);
+    if (np) small.download(out.data(), np, s);
     sync();
     return out;
   }
@@ -731,7 +754,7 @@ struct idft_ctx {
   void compute_mu(const std::vector<double>& occv) {
     const int Bb = adj.B;
     if (!adj.havePairQ) {
-      adj.pairQ = pair_quad_sum(adj.psi->p(), adj.psi->p(), Bb, adj.uJxW.p, t.nq);
+      adj.pairQ = quad_pairs(adj.psi->p(), nullptr, adj.psi->p(), Bb, adj.uJxW.p, t.nq, nullptr);
       adj.havePairQ = true;
     }
     const std::vector<double>& v = adj.pairQ;
@@ -740,6 +763,36 @@ struct idft_ctx {
       const int i = adj.pairs[2 * k], j = adj.pairs[2 * k + 1];
       adj.Mu[(size_t)i * Bb + j] += 2.0 * occv[i] * v[k];
     }
+  }
+  // Column lists of a b x b matrix C (row-major, column i combines psi's columns
+  // k with C[k][i]) that is zero outside the adjoint's pairs, either way round;
+  // uploaded for k_pair_combine.  Returns the entry count, or -1 if a dense
+  // product is the better one: more than kSparsePairs entries per column on
+  // average.
+  static constexpr int kSparsePairs = 8;
+  int pair_lists(const std::vector<double>& C, int b) {
+    std::vector<char> used((size_t)b * b, 0);
+    int nnz = 0;
+    for (size_t k = 0; k + 1 < adj.pairs.size(); k += 2) {
+      const int i = adj.pairs[k], j = adj.pairs[k + 1];
+      for (const size_t e : {(size_t)i * b + j, (size_t)j * b + i})
+        if (!used[e] && C[e] != 0.0) { used[e] = 1; ++nnz; }
+    }
+    if (nnz > kSparsePairs * b || b > 2 * kMaxCols) return -1;
+    std::vector<double> coef;
+    std::vector<int> list((size_t)b + 1, 0), rows;
+    for (int i = 0; i < b; ++i) {
+      for (int k = 0; k < b; ++k)
+        if (used[(size_t)k * b + i]) {
+          coef.push_back(C[(size_t)k * b + i]);
+          rows.push_back(k);
+        }
+      list[i + 1] = (int)coef.size();
+    }
+    list.insert(list.end(), rows.begin(), rows.end());
+    if (nnz) pairCoef.upload(coef.data(), coef.size(), s);
+    pairList.upload(list.data(), list.size(), s);
+    return nnz;
   }
 
   void update_input_psi(idft_mv* psi, const double* occv, const double* u_dev_or_null,
@@ -780,40 +833,26 @@ struct idft_ctx {
     if (x && x->ncols != b) throw Error(IDFT_EINVAL, "block size mismatch");
     A.x = x;
     const double* psi = A.psi->p();
-    // T2 = R psi, R = N^T diag(u JxW) N assembled over the cells
+    // T2 = R psi, R = N^T diag(u JxW) N, and the pairs' quadrature sums
+    // sum_q u JxW psi_i psi_j = psi_i . (R psi)_j
     T2buf.resize(NB(b));
     double* T2 = T2buf.p;
-    launch_lincomb<double>(t.N, b, T2, 0.0, nullptr, 0.0, nullptr, nullptr, 0.0, nullptr, nullptr, s);
-    for (int colour = 0; colour < 8; ++colour)
-      launch_quad_operator(g, dt, psi, b, A.uJxW.p, T2, colour, s);
-    // the pairs' quadrature sums sum_q u JxW psi_i psi_j = psi_i . (R psi)_j
-    // (R assembled from the same quadrature), before T2's boundary rows are
-    // cleared; more pairs than the node-dot kernel takes (256) are summed at
-    // the quadrature points by compute_mu instead
-    const int np = (int)A.pairs.size() / 2;
-    A.havePairQ = false;
-    if (np > 0 && np <= 256) {
-      partial.resize((size_t)1024 * np);
-      small.resize(std::max(np, 16));
-      const int nb = launch_pairdot_partial(t.N, b, psi, T2, nullptr, A.dpairs.p, np, partial.p, s);
-      launch_sum_partials(nb, np, partial.p, small.p, s);
-      A.pairQ.resize(np);
-      small.download(A.pairQ.data(), np, s);
-      sync();
-      A.havePairQ = true;
-    } else if (np == 0) {
-      A.pairQ.clear();
-      A.havePairQ = true;
-    }
+    A.pairQ = quad_pairs(psi, nullptr, psi, b, A.uJxW.p, t.nq, T2);
+    A.havePairQ = true;
     compute_mu(A.occ);
-    // rhs = -2 sqrt(M) psi Mu   (column i: -2 sum_k Mu[k][i] M^{1/2} psi_k)
+    // rhs = 4 f M^{-1/2} R psi - 2 sqrt(M) psi Mu   (column i: sum_k Mu[k][i] psi_k)
     std::vector<double> C((size_t)b * b);
     for (size_t k = 0; k < C.size(); ++k) C[k] = -2.0 * A.Mu[k];
-    right_mult(psi, C, rhs, b, sqrtM.p, 0.0);
-    // rhs += 4 f M^{-1/2} R psi
-    zero_boundary(T2, b);
-    launch_lincomb<double>(t.N, b, rhs, 1.0, T2, 1.0, A.docc4.p, nullptr, 0.0, nullptr, invSqrtM.p, s);
-    zero_boundary(rhs, b);
+    const int nnz = pair_lists(C, b);
+    if (nnz >= 0) {
+      launch_pair_combine(t.N, b, true, T2, S.p, sqrtM.p, psi, A.docc4.p, pairCoef.p, pairList.p,
+                          nnz, rhs, s);
+    } else {
+      right_mult(psi, C, rhs, b, sqrtM.p, 0.0);
+      zero_boundary(T2, b);
+      launch_lincomb<double>(t.N, b, rhs, 1.0, T2, 1.0, A.docc4.p, nullptr, 0.0, nullptr, invSqrtM.p, s);
+      zero_boundary(rhs, b);
+    }
     sync();
   }
 
@@ -858,7 +897,7 @@ struct idft_ctx {
   }
 
   std::vector<double> dot_quad_wise(const double* v1, const double* v2, int b) {
-    return pair_quad_sum(v1, v2, b, jxw.p, 0);
+    return quad_pairs(v1, nullptr, v2, b, jxw.p, 0, nullptr);
   }
 
   void distribute_x() {
@@ -867,11 +906,13 @@ struct idft_ctx {
     const int b = A.B;
     double* x = A.x->p();
     const double* psi = A.psi->p();
-    launch_lincomb<double>(t.N, b, x, 0.0, x, 1.0, nullptr, nullptr, 0.0, nullptr, invSqrtM.p, s);
-    zero_boundary(x, b);
+    // x is M^{-1/2} x~ (S, zero on the boundary) from here on; the pass that
+    // stores it comes last, with the null-space correction
     const int np = (int)A.pairs.size() / 2;
     std::vector<double> dot;
     if (d.gradient_mode == IDFT_GRADIENT_EXACT) {
+      launch_lincomb<double>(t.N, b, x, 0.0, x, 1.0, nullptr, nullptr, 0.0, nullptr, invSqrtM.p, s);
+      zero_boundary(x, b);
       partial.resize((size_t)1024 * std::max(np, 1));
       small.resize(std::max(np, 16));
       const int nb = launch_pairdot_partial(t.N, b, x, psi, Mdiag.p, A.dpairs.p, np, partial.p, s);
@@ -880,7 +921,8 @@ struct idft_ctx {
       small.download(dot.data(), np, s);
       sync();
     } else {
-      dot = dot_quad_wise(x, psi, b);
+      // sum_q JxW x_i psi_j = x_i . (M psi)_j, M the consistent mass
+      dot = quad_pairs(x, S.p, psi, b, jxw.p, 0, nullptr);
     }
     compute_mu(std::vector<double>(b, 1.0));
     double sumD = 0.0, etaR = 0.0;
@@ -898,7 +940,18 @@ struct idft_ctx {
       if (i == j) corr += dFi * eta;
       C[(size_t)j * b + i] += -dot[k] + corr;
     }
-    right_mult(psi, C, x, b, nullptr, 1.0);
+    const bool exact = d.gradient_mode == IDFT_GRADIENT_EXACT;
+    const int nnz = exact ? -1 : pair_lists(C, b);
+    if (nnz >= 0) {
+      launch_pair_combine(t.N, b, false, x, S.p, nullptr, psi, nullptr, pairCoef.p, pairList.p, nnz,
+                          x, s);
+    } else {
+      if (!exact) {
+        launch_lincomb<double>(t.N, b, x, 0.0, x, 1.0, nullptr, nullptr, 0.0, nullptr, invSqrtM.p, s);
+        zero_boundary(x, b);
+      }
+      right_mult(psi, C, x, b, nullptr, 1.0);
+    }
     sync();
   }
 
@@ -1327,8 +1380,9 @@ struct idft_ctx {
   void integrate_parent(const double* w, double* f) {
     DevBuf<double> ones(t.N);
     fill_ones(ones.p, t.N);
-    launch_lincomb<double>(t.N, 1, f, 0.0, nullptr, 0.0, nullptr, nullptr, 0.0, nullptr, nullptr, s);
-    for (int colour = 0; colour < 8; ++colour) launch_quad_operator(g, dt, ones.p, 1, w, f, colour, s);
+    Yc64.resize(cell_scratch_elems(g, 1));
+    launch_quad_pairs(g, w, t.nq, ones.p, 1, 1, Yc64.p, nullptr, 1, nullptr, f, 1, nullptr, 0, partial,
+                      nullptr, s);
   }
   void fill_ones(double* v, int64_t n) {
     std::vector<double> h((size_t)n, 1.0);

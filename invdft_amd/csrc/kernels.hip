@@ -71,6 +71,19 @@ __device__ inline double block_sum_contig(const double* __restrict__ v, int n, d
   return block_total<NT>((s0 + s1) + (s2 + s3), red);
 }
 
+// Sums over k < per of red[k B + c] into red[c] for every c < B, by the
+// threads tid = k B + c (off = tid / B, tid < per B): a tree of ceil(log2 per)
+// steps in a fixed order, all threads call it.
+__device__ inline void tree_cols(double* red, int per, int B, int tid, int off) {
+  __syncthreads();
+  for (int n = per; n > 1;) {
+    const int h = (n + 1) / 2;
+    if (off < n - h) red[tid] += red[tid + h * B];
+    __syncthreads();
+    n = h;
+  }
+}
+
 // Work-group size of the per-column reductions of long partial rows (cell
 // dots, gather partials, Gram partials): 16 waves, about 12 values per thread
 // for the 12-16 k values of a column.
@@ -766,10 +779,14 @@ __device__ inline T eo_unsplit(const Pack<T, VC> (&xp)[(C + 1) / 2], const Pack<
   }
 }
 
-template <typename T, typename TV, int P, int CG, int VC, bool XN>
+// KIN = false: the potential chain alone on the unscaled input (S unused):
+// Yc = Lq^T diag(w_e) Lq X_e, the quadrature operator of a weight (stages 1 and
+// 4 to 8).  wstride: the weights' step from cell to cell (0: the same weights
+// in every cell); ldx: the row length of X (B, or more for a block of columns).
+template <typename T, typename TV, int P, int CG, int VC, bool XN, bool KIN>
 __global__ __launch_bounds__(kThreads) void k_cell_sf(Geo g, T hq, const T* __restrict__ W,
-                                                      const T* __restrict__ S,
-                                                      const TV* __restrict__ X,
+                                                      uint32_t wstride, const T* __restrict__ S,
+                                                      const TV* __restrict__ X, uint32_t ldx,
                                                       const double* __restrict__ xn,
                                                       const double* __restrict__ xcol,
                                                       T* __restrict__ Yc, int B,
@@ -791,8 +808,8 @@ __global__ __launch_bounds__(kThreads) void k_cell_sf(Geo g, T hq, const T* __re
   // SWZ: D unpadded (QS = Q = 8), entry (c, y, x) at slot x ^ y of its line
   constexpr bool SWZ = sizeof(T) == 8 && Q == 8;
   constexpr int QS = SWZ ? Q : QP;
-  __shared__ __align__(16) pk rA[N2 * N1P * NV];
-  __shared__ __align__(16) pk rBD[cmax(N2 * N1P, N1 * Q * QS) * NV];
+  __shared__ __align__(16) pk rA[KIN ? N2 * N1P * NV : 1];
+  __shared__ __align__(16) pk rBD[cmax(KIN ? N2 * N1P : 0, N1 * Q * QS) * NV];
   pk* const rB = rBD;
   // Byte offsets into D of entry (c, y, x), column pack jv, from a per-item
   // base and the one index that is a compile-time constant at the access
@@ -836,7 +853,7 @@ __global__ __launch_bounds__(kThreads) void k_cell_sf(Geo g, T hq, const T* __re
   const int bw = min(CG, B - c0);
   const int tid = threadIdx.x;
   const uint32_t cx = e % nc, cy = (e / nc) % nc, cz = e / (nc * nc);
-  const T* we = W + e * (uint32_t)(Q2 * Q);
+  const T* we = W + (size_t)e * wstride;
   // the column scales of this thread's columns (every item of a thread has
   // column pack jv = tid % NV, since kThreads is a multiple of NV), loaded
   // first: a later load would make their first use wait for the weights too
@@ -873,26 +890,28 @@ __global__ __launch_bounds__(kThreads) void k_cell_sf(Geo g, T hq, const T* __re
     // nodes at immediate offsets (the X rows B apart).  All loads of the line
     // are issued before the first product (the node scale xn is a
     // compile-time choice, so no branch separates them).
-    const T* Sp = S + n0;
+    const T* Sp = KIN ? S + n0 : nullptr;
 #pragma unroll
     for (int u = 0; u < VC; ++u) {
       const int j = jv * VC + u;
       if (j < bw) {
-        const TV* Xp = X + (size_t)n0 * ub + (uint32_t)(c0 + j);
+        const TV* Xp = X + (size_t)n0 * ldx + (uint32_t)(c0 + j);
         const double xc = xcl[u];
         T sv[N1];
         TV xv[N1];
         double nv[N1];
 #pragma unroll
         for (int a = 0; a < N1; ++a) {
-          sv[a] = Sp[a];
-          xv[a] = Xp[(size_t)a * ub];
+          if constexpr (KIN) sv[a] = Sp[a];
+          xv[a] = Xp[(size_t)a * ldx];
           if constexpr (XN) nv[a] = xn[n0 + a];
           else nv[a] = 1.0;
         }
 #pragma unroll
         for (int a = 0; a < N1; ++a) {
-          if constexpr (std::is_same<T, TV>::value) {
+          if constexpr (!KIN) {
+            v[a].v[u] = (T)xv[a];
+          } else if constexpr (std::is_same<T, TV>::value) {
             T x = sv[a] * xv[a];
             if constexpr (XN) x *= (T)nv[a];
             if (xcol) x *= (T)xc;
@@ -910,6 +929,7 @@ __global__ __launch_bounds__(kThreads) void k_cell_sf(Geo g, T hq, const T* __re
       }
     }
     eo_split(v, keep_p[ki], keep_m[ki]);
+    if constexpr (!KIN) continue;
     eo_out<N1, T, VC>(
         [&](auto i, pk& s, pk& d) { eo_row<T, TM, IDFT_IC(i)>(keep_p[ki], keep_m[ki], s, d, eo); },
         [&](auto a2, const pk& r) { rA[(ln * N1P + IDFT_IC(a2)) * NV + jv] = r; });
@@ -917,6 +937,7 @@ __global__ __launch_bounds__(kThreads) void k_cell_sf(Geo g, T hq, const T* __re
         [&](auto i, pk& s, pk& d) { eo_row<T, TD, IDFT_IC(i)>(keep_p[ki], keep_m[ki], s, d, eo); },
         [&](auto a2, const pk& r) { rB[(ln * N1P + IDFT_IC(a2)) * NV + jv] = r; });
   }
+  if constexpr (KIN) {
   __syncthreads();
   // stage 2: y lines (c, a) of the kinetic chain, in place:
   // k1 = M ka (over ka), k2 = D ka + M kb (over kb)
@@ -962,6 +983,7 @@ __global__ __launch_bounds__(kThreads) void k_cell_sf(Geo g, T hq, const T* __re
         [&](auto c2, const pk& r) { rA[((IDFT_IC(c2) * N1 + b) * N1P + a) * NV + jv] = r; });
   }
   __syncthreads();
+  }
   // stage 4: x lines of the potential chain from the kept input:
   // t1[c][b][qx] = Lq x (over k2, which stage 3 has consumed)
 #pragma unroll
@@ -1052,10 +1074,12 @@ __global__ __launch_bounds__(kThreads) void k_cell_sf(Geo g, T hq, const T* __re
     eo_out<N1, T, VC>([&](auto i, pk& s, pk& d) { eo_row<T, TLt, IDFT_IC(i)>(vp, vm, s, d, eo); },
                       [&](auto a, const pk& r) {
                         constexpr int A = IDFT_IC(a);
-                        const pk kin = rA[(ln * N1P + A) * NV + jv];
+                        pk kin;
+                        if constexpr (KIN) kin = rA[(ln * N1P + A) * NV + jv];
 #pragma unroll
                         for (int u = 0; u < VC; ++u) {
-                          const T y = hq * kin.v[u] + r.v[u];
+                          T y = r.v[u];
+                          if constexpr (KIN) y = hq * kin.v[u] + y;
                           if (jv * VC + u < bw) yp[(size_t)A * ub + u] = y;
                           if constexpr (XN) {
                             if (dotp)
@@ -1284,6 +1308,71 @@ __global__ __launch_bounds__(kThreads) void k_cell_gather(
   }
 }
 
+// Node sums of the quadrature operator's cell products (k_cell_sf without the
+// kinetic chain) and, while a node's row is at hand, the pair sums
+//   partial[k gridDim.x + block] = sum over the block's nodes of
+//                                  asc[n] A[n][i_k] T[n][j_k],  k < np <= 256,
+// T = sum_e Yc optionally stored (T2, row length ldt).  Where A's node scale
+// asc is 0 (the boundary) A counts as 0, whatever it holds.
+// Bound by HBM: Yc, A and T2 once.  The rows of A and T of a chunk of
+// per = 256 / (wb / VW) nodes go through LDS, because a pair's two columns sit in
+// different lanes; thread t sums pair t % np over every (256 / np)-th node of
+// the chunk, so 8 to 256 pairs keep most lanes busy.  It replaces an
+// interpolation of both blocks to the quadrature points per pair (1.80 ms for 14
+// pairs at 121^3 nodes x 12 columns) and 8 launches of coloured cells
+// (2.18 ms for the operator).
+template <int P, int VW>
+__global__ __launch_bounds__(kThreads) void k_quad_gather(
+    Geo g, FastDiv divN1, uint32_t wb, uint32_t R, const double* __restrict__ Yc,
+    const double* __restrict__ A, uint32_t lda, const double* __restrict__ asc,
+    double* __restrict__ T2, uint32_t ldt, const int* __restrict__ pairs, uint32_t np,
+    double* __restrict__ partial) {
+  __shared__ double ta[kThreads * VW], tb[kThreads * VW], red[kThreads];
+  const uint32_t nb = wb / VW, tid = threadIdx.x, per = kThreads / nb;
+  const uint32_t jg = tid % nb, off = tid / nb, j0 = jg * VW;
+  const uint32_t nn = (uint32_t)g.N;
+  const uint32_t nsl = np ? kThreads / np : 1, sl = np ? tid / np : 0;
+  uint32_t pi = 0, pj = 0;
+  if (np && sl < nsl) {
+    pi = pairs[2 * (tid % np)];
+    pj = pairs[2 * (tid % np) + 1];
+  }
+  double acc = 0.0;
+  const uint32_t ngroups = (nn + R * per - 1) / (R * per);
+  for (uint32_t grp = blockIdx.x; grp < ngroups; grp += gridDim.x)
+    for (uint32_t rr = 0; rr < R; ++rr) {
+      const uint32_t n0 = (grp * R + rr) * per;  // uniform: every thread reaches the barriers
+      if (n0 >= nn) break;
+      const uint32_t cnt = min(per, nn - n0), n = n0 + off;
+      if (off < cnt) {
+        double sum[VW];
+        gather_node<double, P, VW>(g, divN1, wb, n, Yc, j0, sum);
+        if (T2) vstore<double, VW>(T2 + (size_t)n * ldt + j0, sum);
+        if (np) {
+          double av[VW];
+          vload<double, VW>(A + (size_t)n * lda + j0, av);
+          const double sc = asc ? asc[n] : 1.0;
+#pragma unroll
+          for (int v = 0; v < VW; ++v) {
+            ta[off * wb + j0 + v] = sc == 0.0 ? 0.0 : sc * av[v];
+            tb[off * wb + j0 + v] = sum[v];
+          }
+        }
+      }
+      if (np) {
+        __syncthreads();
+        if (sl < nsl)
+          for (uint32_t m = sl; m < cnt; m += nsl) acc += ta[m * wb + pi] * tb[m * wb + pj];
+        __syncthreads();
+      }
+    }
+  if (np) {
+    red[tid] = acc;
+    tree_cols(red, (int)nsl, (int)np, (int)tid, (int)(sl < nsl ? sl : kThreads));
+    if (tid < np) partial[(size_t)tid * gridDim.x + blockIdx.x] = red[tid];
+  }
+}
+
 // MINRES step, phase 2 with the Lanczos recurrence fused in (sum-factorised
 // cell products, whose cell kernel has already produced v.Hv, so that the
 // step's alpha is known before this kernel runs):
@@ -1493,40 +1582,6 @@ __device__ void tp_eval(const double* A, const double* in, double* t1, double* t
   __syncthreads();
 }
 
-// Transpose: in [Q][Q][Q][NC] -> out [N1][N1][N1][NC] (integration against N).
-template <int N1, int Q, int NC>
-__device__ void tp_integrate(const double* A, const double* in, double* t1, double* t2,
-                             double* out) {
-  const int tid = threadIdx.x;
-  for (int i = tid; i < Q * Q * N1 * NC; i += kThreads) {  // t1[qz][qy][a][col]
-    const int col = i % NC, a = (i / NC) % N1, qzy = i / (NC * N1);
-    const double* src = in + qzy * Q * NC + col;
-    double s = 0.0;
-#pragma unroll
-    for (int qx = 0; qx < Q; ++qx) s += A[qx * N1 + a] * src[qx * NC];
-    t1[i] = s;
-  }
-  __syncthreads();
-  for (int i = tid; i < Q * N1 * N1 * NC; i += kThreads) {  // t2[qz][b][a][col]
-    const int col = i % NC, a = (i / NC) % N1, b = (i / (NC * N1)) % N1, qz = i / (NC * N1 * N1);
-    const double* src = t1 + (qz * Q * N1 + a) * NC + col;
-    double s = 0.0;
-#pragma unroll
-    for (int qy = 0; qy < Q; ++qy) s += A[qy * N1 + b] * src[qy * N1 * NC];
-    t2[i] = s;
-  }
-  __syncthreads();
-  for (int i = tid; i < N1 * N1 * N1 * NC; i += kThreads) {  // out[c][b][a][col]
-    const int col = i % NC, ba = (i / NC) % (N1 * N1), c = i / (NC * N1 * N1);
-    const double* src = t2 + ba * NC + col;
-    double s = 0.0;
-#pragma unroll
-    for (int qz = 0; qz < Q; ++qz) s += A[qz * N1 + c] * src[qz * N1 * N1 * NC];
-    out[i] = s;
-  }
-  __syncthreads();
-}
-
 template <int N1, int Q, int NC>
 struct TpScratch {
   static constexpr int kIn = (N1 * N1 * N1 > Q * Q * Q ? N1 * N1 * N1 : Q * Q * Q) * NC;
@@ -1574,104 +1629,6 @@ __global__ __launch_bounds__(kThreads) void k_density(Geo g, const double* __res
     __syncthreads();
   }
   for (int q = tid; q < NQ; q += kThreads) rho[e * NQ + q] = acc[q];
-}
-
-// ---------------------------------------------------- pair quadrature dots
-// out[cell][k] = sum_q wq[cell][q] A_{i_k}(q) B_{j_k}(q)
-template <int P, int NC>
-__global__ __launch_bounds__(kThreads) void k_pair_quad(Geo g, const double* __restrict__ Lq,
-                                                        const double* __restrict__ Av,
-                                                        const double* __restrict__ Bv, int B,
-                                                        const int* __restrict__ pairs, int np,
-                                                        const double* __restrict__ wq,
-                                                        int64_t wstride,
-                                                        double* __restrict__ out) {
-  constexpr int N1 = P + 1, Q = P + 3, NE = ne_of(P), NQ = Q * Q * Q, H = NC / 2;
-  typedef TpScratch<N1, Q, NC> Sz;
-  __shared__ double A[Q * N1];
-  __shared__ double sin_[Sz::kIn], t1[Sz::kT1], t2[Sz::kT2], sout[Sz::kOut];
-  __shared__ double w[NQ];
-  __shared__ int64_t nodes[NE];
-  __shared__ double red[kThreads / 64][H];
-  const int64_t e = blockIdx.x;
-  const int64_t cx = e % g.nc, cy = (e / g.nc) % g.nc, cz = e / ((int64_t)g.nc * g.nc);
-  const int tid = threadIdx.x;
-  for (int i = tid; i < Q * N1; i += kThreads) A[i] = Lq[i];
-  for (int l = tid; l < NE; l += kThreads) nodes[l] = cell_node(g, cx, cy, cz, l);
-  for (int q = tid; q < NQ; q += kThreads) w[q] = wq[e * wstride + q];
-  __syncthreads();
-  for (int k0 = 0; k0 < np; k0 += H) {
-    // columns 0..H-1 <- A_i, H..NC-1 <- B_j of pairs k0..k0+H-1
-    for (int i = tid; i < NE * NC; i += kThreads) {
-      const int l = i / NC, k = i % NC, kp = k0 + (k % H);
-      double v = 0.0;
-      if (kp < np) {
-        if (k < H) v = Av[nodes[l] * B + pairs[2 * kp]];
-        else v = Bv[nodes[l] * B + pairs[2 * kp + 1]];
-      }
-      sin_[i] = v;
-    }
-    __syncthreads();
-    tp_eval<N1, Q, NC>(A, sin_, t1, t2, sout);
-    double part[H];
-#pragma unroll
-    for (int k = 0; k < H; ++k) part[k] = 0.0;
-    for (int q = tid; q < NQ; q += kThreads) {
-#pragma unroll
-      for (int k = 0; k < H; ++k) part[k] += w[q] * sout[q * NC + k] * sout[q * NC + H + k];
-    }
-#pragma unroll
-    for (int k = 0; k < H; ++k) {
-      double v = part[k];
-      for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
-      if ((tid & 63) == 0) red[tid / 64][k] = v;
-    }
-    __syncthreads();
-    if (tid < H && k0 + tid < np) {
-      double s = 0.0;
-      for (int wv = 0; wv < kThreads / 64; ++wv) s += red[wv][tid];
-      out[e * np + k0 + tid] = s;
-    }
-    __syncthreads();
-  }
-}
-
-// --------------------------------------------- quadrature cell operator
-// Y += N^T diag(wq) N X on the cells of one colour (no write conflicts).
-template <int P, int NC>
-__global__ __launch_bounds__(kThreads) void k_quad_operator(Geo g, const double* __restrict__ Lq,
-                                                            const double* __restrict__ X, int B,
-                                                            const double* __restrict__ wq,
-                                                            double* __restrict__ Y, int colour,
-                                                            int64_t nw) {
-  constexpr int N1 = P + 1, Q = P + 3, NE = ne_of(P), NQ = Q * Q * Q;
-  typedef TpScratch<N1, Q, NC> Sz;
-  __shared__ double A[Q * N1];
-  __shared__ double sin_[Sz::kIn], t1[Sz::kT1], t2[Sz::kT2], sout[Sz::kOut];
-  __shared__ int64_t nodes[NE];
-  const int64_t e = colour_cell(g, colour, blockIdx.x, nw);
-  if (e < 0) return;
-  const int64_t cx = e % g.nc, cy = (e / g.nc) % g.nc, cz = e / ((int64_t)g.nc * g.nc);
-  const int tid = threadIdx.x;
-  for (int i = tid; i < Q * N1; i += kThreads) A[i] = Lq[i];
-  for (int l = tid; l < NE; l += kThreads) nodes[l] = cell_node(g, cx, cy, cz, l);
-  __syncthreads();
-  for (int j0 = 0; j0 < B; j0 += NC) {
-    for (int i = tid; i < NE * NC; i += kThreads) {
-      const int l = i / NC, j = j0 + i % NC;
-      sin_[i] = j < B ? X[nodes[l] * B + j] : 0.0;
-    }
-    __syncthreads();
-    tp_eval<N1, Q, NC>(A, sin_, t1, t2, sout);
-    for (int i = tid; i < NQ * NC; i += kThreads) sout[i] *= wq[e * NQ + i / NC];
-    __syncthreads();
-    tp_integrate<N1, Q, NC>(A, sout, t1, t2, sin_);
-    for (int i = tid; i < NE * NC; i += kThreads) {
-      const int l = i / NC, j = j0 + i % NC;
-      if (j < B) Y[nodes[l] * B + j] += sin_[i];
-    }
-    __syncthreads();
-  }
 }
 
 // ------------------------------------------------------------ v_xc -> quad
@@ -2343,6 +2300,46 @@ __global__ __launch_bounds__(kThreads) void k_pairdot(int64_t N, int B, const do
   }
 }
 
+// Sparse column combination of the adjoint's two ends, in one pass over T, psi
+// and Y (Y may be T):
+//   RHS:  Y[n][i] = S[n] (cc[i] T[n][i]) + q[n] sum_e coef[e] psi[n][idx[e]]
+//   else: Y[n][i] = S[n] T[n][i]         +      sum_e coef[e] psi[n][idx[e]]
+// over the entries e in [start[i], start[i + 1]) of column i; where S[n] = 0
+// (the boundary) the T term is 0 whatever T holds and, with RHS, so is Y.  The
+// matrix couples degenerate pairs only, a few entries per column, so this is
+// bound by HBM (3 streams) where a dense product also spends N B^2 multiply-adds.
+// The lists sit in LDS; a lane's psi entries lie in the node's row, which the
+// neighbouring lanes read anyway.
+template <int VW, bool RHS>
+__global__ __launch_bounds__(kThreads) void k_pair_combine(
+    uint32_t NG, uint32_t B, const double* T, const double* __restrict__ S,
+    const double* __restrict__ q, const double* __restrict__ psi, const double* __restrict__ cc,
+    const double* __restrict__ coef_g, const int* __restrict__ list, uint32_t nnz, double* Y) {
+  extern __shared__ double lds[];
+  double* coef = lds;
+  int* start = reinterpret_cast<int*>(lds + nnz);
+  const int* idx = start + B + 1;
+  for (uint32_t i = threadIdx.x; i < nnz; i += kThreads) coef[i] = coef_g[i];
+  for (uint32_t i = threadIdx.x; i < B + 1 + nnz; i += kThreads) start[i] = list[i];
+  __syncthreads();
+  const uint32_t nb = B / VW;
+  for (uint32_t gi = blockIdx.x * kThreads + threadIdx.x; gi < NG; gi += gridDim.x * kThreads) {
+    const uint32_t n = gi / nb, j0 = (gi - n * nb) * VW, i = gi * VW;
+    const double s = S[n];
+    double t[VW], y[VW];
+    vload<double, VW>(T + i, t);
+    const double* pr = psi + (size_t)n * B;
+#pragma unroll
+    for (int v = 0; v < VW; ++v) {
+      double a = 0.0;
+      for (int e = start[j0 + v]; e < start[j0 + v + 1]; ++e) a += coef[e] * pr[idx[e]];
+      if constexpr (RHS) y[v] = s == 0.0 ? 0.0 : q[n] * a + s * (cc[j0 + v] * t[v]);
+      else y[v] = (s == 0.0 ? 0.0 : s * t[v]) + a;
+    }
+    vstore<double, VW>(Y + i, y);
+  }
+}
+
 // Attainable FMA rate: `CH` independent multiply-add chains per thread,
 // `iters` rounds, one store per thread (out holds one value per thread).
 template <typename T, int CH>
@@ -2407,6 +2404,7 @@ static void cell_sf_cg(const Geo& g, const CellOp<T>& op, const T* S, const TV* 
   check_u32(8 * ((npair + 7) / 8));
   dim3 grid((unsigned)(8 * ((npair + 7) / 8))), block(kThreads);
   const T hq = (T)op.kin_scale;
+  const uint32_t nq = (P + 3) * (P + 3) * (P + 3);
   const double* eo = sf_eo_table(P);
   // per-cell dots only with node-scaled inputs (the MINRES steps)
   if (dotp && !xn) throw Error(IDFT_EINVAL, "per-cell dots need a node-scaled input");
@@ -2414,15 +2412,15 @@ static void cell_sf_cg(const Geo& g, const CellOp<T>& op, const T* S, const TV* 
   // carry a node scale
   if constexpr (std::is_same<TV, double>::value) {
     if (xn) {
-      k_cell_sf<T, TV, P, CG, 1, true><<<grid, block, 0, s>>>(g, hq, op.W, S, X, xn, xcol, Yc, B,
-                                                               dotp, eo);
+      k_cell_sf<T, TV, P, CG, 1, true, true><<<grid, block, 0, s>>>(
+          g, hq, op.W, nq, S, X, (uint32_t)B, xn, xcol, Yc, B, dotp, eo);
       return;
     }
   } else {
     if (xn) throw Error(IDFT_EINVAL, "node-scaled input needs FP64 vectors");
   }
-  k_cell_sf<T, TV, P, CG, 1, false><<<grid, block, 0, s>>>(g, hq, op.W, S, X, nullptr, xcol, Yc, B,
-                                                             nullptr, eo);
+  k_cell_sf<T, TV, P, CG, 1, false, true><<<grid, block, 0, s>>>(
+      g, hq, op.W, nq, S, X, (uint32_t)B, nullptr, xcol, Yc, B, nullptr, eo);
 }
 
 template <typename T, typename TV, int P>
@@ -2620,6 +2618,90 @@ template int launch_cell_apply<float, double>(const Geo&, const CellOp<float>&, 
                                               const double*, const double*, float*, int,
                                               const ApplyEpilogue<double>&, const GemmShape&,
                                               hipStream_t);
+
+template <int P>
+static void quad_cells_p(const Geo& g, const double* W, int64_t wstride, const double* X, int ldx,
+                         int wb, double* Yc, int cg, hipStream_t s) {
+  const int64_t npair = g.ncell * ((wb + cg - 1) / cg);
+  check_u32(8 * ((npair + 7) / 8));
+  const unsigned grid = (unsigned)(8 * ((npair + 7) / 8));
+  const double* eo = sf_eo_table(P);
+#define IDFT_QC(CG)                                                                            \
+  k_cell_sf<double, double, P, CG, 1, false, false><<<grid, kThreads, 0, s>>>(                 \
+      g, 0.0, W, (uint32_t)wstride, nullptr, X, (uint32_t)ldx, nullptr, nullptr, Yc, wb, nullptr, eo)
+  if (cg == 2) IDFT_QC(2);
+  else if (cg == 4) IDFT_QC(4);
+  else IDFT_QC(8);
+#undef IDFT_QC
+}
+
+int quad_gather_blocks(const Geo& g, int wb, int vw) {
+  unsigned gx, gy;
+  uint32_t R;
+  gather_grid(g, wb, vw, 0, gx, gy, R);
+  return (int)std::min<unsigned>(gx, (unsigned)kMinresGatherBlocks);
+}
+
+void launch_quad_pairs(const Geo& g, const double* W, int64_t wstride, const double* Bv, int ldb,
+                       int wb, double* Yc, const double* A, int lda, const double* asc, double* T2,
+                       int ldt, const int* pairs, int np, DevBuf<double>& partial, double* out,
+                       hipStream_t s) {
+  if (wb < 1 || wb > kMaxCols || np < 0 || np > kThreads)
+    throw Error(IDFT_EINVAL, "block or pair count out of range");
+  check_u32(g.N);
+  check_u32(cell_scratch_elems(g, wb));
+  // columns per work-group: the narrowest group that holds a narrow block
+  const int cg = wb <= 2 ? 2 : 4;
+  // two columns per 16-byte access where every row starts at an even column
+  const int vw = wb % 2 == 0 && (np == 0 || lda % 2 == 0) && (!T2 || ldt % 2 == 0) ? 2 : 1;
+  const int nblk = quad_gather_blocks(g, wb, vw);
+  if (np) partial.resize((size_t)nblk * np);
+  unsigned gx, gy;
+  uint32_t R;
+  gather_grid(g, wb, vw, 0, gx, gy, R);
+  const FastDiv divN1 = make_fastdiv((uint32_t)g.N1);
+#define IDFT_QG(PP, VW)                                                                         \
+  k_quad_gather<PP, VW><<<nblk, kThreads, 0, s>>>(g, divN1, (uint32_t)wb, R, Yc, A, (uint32_t)lda, \
+                                                  asc, T2, (uint32_t)ldt, pairs, (uint32_t)np,  \
+                                                  partial.p)
+#define IDFT_QP(PP)                                                \
+  quad_cells_p<PP>(g, W, wstride, Bv, ldb, wb, Yc, cg, s);         \
+  IDFT_HIP(hipGetLastError());                                     \
+  if (vw == 2) IDFT_QG(PP, 2);                                     \
+  else IDFT_QG(PP, 1);
+  switch (g.p) {
+    case 2: IDFT_QP(2); break;
+    case 3: IDFT_QP(3); break;
+    case 4: IDFT_QP(4); break;
+    case 5: IDFT_QP(5); break;
+    default: throw Error(IDFT_EINVAL, "degree not supported by the HIP kernels (2..5)");
+  }
+#undef IDFT_QP
+#undef IDFT_QG
+  IDFT_HIP(hipGetLastError());
+  if (np) {
+    k_sum_rows<<<np, kRedThreads, 0, s>>>(nblk, partial.p, out);
+    IDFT_HIP(hipGetLastError());
+  }
+}
+
+void launch_pair_combine(int64_t N, int B, bool rhs, const double* T, const double* S,
+                         const double* q, const double* psi, const double* cc, const double* coef,
+                         const int* list, int nnz, double* Y, hipStream_t s) {
+  check_u32(N * B);
+  const size_t lds = (size_t)nnz * sizeof(double) + ((size_t)B + 1 + nnz) * sizeof(int);
+  if (lds > 65536) throw Error(IDFT_EINVAL, "too many column pairs");
+  const int vw = B % 2 == 0 ? 2 : 1;
+  const uint32_t NG = (uint32_t)(N * B / vw);
+  const int grid = grid_for(NG);
+#define IDFT_PC(VW, RHS)                                                                      \
+  k_pair_combine<VW, RHS><<<grid, kThreads, lds, s>>>(NG, (uint32_t)B, T, S, q, psi, cc, coef, \
+                                                      list, (uint32_t)nnz, Y)
+  if (rhs) { if (vw == 2) IDFT_PC(2, true); else IDFT_PC(1, true); }
+  else { if (vw == 2) IDFT_PC(2, false); else IDFT_PC(1, false); }
+#undef IDFT_PC
+  IDFT_HIP(hipGetLastError());
+}
 
 template <typename T, typename TV>
 void launch_cell_dot(const Geo& g, const CellOp<T>& op, const T* Sg, const TV* X, int B,
@@ -2845,36 +2927,6 @@ void launch_loss(int64_t nQ, int nq, const double* rho, const double* rhoT, cons
                  const double* veff, const double* jxw, double* u, double* partial,
                  hipStream_t s) {
   k_loss<<<256, kThreads, 0, s>>>(nQ, nq, rho, rhoT, w, veff, jxw, u, partial);
-  IDFT_HIP(hipGetLastError());
-}
-
-void launch_pair_quad(const Geo& g, const DevTables& t, const double* A, const double* Bv, int B,
-                      const int* pairs, int np, const double* wq, int64_t wstride, double* out,
-                      hipStream_t s) {
-  if (np == 0) return;
-  dim3 grid((unsigned)g.ncell), block(kThreads);
-  switch (g.p) {
-    case 2: k_pair_quad<2, 8><<<grid, block, 0, s>>>(g, t.Lq.p, A, Bv, B, pairs, np, wq, wstride, out); break;
-    case 3: k_pair_quad<3, 8><<<grid, block, 0, s>>>(g, t.Lq.p, A, Bv, B, pairs, np, wq, wstride, out); break;
-    case 4: k_pair_quad<4, 8><<<grid, block, 0, s>>>(g, t.Lq.p, A, Bv, B, pairs, np, wq, wstride, out); break;
-    case 5: k_pair_quad<5, 8><<<grid, block, 0, s>>>(g, t.Lq.p, A, Bv, B, pairs, np, wq, wstride, out); break;
-    default: throw Error(IDFT_EINVAL, "degree not supported");
-  }
-  IDFT_HIP(hipGetLastError());
-}
-
-void launch_quad_operator(const Geo& g, const DevTables& t, const double* X, int B,
-                          const double* wq, double* Y, int colour, hipStream_t s) {
-  const int64_t nw = colour_count(g, colour);
-  if (nw == 0) return;
-  dim3 grid(colour_grid(nw)), block(kThreads);
-  switch (g.p) {
-    case 2: k_quad_operator<2, 8><<<grid, block, 0, s>>>(g, t.Lq.p, X, B, wq, Y, colour, nw); break;
-    case 3: k_quad_operator<3, 8><<<grid, block, 0, s>>>(g, t.Lq.p, X, B, wq, Y, colour, nw); break;
-    case 4: k_quad_operator<4, 8><<<grid, block, 0, s>>>(g, t.Lq.p, X, B, wq, Y, colour, nw); break;
-    case 5: k_quad_operator<5, 8><<<grid, block, 0, s>>>(g, t.Lq.p, X, B, wq, Y, colour, nw); break;
-    default: throw Error(IDFT_EINVAL, "degree not supported");
-  }
   IDFT_HIP(hipGetLastError());
 }
 

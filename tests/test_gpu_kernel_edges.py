@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 
 from invdft_amd import abi
-from tests.helpers import bare_pair
+from tests.helpers import bare_pair, rel
 
 pytestmark = pytest.mark.gpu
 
@@ -33,3 +33,39 @@ def test_vmult_clears_exactly_the_boundary_rows(glib, olib, n_cells, degree, b):
     want = np.where(_boundary(n_cells * degree + 1)[:, None], 0.0, x)
     assert np.array_equal(xv.get(), want)
     assert np.array_equal(psi.get(), want)
+
+
+def _adjoint_pair(glib, olib, n_cells, degree, b, pairs, seed=3):
+    """computeRhs and distributeX of both backends on the same block."""
+    g, o, s = bare_pair(glib, olib, n_cells, degree, 4)
+    rng = np.random.default_rng(seed)
+    psi = np.linalg.qr(rng.standard_normal((s.n_nodes, b)))[0]
+    x = rng.standard_normal((s.n_nodes, b))
+    u = rng.standard_normal(s.n_cells * s.quad_per_cell)
+    eig = np.sort(rng.uniform(-2.0, -0.5, b))
+    occ = rng.uniform(0.1, 1.0, b)
+    out = []
+    for c in (g, o):
+        mp, mx, rhs = c.mv(b, psi), c.mv(b, x), c.mv(b)
+        c.adj_update_input_psi(mp, occ, u, pairs, -0.5, eig.copy())
+        c.adj_compute_rhs(None, mx, rhs)
+        dots = c.adj_dot_quad_wise(mx, mp, len(pairs))
+        c.adj_distribute_x()
+        out.append((rhs.get(), mx.get(), dots))
+    return out
+
+
+# one column, odd and even widths, more pairs than columns (the dense product),
+# and more than one run of 256 pairs
+@pytest.mark.parametrize("n_cells,degree,b,extra", [(2, 2, 1, 0), (3, 5, 3, 2), (2, 4, 24, 6),
+                                                    (2, 3, 11, 90), (2, 2, 20, 300)])
+def test_adjoint_ends_match_oracle(glib, olib, n_cells, degree, b, extra):
+    _say("ends", n_cells, degree, b, extra)
+    rng = np.random.default_rng(b + extra)
+    pairs = {(i, i) for i in range(b)}
+    while len(pairs) < min(b + extra, b * b):
+        pairs.add(tuple(int(v) for v in rng.integers(0, b, 2)))
+    (rg, xg, dg), (ro, xo, do) = _adjoint_pair(glib, olib, n_cells, degree, b, sorted(pairs))
+    # sums of some 10^4 products in another order: 1e-15 sqrt(1e4) relative
+    assert rel(rg, ro) < 1e-12 and rel(xg, xo) < 1e-12
+    assert np.max(np.abs(np.asarray(dg) - do)) < 1e-12 * np.max(np.abs(do))
