@@ -67,7 +67,8 @@ int idft_loss_weights(int64_t n, const double* rho_spin, double spin_factor, dou
  * InverseDFTEngine.cpp:2457-2624, a CG solve of DFT-FE's poissonSolverProblem):
  *   -lap phi = 4 pi c,   phi = g on the boundary,
  * c the charge density at parent quadrature (electrons positive), by
- * Jacobi-preconditioned CG on the stiffness matrix to ||r||_D <= tol ||b||_D.
+ * CG on the stiffness matrix to ||r||_D <= tol ||b||_D, D its Jacobi diagonal,
+ * preconditioned by the matrix's tensor-product inverse (one or two steps).
  * boundary_nodal (may be NULL): g at the parent nodes (only boundary entries
  * are read); NULL takes the monopole + dipole field of c about the origin
  * (multipole boundary conditions).  phi_q [cells*Q^3] and phi_nodal [N]

@@ -4,6 +4,7 @@
 #include <cstring>
 
 #include "common.h"
+#include "setup.h"
 
 namespace idft {
 
@@ -273,6 +274,78 @@ bool cholesky_lower(int n, std::vector<double>& S) {
     for (int i = 0; i < j; ++i) S[(size_t)i * n + j] = 0.0;
   }
   return true;
+}
+
+// The assembled 1D mass and stiffness matrices are symmetric about the cell
+// row's centre, so the pencil splits into its even and odd halves (basis
+// (e_i +- e_{n-1-i}) / sqrt 2), a quarter of the work and exactly symmetric
+// vectors.  Each half: M = R R^T, eigenpairs of R^-1 D R^-T, v = R^-T q.
+void axis_eigenpairs(const Tables& t, std::vector<double>& lam, std::vector<double>& V) {
+  const int N1 = t.N1, n = N1 - 2;
+  std::vector<double> M((size_t)N1 * N1, 0.0), D((size_t)N1 * N1, 0.0);
+  for (int c = 0; c < t.nc; ++c)
+    for (int a = 0; a < t.n1; ++a)
+      for (int b = 0; b < t.n1; ++b) {
+        M[(size_t)(c * t.p + a) * N1 + c * t.p + b] += t.M1[a * t.n1 + b];
+        D[(size_t)(c * t.p + a) * N1 + c * t.p + b] += t.D1[a * t.n1 + b];
+      }
+  lam.assign(n, 0.0);
+  V.assign((size_t)n * n, 0.0);
+  int col = 0;
+  for (int odd = 0; odd < 2; ++odd) {
+    const int h = odd ? n / 2 : (n + 1) / 2;
+    if (h == 0) continue;
+    const double sg = odd ? -1.0 : 1.0;
+    // entry (i, j) of B^T A B: A_ij + sg A_i,n-1-j, the middle node scaled
+    auto half = [&](const std::vector<double>& A) {
+      std::vector<double> H((size_t)h * h);
+      for (int i = 0; i < h; ++i)
+        for (int j = 0; j < h; ++j) {
+          const int i2 = n - 1 - i, j2 = n - 1 - j;
+          const double aij = A[(size_t)(i + 1) * N1 + j + 1];
+          double v;
+          if (i == i2 && j == j2) v = aij;
+          else if (i == i2 || j == j2) v = std::sqrt(2.0) * aij;
+          else v = aij + sg * A[(size_t)(i + 1) * N1 + j2 + 1];
+          H[(size_t)i * h + j] = v;
+        }
+      return H;
+    };
+    std::vector<double> R = half(M), C = half(D), ev, Q;
+    if (!cholesky_lower(h, R)) throw Error(IDFT_EINVAL, "1D mass matrix not positive definite");
+    for (int j = 0; j < h; ++j)  // C <- R^-1 C (rows), then C <- C R^-T (columns)
+      for (int i = 0; i < h; ++i) {
+        double v = C[(size_t)i * h + j];
+        for (int k = 0; k < i; ++k) v -= R[(size_t)i * h + k] * C[(size_t)k * h + j];
+        C[(size_t)i * h + j] = v / R[(size_t)i * h + i];
+      }
+    for (int i = 0; i < h; ++i)
+      for (int j = 0; j < h; ++j) {
+        double v = C[(size_t)i * h + j];
+        for (int k = 0; k < j; ++k) v -= R[(size_t)j * h + k] * C[(size_t)i * h + k];
+        C[(size_t)i * h + j] = v / R[(size_t)j * h + j];
+      }
+    for (int i = 0; i < h; ++i)
+      for (int j = i + 1; j < h; ++j)
+        C[(size_t)i * h + j] = C[(size_t)j * h + i] =
+            0.5 * (C[(size_t)i * h + j] + C[(size_t)j * h + i]);
+    sym_eig(h, C, ev, Q);
+    for (int e = 0; e < h; ++e, ++col) {
+      std::vector<double> v(h);
+      for (int i = h - 1; i >= 0; --i) {
+        double s = Q[(size_t)i * h + e];
+        for (int k = i + 1; k < h; ++k) s -= R[(size_t)k * h + i] * v[k];
+        v[i] = s / R[(size_t)i * h + i];
+      }
+      lam[col] = ev[e];
+      for (int i = 0; i < h; ++i) {
+        const int i2 = n - 1 - i;
+        const double w = i == i2 ? v[i] : v[i] * std::sqrt(0.5);
+        V[(size_t)i * n + col] = w;
+        if (i2 != i) V[(size_t)i2 * n + col] = sg * w;
+      }
+    }
+  }
 }
 
 uint64_t splitmix64(uint64_t& s) {

@@ -56,6 +56,23 @@ void launch_guess(int64_t n, const GuessArgs& ga, const double* rho_spin, const 
                   const double* vH, double* v, hipStream_t s);
 void launch_nodal_to_quad(const Geo& g, const double* Lq, const double* x, double* out,
                           hipStream_t s);
+// w4 = 4 pi c JxW; partial [kChargeBlocks][4] = partials of (int c, int c x,y,z)
+constexpr int kChargeBlocks = 1024;
+void launch_charge(const QuadGeo& qg, int64_t nQ, const double* c, const double* jxw, double* w4,
+                   double* partial, hipStream_t s);
+void launch_boundary_values(const Geo& g, const double* x1, const double* bc, const double* mom,
+                            double* gv, double* mask, hipStream_t s);
+void launch_fill(int64_t n, double a, double* v, hipStream_t s);
+// compact interior of a node vector times a node scale, or back into one
+void launch_interior(const Geo& g, const double* x, const double* sc, double* out, bool back,
+                     hipStream_t s);
+// Y[m][i] = sum_k Bt[k][i] X[k][m] of an n x n^2 array, divided by
+// hq (lam_a + lam_b + lam_i), m = a n + b, if lam is given
+void launch_axis_transform(int n, const double* Bt, const double* X, double* Y, double hq,
+                           const double* lam, hipStream_t s);
+// Eigenpairs of the interior 1D pencil D v = lam M v of the mesh: V (n x n
+// row-major, column i the i-th vector, V^T M V = I), n = N1 - 2.
+void axis_eigenpairs(const Tables& t, std::vector<double>& lam, std::vector<double>& V);
 void child_mass_factors(int NV1, double hc, std::vector<double>& cp, std::vector<double>& inv);
 void launch_child_mass_solve(int NV1, double hc, const double* cp, const double* inv, double* v,
                              hipStream_t s);

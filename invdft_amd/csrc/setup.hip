@@ -187,26 +187,164 @@ __global__ void k_guess(int64_t n, GuessArgs ga, const double* __restrict__ rho_
   v[i] = val;
 }
 
-// out[e][q] = sum_abc Lq[qx][a] Lq[qy][b] Lq[qz][c] x[node(e, a, b, c)]
-__global__ void k_nodal_to_quad(Geo g, const double* __restrict__ Lq, const double* __restrict__ x,
-                                double* __restrict__ out) {
-  const int nq = g.q1 * g.q1 * g.q1;
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= g.ncell * nq) return;
-  const int64_t e = i / nq;
-  const int q = (int)(i - e * nq);
+// Node field at the parent quadrature points, one work-group per cell: three 1D
+// contractions in LDS instead of the (p+1)^3 terms of every point (180 us at
+// 16 cells, p = 4).
+__global__ __launch_bounds__(kT) void k_nodal_to_quad(Geo g, const double* __restrict__ Lq,
+                                                      const double* __restrict__ x,
+                                                      double* __restrict__ out) {
+  __shared__ double L[8 * 6], a[8 * 8 * 8], b[8 * 8 * 8];  // p <= 5
+  const int n1 = g.n1, q1 = g.q1, tid = threadIdx.x;
+  const int64_t e = blockIdx.x;
   const int64_t cx = e % g.nc, cy = (e / g.nc) % g.nc, cz = e / ((int64_t)g.nc * g.nc);
-  const int qx = q % g.q1, qy = (q / g.q1) % g.q1, qz = q / (g.q1 * g.q1);
-  double s = 0.0;
-  for (int c = 0; c < g.n1; ++c) {
-    const double lc = Lq[qz * g.n1 + c];
-    for (int b = 0; b < g.n1; ++b) {
-      const double lbc = lc * Lq[qy * g.n1 + b];
-      const int64_t row = ((cz * g.p + c) * g.N1 + (cy * g.p + b)) * (int64_t)g.N1 + cx * g.p;
-      for (int a = 0; a < g.n1; ++a) s += lbc * Lq[qx * g.n1 + a] * x[row + a];
+  for (int i = tid; i < q1 * n1; i += kT) L[i] = Lq[i];
+  for (int i = tid; i < n1 * n1 * n1; i += kT) {
+    const int ax = i % n1, ay = (i / n1) % n1, az = i / (n1 * n1);
+    a[i] = x[((cz * g.p + az) * g.N1 + (cy * g.p + ay)) * (int64_t)g.N1 + cx * g.p + ax];
+  }
+  __syncthreads();
+  for (int i = tid; i < n1 * n1 * q1; i += kT) {  // [az][ay][qx]
+    const int q = i % q1, r = i / q1;
+    double s = 0.0;
+    for (int k = 0; k < n1; ++k) s += L[q * n1 + k] * a[r * n1 + k];
+    b[i] = s;
+  }
+  __syncthreads();
+  for (int i = tid; i < n1 * q1 * q1; i += kT) {  // [az][qy][qx]
+    const int qx = i % q1, qy = (i / q1) % q1, r = i / (q1 * q1);
+    double s = 0.0;
+    for (int k = 0; k < n1; ++k) s += L[qy * n1 + k] * b[(r * n1 + k) * q1 + qx];
+    a[i] = s;
+  }
+  __syncthreads();
+  const int nq = q1 * q1 * q1;
+  for (int i = tid; i < nq; i += kT) {
+    const int qxy = i % (q1 * q1), qz = i / (q1 * q1);
+    double s = 0.0;
+    for (int k = 0; k < n1; ++k) s += L[qz * n1 + k] * a[k * q1 * q1 + qxy];
+    out[e * nq + i] = s;
+  }
+}
+
+// Charge c at the quadrature points -> w4 = (4 pi c) JxW and the block partials
+// (int c, int c x, int c y, int c z) about the origin.
+__global__ __launch_bounds__(kT) void k_charge(QuadGeo qg, int64_t nQ, const double* __restrict__ c,
+                                               const double* __restrict__ jxw,
+                                               double* __restrict__ w4,
+                                               double* __restrict__ partial) {
+  __shared__ double red[4][kT];
+  const int nq = qg.q1 * qg.q1 * qg.q1, tid = threadIdx.x;
+  double m[4] = {0.0, 0.0, 0.0, 0.0};
+  for (int64_t i = blockIdx.x * (int64_t)kT + tid; i < nQ; i += (int64_t)gridDim.x * kT) {
+    double x[3];
+    quad_point(qg, i, x);
+    const double ci = c[i], jw = jxw[i % nq], w = ci * jw;
+    w4[i] = 4.0 * M_PI * ci * jw;
+    m[0] += w;
+    for (int k = 0; k < 3; ++k) m[1 + k] += w * x[k];
+  }
+  for (int k = 0; k < 4; ++k) red[k][tid] = m[k];
+  __syncthreads();
+  for (int st = kT / 2; st > 0; st >>= 1) {
+    if (tid < st)
+      for (int k = 0; k < 4; ++k) red[k][tid] += red[k][tid + st];
+    __syncthreads();
+  }
+  if (tid < 4) partial[blockIdx.x * 4 + tid] = red[tid][0];
+}
+
+// Dirichlet values on the boundary nodes (bc, or the monopole and dipole of
+// mom = (Q, dipole)), 0 inside; mask = 1 on the boundary nodes, 0 inside.
+__global__ __launch_bounds__(kT) void k_boundary_values(Geo g, const double* __restrict__ x1,
+                                                        const double* __restrict__ bc,
+                                                        const double* __restrict__ mom,
+                                                        double* __restrict__ gv,
+                                                        double* __restrict__ mask) {
+  const int64_t n = blockIdx.x * (int64_t)kT + threadIdx.x;
+  if (n >= g.N) return;
+  const int e = g.N1 - 1;
+  const int i = (int)(n % g.N1), j = (int)((n / g.N1) % g.N1), k = (int)(n / ((int64_t)g.N1 * g.N1));
+  const bool edge = i == 0 || j == 0 || k == 0 || i == e || j == e || k == e;
+  mask[n] = edge ? 1.0 : 0.0;
+  double v = 0.0;
+  if (edge && bc) {
+    v = bc[n];
+  } else if (edge) {
+    const double x = x1[i], y = x1[j], z = x1[k], r = sqrt(x * x + y * y + z * z);
+    v = mom[0] / r + (mom[1] * x + mom[2] * y + mom[3] * z) / (r * r * r);
+  }
+  gv[n] = v;
+}
+
+__global__ __launch_bounds__(kT) void k_fill(int64_t n, double a, double* __restrict__ v) {
+  const int64_t i = blockIdx.x * (int64_t)kT + threadIdx.x;
+  if (i < n) v[i] = a;
+}
+
+// Interior nodes of a node vector, compact (n = N1 - 2 per axis), times the node
+// scale: out = sc x, and back (boundary 0).
+__global__ __launch_bounds__(kT) void k_interior(Geo g, const double* __restrict__ x,
+                                                 const double* __restrict__ sc,
+                                                 double* __restrict__ out, int back) {
+  const int64_t t = blockIdx.x * (int64_t)kT + threadIdx.x;
+  if (t >= g.N) return;
+  const int n = g.N1 - 2;
+  const int i = (int)(t % g.N1) - 1, j = (int)((t / g.N1) % g.N1) - 1,
+            k = (int)(t / ((int64_t)g.N1 * g.N1)) - 1;
+  const bool in = i >= 0 && j >= 0 && k >= 0 && i < n && j < n && k < n;
+  const int64_t m = ((int64_t)k * n + j) * n + i;
+  if (back) out[t] = in ? sc[t] * x[m] : 0.0;
+  else if (in) out[m] = sc[t] * x[t];
+}
+
+// One axis of a tensor-product transform of an n^3 array with the array's axes
+// rotated: Y[m][i] = sum_k Bt[k][i] X[k][m], k the slowest axis of X, m = the n^2
+// entries of the other two.  Three in a row transform all axes and return to
+// the original order, with every load and store of X and Y along the fastest
+// index.  lam (optional): Y divided by hq (lam_a + lam_b + lam_i), m = a n + b.
+// A wave forms a 16 (m) x 16 (i) tile on v_mfma_f64_16x16x4 from operands read
+// straight from memory (n^2 work-rows of n; a tile of X is shared by the four
+// waves through the L1): 2 n^4 operations on 2 n^3 values, matrix cores from
+// n of about 60 on, launch latency below.
+typedef double v4d __attribute__((ext_vector_type(4)));
+__global__ __launch_bounds__(kT) void k_axis_transform(int n, const double* __restrict__ Bt,
+                                                       const double* __restrict__ X,
+                                                       double* __restrict__ Y, double hq,
+                                                       const double* __restrict__ lam) {
+  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64, lr = lane % 16, lk = lane / 16;
+  const int64_t n2 = (int64_t)n * n, m0 = (int64_t)blockIdx.x * 16;
+  const int i0 = (blockIdx.y * 4 + wave) * 16;
+  if (i0 >= n) return;
+  const int64_t ma = m0 + lr < n2 ? m0 + lr : n2 - 1;
+  const int ib = i0 + lr < n ? i0 + lr : n - 1;
+  v4d acc = {0.0, 0.0, 0.0, 0.0};
+  const int kd = (n / 16) * 16;
+  for (int k = 0; k < kd; k += 16) {  // four k-steps per round, their loads issued together
+    double a[4], b[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      a[u] = X[(int64_t)(k + 4 * u + lk) * n2 + ma];
+      b[u] = Bt[(int64_t)(k + 4 * u + lk) * n + ib];
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u], b[u], acc, 0, 0, 0);
+  }
+  for (int kk = kd; kk < n; kk += 4) {
+    const bool ok = kk + lk < n;
+    const double a = ok ? X[(int64_t)(kk + lk) * n2 + ma] : 0.0;
+    const double b = ok ? Bt[(int64_t)(kk + lk) * n + ib] : 0.0;
+    acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc, 0, 0, 0);
+  }
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int64_t m = m0 + lk + 4 * u;  // the f64 MFMA's rows (lane / 16) + 4 u
+    const int i = i0 + lr;
+    if (m < n2 && i < n) {
+      double y = acc[u];
+      if (lam) y /= hq * (lam[m / n] + lam[m % n] + lam[i]);
+      Y[m * n + i] = y;
     }
   }
-  out[i] = s;
 }
 
 // In-place solve along one axis of the child grid (NV1^3 nodes) with the 1D
@@ -284,8 +422,34 @@ void launch_guess(int64_t n, const GuessArgs& ga, const double* rho_spin, const 
 }
 void launch_nodal_to_quad(const Geo& g, const double* Lq, const double* x, double* out,
                           hipStream_t s) {
-  const int64_t n = g.ncell * (int64_t)g.q1 * g.q1 * g.q1;
-  k_nodal_to_quad<<<grid_of(n), kT, 0, s>>>(g, Lq, x, out);
+  if (g.q1 > 8) throw Error(IDFT_EINVAL, "degree not supported by the HIP kernels (2..5)");
+  k_nodal_to_quad<<<(unsigned)g.ncell, kT, 0, s>>>(g, Lq, x, out);
+  IDFT_HIP(hipGetLastError());
+}
+void launch_charge(const QuadGeo& qg, int64_t nQ, const double* c, const double* jxw, double* w4,
+                   double* partial, hipStream_t s) {
+  k_charge<<<kChargeBlocks, kT, 0, s>>>(qg, nQ, c, jxw, w4, partial);
+  IDFT_HIP(hipGetLastError());
+}
+void launch_boundary_values(const Geo& g, const double* x1, const double* bc, const double* mom,
+                            double* gv, double* mask, hipStream_t s) {
+  k_boundary_values<<<grid_of(g.N), kT, 0, s>>>(g, x1, bc, mom, gv, mask);
+  IDFT_HIP(hipGetLastError());
+}
+void launch_fill(int64_t n, double a, double* v, hipStream_t s) {
+  if (n <= 0) return;
+  k_fill<<<grid_of(n), kT, 0, s>>>(n, a, v);
+  IDFT_HIP(hipGetLastError());
+}
+void launch_interior(const Geo& g, const double* x, const double* sc, double* out, bool back,
+                     hipStream_t s) {
+  k_interior<<<grid_of(g.N), kT, 0, s>>>(g, x, sc, out, back ? 1 : 0);
+  IDFT_HIP(hipGetLastError());
+}
+void launch_axis_transform(int n, const double* Bt, const double* X, double* Y, double hq,
+                           const double* lam, hipStream_t s) {
+  const dim3 grid((unsigned)(((int64_t)n * n + 15) / 16), (unsigned)((n + 63) / 64));
+  k_axis_transform<<<grid, kT, 0, s>>>(n, Bt, X, Y, hq, lam);
   IDFT_HIP(hipGetLastError());
 }
 void launch_child_mass_solve(int NV1, double hc, const double* cp, const double* inv, double* v,

@@ -5,6 +5,7 @@ import pytest
 
 from invdft_amd import abi
 from tests.helpers import bare_pair, rel
+from tests.setup_abi import poisson
 
 pytestmark = pytest.mark.gpu
 
@@ -69,3 +70,23 @@ def test_adjoint_ends_match_oracle(glib, olib, n_cells, degree, b, extra):
     # sums of some 10^4 products in another order: 1e-15 sqrt(1e4) relative
     assert rel(rg, ro) < 1e-12 and rel(xg, xo) < 1e-12
     assert np.max(np.abs(np.asarray(dg) - do)) < 1e-12 * np.max(np.abs(do))
+
+
+# interior sizes n = N1 - 2 of the axis transforms: 3, 8, 15, 32 (whole tiles), 65
+@pytest.mark.parametrize("n_cells,degree,with_bc", [(2, 2, True), (3, 3, False), (8, 2, True),
+                                                    (11, 3, False), (22, 3, True)])
+def test_poisson_tile_edges_match_oracle(glib, olib, n_cells, degree, with_bc):
+    _say("poisson", n_cells, degree, with_bc)
+    d = abi.default_desc(olib, n_cells=n_cells, degree=degree, half_width=3.0)
+    xyz = abi.quad_points(olib, d)
+    c = np.exp(-np.sum((xyz - [0.4, -0.3, 0.2]) ** 2, axis=1)) * (1.0 + 0.3 * xyz[:, 1])
+    bc = None
+    if with_bc:
+        nx = abi.node_points(olib, d)
+        bc = 0.5 + 0.1 * nx[:, 0] - 0.2 * nx[:, 1] * nx[:, 2]
+    pg, ng, sg = poisson(glib, d, c, bc=bc, tol=1e-12)
+    po, no, so = poisson(olib, d, c, bc=bc, tol=1e-12)
+    # both stop at a relative residual of 1e-12; the operator's condition number
+    # in the residual's norm is below 1e3 here
+    assert rel(pg, po) < 1e-9 and rel(ng, no) < 1e-9
+    assert sg.rel_residual <= 1e-12 and abs(sg.charge - so.charge) < 1e-12 * abs(so.charge)
