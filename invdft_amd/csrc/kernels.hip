@@ -557,57 +557,31 @@ __global__ __launch_bounds__(kSymmThreads) void k_cell_symm(Geo g, const T* __re
 // the (p+3)^3 weights w_e are read from HBM instead of n_e(n_e+1)/2 entries of
 // H_e.  The 1D tables are compile-time constants (SfC<P>): after unrolling
 // every FP32 coefficient is an immediate operand, and the FP64 ones come from
-// a constant-memory table (eo_coef below); h/4 scales the kinetic sum once.
+// a constant-memory table (PlCoef below); h/4 scales the kinetic sum once.
 //
-// One work-group handles one cell and CG columns; an item is one line of the
-// cell's tensor along one axis for VC consecutive columns (VC-wide LDS
-// accesses).  Intermediates live in LDS as [entry][CG / VC] packs, with padded
-// line strides (N1 and Q rounded up to odd: 5, 7 at p = 4; 7, 9 at p = 5) so
-// that the 64 lanes of a wave spread over the banks (an even stride such as 6
-// or 8 at p = 4 folds the lines of a wave onto a few banks).  The exception is
-// region D in FP64 at p = 5 (Q = 8): unpadded lines, entry x of line (c, y)
-// at slot x ^ y, which spreads the lanes over the banks as the stride 9 does,
-// and puts the lines that one stage-6 item reads 512 B apart, so that the
-// compiler pairs those accesses (ds_read2st64 / ds_write2st64).  It also
-// takes 20.4 KB instead of 21.9 KB per work-group, which does not raise the
-// occupancy: the kernel's 71 registers allow 7 waves per SIMD either way (with
-// the stage-6 weights loaded after stage 3 it fits 64 registers and 8
-// work-groups per CU, but measured slower: the weights' latency shows).  The kinetic
-// chain runs first and the x-line input stays in registers for the potential
-// chain, and the y and z stages overwrite their input in place (each item
-// reads its whole line before writing the same positions; in stage 5 the
-// item (c, qx) owns the column [c][*][qx] of D, which holds t1 along b and
-// then t2 along qy).  Region Bk is dead once stage 3 has run, so D shares its
-// memory:
-//   1  x lines (c,b):  ka = M x -> A,  kb = D x -> Bk      (x gathered from HBM)
-//   2  y lines (c,a):  k1 = M ka -> A,  k2 = D ka + M kb -> Bk
-//   3  z lines (b,a):  yk = D k1 + M k2 -> A
-//   4  x lines (c,b):  t1[c][b][qx] = Lq x -> D             (x from registers)
-//   5  y lines (c,qx): t2[c][qy][qx] = Lq t1 -> D
-//   6  z lines (qy,qx): s2 = Lq^T (w .* (Lq t2)) -> D
-//   7  y lines (c,qx): s1[c][b][qx] = Lq^T s2 -> D
-//   8  x lines (c,b):  Yc[e][(c,b,a)][j] = (Lq^T s1)[a] + (h/4) yk[a]
-// At p = 5 that is 252 + 432 = 684 entries per column, 252 + 384 = 636 with
-// the unpadded FP64 region D.
-__host__ __device__ constexpr int cmax(int a, int b) { return a > b ? a : b; }
-
-template <typename T, int VC>
-struct alignas(sizeof(T) * VC) Pack {
-  T v[VC];
-};
-template <typename T, int VC>
-__device__ inline void pack_zero(Pack<T, VC>& p) {
-#pragma unroll
-  for (int u = 0; u < VC; ++u) p.v[u] = T(0);
-}
-template <typename T, int VC>
-__device__ inline void pack_fma(Pack<T, VC>& acc, T c, const Pack<T, VC>& x) {
-#pragma unroll
-  for (int u = 0; u < VC; ++u) acc.v[u] += c * x.v[u];
-}
-
+// Layout.  A lane owns one (cell, column) slot and one of its Q = p + 3 Gauss
+// planes along z; a wave holds NS = 64 / Q slots and works alone (no barriers).
+// Along x and y everything happens in the lane's registers, so the tensor crosses
+// LDS only where z mixes the planes:
+//   1  z lines of the scaled input (from HBM): u[q] = Lq x, to LDS
+//   2  the lane's plane u: m = (M (x) M) u and
+//      p = (h/4) g_q (D (x) M + M (x) D) u + (Lq (x) Lq)^T diag(w) (Lq (x) Lq) u
+//      with g_q the Gauss weight, since M = Lq^T diag(g) Lq along z
+//   3  z lines back: y = Lq^T p + (h/4) E m, E Lq = D, to the cell scratch
+// That is about 2000 LDS entries per cell and column at p = 5 where the same chain
+// taken line by line (one work-group per cell and 4 columns, eight stages with a
+// barrier each) moved 4850 and left a quarter of its lanes idle in most stages.
+// Slots are numbered cell B + column over the whole mesh, so that a wave is full at
+// every block width.
+// Bound by VALU issue: about 60 % of it in FP64, 80 % in FP32 (2 to 5 waves per
+// SIMD; FP64 at p = 5 takes 246 registers).  Measured against the line-by-line
+// kernel, us of the cell product alone: FP64 27 cells p = 3 B = 12 135 -> 96,
+// 19 p = 4 B = 21 171 -> 111, 30 p = 4 B = 64 1383 -> 1139, 24 p = 5 B = 1 65 -> 26
+// and B = 12 261 -> 233, 40 p = 2 B = 8 190 -> 73; FP32 87 -> 42, 93 -> 57,
+// 921 -> 735, 39 -> 18, 154 -> 138 and 136 -> 34; 8 p = 3 B = 5, where one wave's
+// latency is the time, 5.4 -> 5.3 and (FP32) 4.1 -> 4.6.
 // The 1D tables as operators A (R x C): K = 0 Lq (Gauss points from nodes),
-// 1 Lq^T, 2 M, 3 D.  The GLL nodes and the Gauss points lie symmetrically
+// 1 Lq^T, 2 M, 3 D, 4 E (D from the Gauss points, E Lq = D).  The GLL nodes and the Gauss points lie symmetrically
 // about the cell centre, so each A is centro-symmetric,
 // A[R-1-i][C-1-j] = A[i][j] (to rounding of the tables).
 template <int P, int K>
@@ -615,12 +589,13 @@ struct SfTab {
   static constexpr int kP = P, kK = K;
   static constexpr int N1 = P + 1, Q = P + 3;
   static constexpr int R = K == 0 ? Q : N1;
-  static constexpr int C = K == 1 ? Q : N1;
+  static constexpr int C = K == 1 || K == 4 ? Q : N1;
   __host__ __device__ static constexpr double at(int i, int j) {
     return K == 0   ? SfC<P>::v.L[i * N1 + j]
            : K == 1 ? SfC<P>::v.L[j * N1 + i]
            : K == 2 ? SfC<P>::v.M[i * N1 + j]
-                    : SfC<P>::v.D[i * N1 + j];
+           : K == 3 ? SfC<P>::v.D[i * N1 + j]
+                    : SfC<P>::v.E[i * Q + j];
   }
 };
 // Even-odd form of y = A x (Kopriva's even-odd decomposition).  With
@@ -656,20 +631,22 @@ __device__ constexpr T eo_mid() {
 template <int P>
 struct EoTable {
   static constexpr int R(int k) { return k == 0 ? P + 3 : P + 1; }
-  static constexpr int C(int k) { return k == 1 ? P + 3 : P + 1; }
+  static constexpr int C(int k) { return k == 1 || k == 4 ? P + 3 : P + 1; }
   static constexpr int stride(int k) { return 2 * (C(k) / 2) + C(k) % 2; }
   static constexpr int base(int k) {
     int b = 0;
     for (int j = 0; j < k; ++j) b += ((R(j) + 1) / 2) * stride(j);
     return b;
   }
-  static constexpr int kSize = base(4);
+  static constexpr int kWeights = base(5);  // then the p + 3 Gauss weights
+  static constexpr int kSize = kWeights + P + 3;
   double v[kSize];
 };
 template <int P>
 constexpr EoTable<P> make_eo_table() {
   EoTable<P> t{};
-  for (int k = 0; k < 4; ++k) {
+  for (int q = 0; q < P + 3; ++q) t.v[EoTable<P>::kWeights + q] = SfC<P>::v.w[q];
+  for (int k = 0; k < 5; ++k) {
     const int r = EoTable<P>::R(k), c = EoTable<P>::C(k), st = EoTable<P>::stride(k);
     for (int i = 0; i < (r + 1) / 2; ++i) {
       double* row = t.v + EoTable<P>::base(k) + i * st;
@@ -677,7 +654,8 @@ constexpr EoTable<P> make_eo_table() {
         return k == 0   ? SfC<P>::v.L[ii * (P + 1) + jj]
                : k == 1 ? SfC<P>::v.L[jj * (P + 1) + ii]
                : k == 2 ? SfC<P>::v.M[ii * (P + 1) + jj]
-                        : SfC<P>::v.D[ii * (P + 1) + jj];
+               : k == 3 ? SfC<P>::v.D[ii * (P + 1) + jj]
+                        : SfC<P>::v.E[ii * (P + 3) + jj];
       };
       for (int j = 0; j < c / 2; ++j) {
         row[j] = 0.5 * (at(i, j) + at(i, c - 1 - j));
@@ -697,439 +675,6 @@ __constant__ EoTable<2> kEo2;
 __constant__ EoTable<3> kEo3;
 __constant__ EoTable<4> kEo4;
 __constant__ EoTable<5> kEo5;
-// Coefficient W (0 even, 1 odd, 2 middle) of row I, column J of operator A:
-// an immediate in FP32, a scalar load from the table eo (EoTable<P>::v) in FP64.
-template <typename T, class A, int I, int J, int W>
-__device__ inline T eo_coef(const double* __restrict__ eo) {
-  if constexpr (std::is_same<T, double>::value) {
-    using E = EoTable<A::kP>;
-    constexpr int c = E::C(A::kK);
-    constexpr int idx = E::base(A::kK) + I * E::stride(A::kK) +
-                        (W == 0 ? J : W == 1 ? c / 2 + J : 2 * (c / 2));
-    return eo[idx];
-  } else if constexpr (W == 0) {
-    return eo_even<T, A, I, J>();
-  } else if constexpr (W == 1) {
-    return eo_odd<T, A, I, J>();
-  } else {
-    return eo_mid<T, A, I>();
-  }
-}
-template <int C, typename T, int VC>
-__device__ inline void eo_split(const Pack<T, VC> (&x)[C], Pack<T, VC> (&xp)[(C + 1) / 2],
-                                Pack<T, VC> (&xm)[C / 2]) {
-#pragma unroll
-  for (int j = 0; j < C / 2; ++j)
-#pragma unroll
-    for (int u = 0; u < VC; ++u) {
-      xp[j].v[u] = x[j].v[u] + x[C - 1 - j].v[u];
-      xm[j].v[u] = x[j].v[u] - x[C - 1 - j].v[u];
-    }
-  if constexpr (C % 2 == 1) xp[C / 2] = x[C / 2];
-}
-// Adds row I's even and odd sums of A applied to the split input (xp, xm).
-template <typename T, class A, int I, int VC>
-__device__ inline void eo_row(const Pack<T, VC> (&xp)[(A::C + 1) / 2],
-                              const Pack<T, VC> (&xm)[A::C / 2], Pack<T, VC>& e,
-                              Pack<T, VC>& o, const double* __restrict__ eo) {
-  static_for<0, A::C / 2>([&](auto j) {
-    constexpr int J = decltype(j)::value;
-    pack_fma(e, eo_coef<T, A, I, J, 0>(eo), xp[J]);
-    if constexpr (2 * I + 1 != A::R) pack_fma(o, eo_coef<T, A, I, J, 1>(eo), xm[J]);
-  });
-  if constexpr (A::C % 2 == 1) pack_fma(e, eo_coef<T, A, I, 0, 2>(eo), xp[A::C / 2]);
-}
-// The R outputs of one or more even-odd contractions: rows(i, e, o) adds the
-// sums of row i, put(i, y) receives output i (i an integral constant).
-template <int R, typename T, int VC, typename Rows, typename Put>
-__device__ inline void eo_out(Rows&& rows, Put&& put) {
-  static_for<0, (R + 1) / 2>([&](auto i) {
-    constexpr int I = decltype(i)::value;
-    Pack<T, VC> e, o;
-    pack_zero(e);
-    pack_zero(o);
-    rows(i, e, o);
-    if constexpr (2 * I + 1 == R) {
-      put(i, e);
-    } else {
-      Pack<T, VC> y0, y1;
-#pragma unroll
-      for (int u = 0; u < VC; ++u) {
-        y0.v[u] = e.v[u] + o.v[u];
-        y1.v[u] = e.v[u] - o.v[u];
-      }
-      put(i, y0);
-      put(ic<R - 1 - I>{}, y1);
-    }
-  });
-}
-#define IDFT_IC(x) decltype(x)::value
-// Entry A of a line from its even-odd split (eo_split): the inverse of the
-// split, to rounding.
-template <int C, int A, typename T, int VC>
-__device__ inline T eo_unsplit(const Pack<T, VC> (&xp)[(C + 1) / 2], const Pack<T, VC> (&xm)[C / 2],
-                               int u) {
-  if constexpr (2 * A + 1 == C) {
-    return xp[A].v[u];
-  } else if constexpr (A < C / 2) {
-    return T(0.5) * (xp[A].v[u] + xm[A].v[u]);
-  } else {
-    constexpr int J = C - 1 - A;
-    return T(0.5) * (xp[J].v[u] - xm[J].v[u]);
-  }
-}
-
-// KIN = false: the potential chain alone on the unscaled input (S unused):
-// Yc = Lq^T diag(w_e) Lq X_e, the quadrature operator of a weight (stages 1 and
-// 4 to 8).  wstride: the weights' step from cell to cell (0: the same weights
-// in every cell); ldx: the row length of X (B, or more for a block of columns).
-template <typename T, typename TV, int P, int CG, int VC, bool XN, bool KIN>
-__global__ __launch_bounds__(kThreads) void k_cell_sf(Geo g, T hq, const T* __restrict__ W,
-                                                      uint32_t wstride, const T* __restrict__ S,
-                                                      const TV* __restrict__ X, uint32_t ldx,
-                                                      const double* __restrict__ xn,
-                                                      const double* __restrict__ xcol,
-                                                      T* __restrict__ Yc, int B,
-                                                      double* __restrict__ dotp,
-                                                      const double* __restrict__ eo) {
-  constexpr int N1 = P + 1, Q = P + 3, N2 = N1 * N1, NE = N2 * N1, Q2 = Q * Q;
-  constexpr int QP = Q | 1, N1P = N1 | 1, NV = CG / VC;
-  // x-line items per thread (lines x column packs over the work-group)
-  constexpr int KI = (N2 * NV + kThreads - 1) / kThreads;
-  typedef Pack<T, VC> pk;
-  typedef SfTab<P, 0> TL;
-  typedef SfTab<P, 1> TLt;
-  typedef SfTab<P, 2> TM;
-  typedef SfTab<P, 3> TD;
-  // regions, each [entry][NV] packs:
-  //   A  [(c,b)][N1P]      ka -> k1 -> yk            (kinetic chain, in place)
-  //   Bk [(c,b)][N1P]      kb -> k2                  (stages 1-3)
-  //   D  [c][Q][QS]        t1 -> t2 -> s2 -> s1      (stages 4-8, over Bk)
-  // SWZ: D unpadded (QS = Q = 8), entry (c, y, x) at slot x ^ y of its line
-  constexpr bool SWZ = sizeof(T) == 8 && Q == 8;
-  constexpr int QS = SWZ ? Q : QP;
-  __shared__ __align__(16) pk rA[KIN ? N2 * N1P * NV : 1];
-  __shared__ __align__(16) pk rBD[cmax(KIN ? N2 * N1P : 0, N1 * Q * QS) * NV];
-  pk* const rB = rBD;
-  // Byte offsets into D of entry (c, y, x), column pack jv, from a per-item
-  // base and the one index that is a compile-time constant at the access
-  // (so that the rest folds into the LDS instruction's offset field):
-  //   dy(c, x, jv) then at_y(base, y);  dx(c, y, jv) then at_x(base, x);
-  //   dc(y, x, jv) then at_c(base, c).
-  // With SWZ the slot x ^ y is an XOR of the offset's slot bits (the slot
-  // field, NV sizeof(pk) bytes per slot and 8 slots, holds no other bits).
-  constexpr uint32_t SB = NV * sizeof(pk);
-  const auto dy = [](uint32_t c, uint32_t x, uint32_t jv) -> uint32_t {
-    return (c * Q * QS + x) * SB + jv * (uint32_t)sizeof(pk);
-  };
-  const auto at_y = [](uint32_t base, uint32_t y) -> uint32_t {
-    return SWZ ? (base ^ (y * SB)) + y * QS * SB : base + y * QS * SB;
-  };
-  const auto dx = [](uint32_t c, uint32_t y, uint32_t jv) -> uint32_t {
-    return ((c * Q + y) * QS + (SWZ ? y : 0u)) * SB + jv * (uint32_t)sizeof(pk);
-  };
-  const auto at_x = [](uint32_t base, uint32_t x) -> uint32_t {
-    return SWZ ? base ^ (x * SB) : base + x * SB;
-  };
-  const auto dc = [](uint32_t y, uint32_t x, uint32_t jv) -> uint32_t {
-    return (y * QS + (SWZ ? (x ^ y) : x)) * SB + jv * (uint32_t)sizeof(pk);
-  };
-  const auto at_c = [](uint32_t base, uint32_t c) -> uint32_t { return base + c * Q * QS * SB; };
-  char* const rDb = reinterpret_cast<char*>(rBD);
-  const auto dref = [rDb](uint32_t off) -> pk& { return *reinterpret_cast<pk*>(rDb + off); };
-  // (cell, column group) pairs dealt to the 8 XCDs in contiguous runs, the
-  // groups of one cell at consecutive slots of one XCD, so that they share
-  // that XCD's L2 for the cell's rows of X and of the cell scratch (each group
-  // holds CG of the B columns of a row).  Every index below fits in 32 bits
-  // (the host checks N B and cells n_e B against 2^32).
-  const uint32_t ncell = (uint32_t)g.ncell, nc = (uint32_t)g.nc, np = (uint32_t)g.p;
-  const uint32_t NN = (uint32_t)g.N1, ub = (uint32_t)B;
-  const uint32_t ngrp = (ub + CG - 1) / CG, npair = ncell * ngrp;
-  const uint32_t per = (npair + 7) / 8;
-  const uint32_t k = (blockIdx.x % 8) * per + blockIdx.x / 8;
-  if (k >= npair) return;
-  const uint32_t e = k / ngrp;
-  const int c0 = (int)(k % ngrp) * CG;
-  const int bw = min(CG, B - c0);
-  const int tid = threadIdx.x;
-  const uint32_t cx = e % nc, cy = (e / nc) % nc, cz = e / (nc * nc);
-  const T* we = W + (size_t)e * wstride;
-  // the column scales of this thread's columns (every item of a thread has
-  // column pack jv = tid % NV, since kThreads is a multiple of NV), loaded
-  // first: a later load would make their first use wait for the weights too
-  double xcl[VC];
-#pragma unroll
-  for (int u = 0; u < VC; ++u) {
-    const int j = min((tid % NV) * VC + u, bw - 1);
-    xcl[u] = xcol ? xcol[c0 + j] : 1.0;
-  }
-  // the quadrature weights of this thread's stage-6 items, loaded now so that
-  // their latency hides behind stages 1-5 (item it6 = tid + k6 kThreads takes
-  // w_e[qz][ln6] for its line ln6 = it6 / NV)
-  constexpr int K6 = (Q2 * NV + kThreads - 1) / kThreads;
-  T wpre[K6][Q];
-#pragma unroll
-  for (int k6 = 0; k6 < K6; ++k6) {
-    const int it6 = tid + k6 * kThreads;
-    const int ln6 = it6 < Q2 * NV ? it6 / NV : 0;
-#pragma unroll
-    for (int qz = 0; qz < Q; ++qz) wpre[k6][qz] = we[qz * Q2 + ln6];
-  }
-  // the input lines stay in registers from stage 1 to stage 4 (even-odd split)
-  pk keep_p[KI][(N1 + 1) / 2], keep_m[KI][N1 / 2];
-  // stage 1: x lines ln = c*N1 + b of the gathered input -> ka = M x, kb = D x
-#pragma unroll
-  for (int ki = 0; ki < KI; ++ki) {
-    const int it = tid + ki * kThreads;
-    if (it >= N2 * NV) break;
-    const int jv = it % NV, ln = it / NV;
-    pk v[N1];
-    const uint32_t b = ln % N1, c = ln / N1;
-    const uint32_t n0 = ((cz * np + c) * NN + (cy * np + b)) * NN + cx * np;
-    // the line's N1 nodes are consecutive: one base pointer per array, the
-    // nodes at immediate offsets (the X rows B apart).  All loads of the line
-    // are issued before the first product (the node scale xn is a
-    // compile-time choice, so no branch separates them).
-    const T* Sp = KIN ? S + n0 : nullptr;
-#pragma unroll
-    for (int u = 0; u < VC; ++u) {
-      const int j = jv * VC + u;
-      if (j < bw) {
-        const TV* Xp = X + (size_t)n0 * ldx + (uint32_t)(c0 + j);
-        const double xc = xcl[u];
-        T sv[N1];
-        TV xv[N1];
-        double nv[N1];
-#pragma unroll
-        for (int a = 0; a < N1; ++a) {
-          if constexpr (KIN) sv[a] = Sp[a];
-          xv[a] = Xp[(size_t)a * ldx];
-          if constexpr (XN) nv[a] = xn[n0 + a];
-          else nv[a] = 1.0;
-        }
-#pragma unroll
-        for (int a = 0; a < N1; ++a) {
-          if constexpr (!KIN) {
-            v[a].v[u] = (T)xv[a];
-          } else if constexpr (std::is_same<T, TV>::value) {
-            T x = sv[a] * xv[a];
-            if constexpr (XN) x *= (T)nv[a];
-            if (xcol) x *= (T)xc;
-            v[a].v[u] = x;
-          } else {  // wider input vectors: scale in FP64, round once
-            double x = (double)sv[a] * (double)xv[a];
-            if constexpr (XN) x *= nv[a];
-            if (xcol) x *= xc;
-            v[a].v[u] = (T)x;
-          }
-        }
-      } else {
-#pragma unroll
-        for (int a = 0; a < N1; ++a) v[a].v[u] = T(0);
-      }
-    }
-    eo_split(v, keep_p[ki], keep_m[ki]);
-    if constexpr (!KIN) continue;
-    eo_out<N1, T, VC>(
-        [&](auto i, pk& s, pk& d) { eo_row<T, TM, IDFT_IC(i)>(keep_p[ki], keep_m[ki], s, d, eo); },
-        [&](auto a2, const pk& r) { rA[(ln * N1P + IDFT_IC(a2)) * NV + jv] = r; });
-    eo_out<N1, T, VC>(
-        [&](auto i, pk& s, pk& d) { eo_row<T, TD, IDFT_IC(i)>(keep_p[ki], keep_m[ki], s, d, eo); },
-        [&](auto a2, const pk& r) { rB[(ln * N1P + IDFT_IC(a2)) * NV + jv] = r; });
-  }
-  if constexpr (KIN) {
-  __syncthreads();
-  // stage 2: y lines (c, a) of the kinetic chain, in place:
-  // k1 = M ka (over ka), k2 = D ka + M kb (over kb)
-  for (int it = tid; it < N2 * NV; it += kThreads) {
-    const int jv = it % NV, l2 = it / NV;
-    const int a = l2 % N1, c = l2 / N1;
-    pk va[N1], vb[N1], ap[(N1 + 1) / 2], am[N1 / 2], bp[(N1 + 1) / 2], bm[N1 / 2];
-#pragma unroll
-    for (int b = 0; b < N1; ++b) {
-      va[b] = rA[((c * N1 + b) * N1P + a) * NV + jv];
-      vb[b] = rB[((c * N1 + b) * N1P + a) * NV + jv];
-    }
-    eo_split(va, ap, am);
-    eo_split(vb, bp, bm);
-    eo_out<N1, T, VC>(
-        [&](auto i, pk& s, pk& d) { eo_row<T, TM, IDFT_IC(i)>(ap, am, s, d, eo); },
-        [&](auto b2, const pk& r) { rA[((c * N1 + IDFT_IC(b2)) * N1P + a) * NV + jv] = r; });
-    eo_out<N1, T, VC>(
-        [&](auto i, pk& s, pk& d) {
-          eo_row<T, TD, IDFT_IC(i)>(ap, am, s, d, eo);
-          eo_row<T, TM, IDFT_IC(i)>(bp, bm, s, d, eo);
-        },
-        [&](auto b2, const pk& r) { rB[((c * N1 + IDFT_IC(b2)) * N1P + a) * NV + jv] = r; });
-  }
-  __syncthreads();
-  // stage 3: z lines (b, a) of the kinetic chain: yk = D k1 + M k2 (over k1)
-  for (int it = tid; it < N2 * NV; it += kThreads) {
-    const int jv = it % NV, l2 = it / NV;  // l2 = b * N1 + a
-    const int a = l2 % N1, b = l2 / N1;
-    pk v1[N1], v2[N1], p1[(N1 + 1) / 2], m1[N1 / 2], p2[(N1 + 1) / 2], m2[N1 / 2];
-#pragma unroll
-    for (int c = 0; c < N1; ++c) {
-      v1[c] = rA[((c * N1 + b) * N1P + a) * NV + jv];
-      v2[c] = rB[((c * N1 + b) * N1P + a) * NV + jv];
-    }
-    eo_split(v1, p1, m1);
-    eo_split(v2, p2, m2);
-    eo_out<N1, T, VC>(
-        [&](auto i, pk& s, pk& d) {
-          eo_row<T, TD, IDFT_IC(i)>(p1, m1, s, d, eo);
-          eo_row<T, TM, IDFT_IC(i)>(p2, m2, s, d, eo);
-        },
-        [&](auto c2, const pk& r) { rA[((IDFT_IC(c2) * N1 + b) * N1P + a) * NV + jv] = r; });
-  }
-  __syncthreads();
-  }
-  // stage 4: x lines of the potential chain from the kept input:
-  // t1[c][b][qx] = Lq x (over k2, which stage 3 has consumed)
-#pragma unroll
-  for (int ki = 0; ki < KI; ++ki) {
-    const int it = tid + ki * kThreads;
-    if (it >= N2 * NV) break;
-    const int jv = it % NV, ln = it / NV;
-    const int b = ln % N1, c = ln / N1;
-    const uint32_t base = dx(c, b, jv);
-    eo_out<Q, T, VC>(
-        [&](auto i, pk& s, pk& d) { eo_row<T, TL, IDFT_IC(i)>(keep_p[ki], keep_m[ki], s, d, eo); },
-        [&](auto q, const pk& r) { dref(at_x(base, IDFT_IC(q))) = r; });
-  }
-  __syncthreads();
-  // stage 5: y lines (c, qx): t2[c][qy][qx] = Lq t1, in place (over t1)
-  for (int it = tid; it < N1 * Q * NV; it += kThreads) {
-    const int jv = it % NV, ln = it / NV;
-    const int qx = ln % Q, c = ln / Q;
-    const uint32_t base = dy(c, qx, jv);
-    pk v[N1], vp[(N1 + 1) / 2], vm[N1 / 2];
-#pragma unroll
-    for (int b = 0; b < N1; ++b) v[b] = dref(at_y(base, b));
-    eo_split(v, vp, vm);
-    eo_out<Q, T, VC>(
-        [&](auto i, pk& s, pk& d) { eo_row<T, TL, IDFT_IC(i)>(vp, vm, s, d, eo); },
-        [&](auto qy, const pk& r) { dref(at_y(base, IDFT_IC(qy))) = r; });
-  }
-  __syncthreads();
-  // stage 6: z lines (qy, qx) through the quadrature weights, in place:
-  // s2 = Lq^T (w .* (Lq t2)) (over t2)
-#pragma unroll
-  for (int k6 = 0; k6 < K6; ++k6) {
-    const int it = tid + k6 * kThreads;
-    if (it >= Q2 * NV) break;
-    const int jv = it % NV, ln = it / NV;  // ln = qy * Q + qx
-    const int qx = ln % Q, qy = ln / Q;
-    const uint32_t base = dc(qy, qx, jv);
-    pk v[N1], vp[(N1 + 1) / 2], vm[N1 / 2];
-#pragma unroll
-    for (int c = 0; c < N1; ++c) v[c] = dref(at_c(base, c));
-    eo_split(v, vp, vm);
-    pk u[Q], up[(Q + 1) / 2], um[Q / 2];
-    eo_out<Q, T, VC>([&](auto i, pk& s, pk& d) { eo_row<T, TL, IDFT_IC(i)>(vp, vm, s, d, eo); },
-                     [&](auto qz, const pk& r) {
-                       const T wq = wpre[k6][IDFT_IC(qz)];
-#pragma unroll
-                       for (int uu = 0; uu < VC; ++uu) u[IDFT_IC(qz)].v[uu] = r.v[uu] * wq;
-                     });
-    eo_split(u, up, um);
-    eo_out<N1, T, VC>([&](auto i, pk& s, pk& d) { eo_row<T, TLt, IDFT_IC(i)>(up, um, s, d, eo); },
-                      [&](auto c, const pk& r) { dref(at_c(base, IDFT_IC(c))) = r; });
-  }
-  __syncthreads();
-  // stage 7: y lines back (c, qx), in place: s1[c][b][qx] = Lq^T s2 (over s2)
-  for (int it = tid; it < N1 * Q * NV; it += kThreads) {
-    const int jv = it % NV, ln = it / NV;
-    const int qx = ln % Q, c = ln / Q;
-    const uint32_t base = dy(c, qx, jv);
-    pk v[Q], vp[(Q + 1) / 2], vm[Q / 2];
-#pragma unroll
-    for (int qy = 0; qy < Q; ++qy) v[qy] = dref(at_y(base, qy));
-    eo_split(v, vp, vm);
-    eo_out<N1, T, VC>(
-        [&](auto i, pk& s, pk& d) { eo_row<T, TLt, IDFT_IC(i)>(vp, vm, s, d, eo); },
-        [&](auto b, const pk& r) { dref(at_y(base, IDFT_IC(b))) = r; });
-  }
-  __syncthreads();
-  // stage 8: x lines back (c, b) plus the kinetic part, into the cell scratch;
-  // with dotp (node-scaled MINRES inputs only, XN), also the cell's x.(H_e x)
-  // per column, into dotp[column * ncell + cell] (x from the kept input lines:
-  // each item holds the same line as in stage 1)
-  double dotv[VC];
-#pragma unroll
-  for (int u = 0; u < VC; ++u) dotv[u] = 0.0;
-#pragma unroll
-  for (int ki = 0; ki < KI; ++ki) {
-    const int it = tid + ki * kThreads;
-    if (it >= N2 * NV) break;
-    const int jv = it % NV, ln = it / NV;
-    if (jv * VC >= bw) continue;
-    const int b = ln % N1, c = ln / N1;
-    const uint32_t base = dx(c, b, jv);
-    pk v[Q], vp[(Q + 1) / 2], vm[Q / 2];
-#pragma unroll
-    for (int qx = 0; qx < Q; ++qx) v[qx] = dref(at_x(base, qx));
-    eo_split(v, vp, vm);
-    T* yp = Yc + (size_t)((e * NE + ln * N1) * ub + c0 + jv * VC);
-    eo_out<N1, T, VC>([&](auto i, pk& s, pk& d) { eo_row<T, TLt, IDFT_IC(i)>(vp, vm, s, d, eo); },
-                      [&](auto a, const pk& r) {
-                        constexpr int A = IDFT_IC(a);
-                        pk kin;
-                        if constexpr (KIN) kin = rA[(ln * N1P + A) * NV + jv];
-#pragma unroll
-                        for (int u = 0; u < VC; ++u) {
-                          T y = r.v[u];
-                          if constexpr (KIN) y = hq * kin.v[u] + y;
-                          if (jv * VC + u < bw) yp[(size_t)A * ub + u] = y;
-                          if constexpr (XN) {
-                            if (dotp)
-                              dotv[u] += (double)eo_unsplit<N1, A>(keep_p[ki], keep_m[ki], u) *
-                                         (double)y;
-                          }
-                        }
-                      });
-  }
-  if (XN && dotp) {
-    // per column jv: the threads tid = jv (mod NV) (kThreads and 64 are
-    // multiples of NV), summed over each wave, then over the 4 waves
-    __syncthreads();  // stage 8 has read rA
-    double* red = reinterpret_cast<double*>(rA);
-    const int lane = tid & 63, wave = tid >> 6;
-#pragma unroll
-    for (int u = 0; u < VC; ++u) {
-      double t = dotv[u];
-#pragma unroll
-      for (int o = 32; o >= NV; o >>= 1) t += __shfl_xor(t, o, 64);
-      if (lane < NV) red[(wave * NV + lane) * VC + u] = t;
-    }
-    __syncthreads();
-    if (tid < NV) {
-#pragma unroll
-      for (int u = 0; u < VC; ++u) {
-        const int j = tid * VC + u;
-        if (j < bw) {
-          double t = 0.0;
-#pragma unroll
-          for (int w = 0; w < kThreads / 64; ++w) t += red[(w * NV + tid) * VC + u];
-          dotp[(size_t)(uint32_t)(c0 + j) * ncell + e] = t;
-        }
-      }
-    }
-  }
-}
-#undef IDFT_IC
-
-// Phase 2: every node sums its contributions from the (at most 8) cells that
-// share it -- found arithmetically on the structured mesh, so no atomics and
-// no colouring -- and combines them with up to three other blocks:
-//   Y = beta Y + alpha S[n] sum + a ca[j] xn[n] X + b cb[j] Z + c cc[j] W
-// (xn, the operator input's node scale, optional).  With `partial`, the
-// per-column block partials of V.Y (FP64) for the scaled operator input
-// V = xcol[j] xn[n] Xin, optionally stored.  Nodes are taken in their
-// linear order n = (iz N1 + iy) N1 + ix: block b covers R consecutive chunks
-// of per = 256 / (B / VW) nodes, [(b R + r) per, (b R + r + 1) per), so a
-// chunk may cross x rows and every lane has work; thread t owns column group
-// t % (B / VW) and position t / (B / VW) within each chunk.
 // Unsigned 32-bit division by a run-time constant d >= 2 through a
 // multiplier computed on the host (Granlund-Montgomery): with
 // s = ceil(log2 d) and m = floor(2^32 (2^s - d) / d) + 1,
@@ -1148,6 +693,430 @@ __device__ inline uint32_t fast_div(uint32_t n, FastDiv f) {
   return (t + ((n - t) >> 1)) >> (f.s - 1);
 }
 
+// x+ and x- of a line (see the even-odd form above).
+template <int C, typename T>
+__device__ inline void pl_split(const T (&x)[C], T (&p)[(C + 1) / 2], T (&m)[C / 2]) {
+#pragma unroll
+  for (int j = 0; j < C / 2; ++j) {
+    p[j] = x[j] + x[C - 1 - j];
+    m[j] = x[j] - x[C - 1 - j];
+  }
+  if constexpr (C % 2 == 1) p[C / 2] = x[C / 2];
+}
+// The even-odd coefficients of operator A for one phase: immediates in FP32; in
+// FP64 one block of scalar registers, loaded together at the phase's start and
+// kept (the empty asm stops the compiler from loading a coefficient again at each
+// use: at 2 waves per SIMD nothing hides those waits).
+template <typename T, class A>
+struct PlCoef {
+  typedef EoTable<A::kP> E;
+  static constexpr bool kTab = sizeof(T) == 8;
+  static constexpr int kMid = A::C % 2 == 1 ? A::C / 2 : -1;  // the middle column
+  static constexpr int kN = ((A::R + 1) / 2) * E::stride(A::kK);
+  T c[kTab ? kN : 1];
+  // after: a value of the phase before.  The offset, a 0 that the compiler does not
+  // see, is tied to it, so that the loads stay behind it: two phases' coefficients
+  // do not fit the scalar registers.
+  __device__ inline PlCoef(const double* __restrict__ eo, T after) {
+    if constexpr (kTab) {
+      int zero = 0;
+      asm("" : "+s"(zero) : "v"(after));
+      static_for<0, kN>([&](auto i) { c[decltype(i)::value] = eo[zero + E::base(A::kK) + decltype(i)::value]; });
+      if constexpr (A::kK != 4)
+        static_for<0, kN>([&](auto i) { asm("" : "+s"(c[decltype(i)::value])); });
+    }
+  }
+  // coefficient W (0 even, 1 odd, 2 middle) of row I, column J
+  template <int I, int J, int W>
+  __device__ inline T at() const {
+    if constexpr (kTab) {
+      constexpr int cc = A::C;
+      return c[I * E::stride(A::kK) + (W == 0 ? J : W == 1 ? cc / 2 + J : 2 * (cc / 2))];
+    } else if constexpr (W == 0) {
+      return eo_even<T, A, I, J>();
+    } else if constexpr (W == 1) {
+      return eo_odd<T, A, I, J>();
+    } else {
+      return eo_mid<T, A, I>();
+    }
+  }
+};
+// The same coefficients read as the transposed operator's (Lq^T from Lq, equal by
+// centro-symmetry).
+template <class CF, int C>
+struct PlTransposed {
+  const CF& f;
+  template <int I, int J, int W>
+  __device__ inline auto at() const {
+    constexpr int row = W == 2 ? C / 2 : J;
+    if constexpr (CF::kMid == I) return f.template at<row, 0, 2>();
+    else return f.template at<row, I, W == 1 ? 1 : 0>();
+  }
+};
+// The even (i < ceil(R/2)) and odd (i < floor(R/2)) halves of A x from x's split:
+// y_i = e_i + o_i, y_{R-1-i} = e_i - o_i, the middle row of an odd R is e alone.
+// ADD: added to what e and o hold.
+template <class A, bool ADD, typename T, class CF>
+__device__ inline void pl_halves(const CF& cf, const T (&p)[(A::C + 1) / 2],
+                                 const T (&m)[A::C / 2], T (&e)[(A::R + 1) / 2],
+                                 T (&o)[A::R / 2]) {
+  static_for<0, (A::R + 1) / 2>([&](auto i) {
+    constexpr int I = decltype(i)::value;
+    T ei = ADD ? e[I] : T(0), oi = T(0);
+    if constexpr (ADD && I < A::R / 2) oi = o[I];
+    static_for<0, A::C / 2>([&](auto j) {
+      constexpr int J = decltype(j)::value;
+      if (!ADD && J == 0) ei = cf.template at<I, J, 0>() * p[J];
+      else ei += cf.template at<I, J, 0>() * p[J];
+      if constexpr (I < A::R / 2) {
+        if (!ADD && J == 0) oi = cf.template at<I, J, 1>() * m[J];
+        else oi += cf.template at<I, J, 1>() * m[J];
+      }
+    });
+    if constexpr (A::C % 2 == 1) ei += cf.template at<I, 0, 2>() * p[A::C / 2];
+    e[I] = ei;
+    if constexpr (I < A::R / 2) o[I] = oi;
+  });
+}
+template <int R, typename T>
+__device__ inline void pl_join(const T (&e)[(R + 1) / 2], const T (&o)[R / 2], T (&y)[R]) {
+#pragma unroll
+  for (int i = 0; i < R / 2; ++i) {
+    y[i] = e[i] + o[i];
+    y[R - 1 - i] = e[i] - o[i];
+  }
+  if constexpr (R % 2 == 1) y[R / 2] = e[R / 2];
+}
+// LDS accesses of one wave complete in order: between phases only the compiler
+// has to be kept from moving them.
+__device__ inline void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// Lanes of a wave: NS (cell, column) slots x Q Gauss planes.
+template <int P>
+struct PlaneLanes {
+  static constexpr int Q = P + 3, NS = 64 / Q;
+};
+// Plane stride in LDS: N1^2 lines of NS entries, padded so that plane r of slot s
+// starts r NS + s banks on, as in the line phases.
+template <typename T, int P>
+struct PlaneStride {
+  static constexpr int NS = PlaneLanes<P>::NS, L = (P + 1) * (P + 1) * NS;
+  static constexpr int M = 256 / (int)sizeof(T);
+  static constexpr int v = L + ((NS - L) % M + M) % M;
+};
+// KIN = false: the potential chain alone on the unscaled input (S unused):
+// Yc = Lq^T diag(w_e) Lq X_e, the quadrature operator of a weight.  wstride: the
+// weights' step from cell to cell (0: the same weights in every cell); ldx: the row
+// length of X (B, or more for a block of columns).  XN: node-scaled input, and with
+// dotp also each slot's x.(H_e x), dotp[column * ncell + cell].
+template <typename T, typename TV, int P, bool XN, bool KIN>
+__global__ __launch_bounds__(64, 2) void k_cell_plane(
+    Geo g, T hq, const T* __restrict__ W, uint32_t wstride, const T* __restrict__ S,
+    const TV* __restrict__ X, uint32_t ldx, const double* __restrict__ xn,
+    const double* __restrict__ xcol, T* __restrict__ Yc, uint32_t B, FastDiv divB, uint32_t nslot,
+    double* __restrict__ dotp, const double* __restrict__ eo) {
+  constexpr int N1 = P + 1, Q = P + 3, N2 = N1 * N1, NE = N2 * N1, Q2 = Q * Q;
+  constexpr int NS = PlaneLanes<P>::NS, PS = PlaneStride<T, P>::v;
+  constexpr int K3 = (N2 + Q - 1) / Q;  // lines per lane in the line phases
+  constexpr int HE = (N1 + 1) / 2, HO = N1 / 2, QE = (Q + 1) / 2, QO = Q / 2;
+  typedef SfTab<P, 0> TL;
+  typedef SfTab<P, 1> TLt;
+  typedef SfTab<P, 2> TM;
+  typedef SfTab<P, 3> TD;
+  typedef SfTab<P, 4> TE;
+  __shared__ __align__(16) T lds[Q * PS];
+  const uint32_t lane = threadIdx.x;
+  if (lane >= NS * Q) return;
+  const uint32_t r = lane / NS, slot = lane % NS;
+  const uint32_t nwave = (nslot + NS - 1) / NS, per = (nwave + 7) / 8;
+  const uint32_t kw = (blockIdx.x % 8) * per + blockIdx.x / 8;
+  if (kw >= nwave) return;
+  const bool live = kw * NS + slot < nslot;
+  const uint32_t sid = live ? kw * NS + slot : nslot - 1;
+  const uint32_t e = B == 1 ? sid : fast_div(sid, divB), j = sid - e * B;
+  const uint32_t nc = (uint32_t)g.nc, NN = (uint32_t)g.N1;
+  const uint32_t cx = e % nc, cyz = e / nc, cy = cyz % nc, cz = cyz / nc;
+  const uint32_t n00 = (cz * P * NN + cy * P) * NN + cx * P;
+  const uint32_t NNN = NN * NN;
+  const T* we = W + (size_t)e * wstride + r * Q2;
+  const double xc = xcol ? xcol[j] : 1.0;
+  const T wg = KIN ? (T)eo[EoTable<P>::kWeights + r] : T(0);
+  // the input of line l of this lane, scaled
+  const auto load_line = [&](uint32_t l, T(&v)[N1]) {
+    const uint32_t n0 = n00 + (l / N1) * NN + l % N1;
+    T sv[N1];
+    TV xv[N1];
+    double nv[N1];
+#pragma unroll
+    for (int c = 0; c < N1; ++c) {
+      const uint32_t n = n0 + c * NNN;
+      xv[c] = X[(size_t)n * ldx + j];
+      if constexpr (KIN) sv[c] = S[n];
+      if constexpr (XN) nv[c] = xn[n];
+    }
+#pragma unroll
+    for (int c = 0; c < N1; ++c) {
+      if constexpr (!KIN) {
+        v[c] = (T)xv[c];
+      } else if constexpr (std::is_same<T, TV>::value) {
+        T x = sv[c] * xv[c];
+        if constexpr (XN) x *= (T)nv[c];
+        v[c] = x * (T)xc;
+      } else {
+        double x = (double)sv[c] * (double)xv[c];
+        if constexpr (XN) x *= nv[c];
+        v[c] = (T)(x * xc);
+      }
+    }
+  };
+  // line index of round k (rounds past the last line repeat it)
+  const auto line_of = [&](int k) -> uint32_t {
+    const uint32_t l = r + Q * k;
+    return l < (uint32_t)N2 ? l : (uint32_t)N2 - 1;
+  };
+  // z lines: u[q] = Lq x for the Q planes
+  T after = T(0);
+  const PlCoef<T, TL> fL0(eo, T(0));
+#pragma unroll
+  for (int k = 0; k < K3; ++k) {
+    const uint32_t l = line_of(k);
+    T v[N1], vp[HE], vm[HO], oe[QE], oo[QO], u[Q];
+    load_line(l, v);
+    pl_split<N1>(v, vp, vm);
+    pl_halves<TL, false>(fL0, vp, vm, oe, oo);
+    pl_join<Q>(oe, oo, u);
+#pragma unroll
+    for (int q = 0; q < Q; ++q) lds[q * PS + l * NS + slot] = u[q];
+    after = u[0];
+  }
+  wave_lds_fence();
+  // this lane's plane: entries (b, a) at pl[(b N1 + a) NS]
+  T* const pl = lds + r * PS + slot;
+  T me[N1][HE], mo[N1][HO];  // m = M (x) M u, even and odd in x
+  T pe[N1][HE], po[N1][HO];  // the plane operator's result
+  const auto u_line = [&](const T* pu, int b, T(&p)[HE], T(&m)[HO]) {
+    T v[N1];
+#pragma unroll
+    for (int a = 0; a < N1; ++a) v[a] = pu[(a * N1 + b) * NS];
+    pl_split<N1>(v, p, m);
+  };
+  if constexpr (KIN) {
+    const PlCoef<T, TM> fM(eo, after);
+    const PlCoef<T, TD> fD(eo, after);
+    const T wk = hq * wg;
+#pragma unroll
+    for (int b = 0; b < N1; ++b) {
+      T p[HE], m[HO];
+      u_line(pl, b, p, m);
+      pl_halves<TM, false>(fM, p, m, me[b], mo[b]);
+      pl_halves<TD, false>(fD, p, m, pe[b], po[b]);
+    }
+    // y columns of M x (ca) and D x (cb), in place: m = M ca, k2 = D ca + M cb
+    const auto kin_column = [&](auto ca, auto cb) {
+      T a[N1], d[N1], ap[HE], am[HO], dp[HE], dm[HO], oe[HE], oo[HO], y[N1];
+#pragma unroll
+      for (int b = 0; b < N1; ++b) { a[b] = ca(b); d[b] = cb(b); }
+      pl_split<N1>(a, ap, am);
+      pl_split<N1>(d, dp, dm);
+      pl_halves<TM, false>(fM, ap, am, oe, oo);
+      pl_join<N1>(oe, oo, y);
+#pragma unroll
+      for (int b = 0; b < N1; ++b) ca(b) = y[b];
+      pl_halves<TD, false>(fD, ap, am, oe, oo);
+      pl_halves<TM, true>(fM, dp, dm, oe, oo);
+      pl_join<N1>(oe, oo, y);
+#pragma unroll
+      for (int b = 0; b < N1; ++b) cb(b) = wk * y[b];
+    };
+#pragma unroll
+    for (int i = 0; i < HE; ++i)
+      kin_column([&](int b) -> T& { return me[b][i]; }, [&](int b) -> T& { return pe[b][i]; });
+#pragma unroll
+    for (int i = 0; i < HO; ++i)
+      kin_column([&](int b) -> T& { return mo[b][i]; }, [&](int b) -> T& { return po[b][i]; });
+  } else {
+#pragma unroll
+    for (int b = 0; b < N1; ++b) {
+#pragma unroll
+      for (int i = 0; i < HE; ++i) pe[b][i] = T(0);
+#pragma unroll
+      for (int i = 0; i < HO; ++i) po[b][i] = T(0);
+    }
+  }
+  const PlCoef<T, TL> fL(eo, KIN ? pe[N1 - 1][HE - 1] : after);
+  const PlTransposed<PlCoef<T, TL>, Q> fLt{fL};
+  // a Gauss line of the plane through its weights, in place: c <- Lq^T (w .* (Lq c))
+  const auto gauss_line = [&](T(&c)[N1], const T(&wq)[Q]) {
+    T cp[HE], cm[HO], oe[QE], oo[QO], t[Q], tp[QE], tm[QO], re[HE], ro[HO];
+    pl_split<N1>(c, cp, cm);
+    pl_halves<TL, false>(fL, cp, cm, oe, oo);
+    pl_join<Q>(oe, oo, t);
+#pragma unroll
+    for (int q = 0; q < Q; ++q) t[q] *= wq[q];
+    pl_split<Q>(t, tp, tm);
+    pl_halves<TLt, false>(fLt, tp, tm, re, ro);
+    pl_join<N1>(re, ro, c);
+  };
+  // the kinetic FP64 kernel at p = 5 reads the plane again for each pair of Gauss
+  // lines: its registers do not hold u, m and p at once (keeping u spills, 477
+  // against 233 us at 24 cells, B = 12)
+  constexpr bool REREAD = KIN && sizeof(T) == 8 && P == 5;
+  T up[REREAD ? 1 : N1][HE], um[REREAD ? 1 : N1][HO];
+  if constexpr (!REREAD) {
+#pragma unroll
+    for (int b = 0; b < N1; ++b) u_line(pl, b, up[b], um[b]);
+  }
+  uint32_t again = 0;  // a 0 the compiler does not see: the plane is read again, not kept
+  static_for<0, QE>([&](auto kk) {
+    constexpr int k = decltype(kk)::value;
+    constexpr bool mid = 2 * k + 1 == Q;
+    if constexpr (REREAD) asm("" : "+v"(again));
+    T w0[Q], w1[Q];
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      w0[q] = we[k * Q + q];
+      w1[q] = we[(Q - 1 - k) * Q + q];
+    }
+    T c0[N1], c1[N1];
+#pragma unroll
+    for (int b = 0; b < N1; ++b) {
+      T tp[HE], tm[HO];
+      if constexpr (REREAD) {
+        u_line(pl + again, b, tp, tm);
+      } else {
+#pragma unroll
+        for (int i = 0; i < HE; ++i) tp[i] = up[b][i];
+#pragma unroll
+        for (int i = 0; i < HO; ++i) tm[i] = um[b][i];
+      }
+      T ev = T(0), ov = T(0);
+      static_for<0, HO>([&](auto jj) {
+        constexpr int J = decltype(jj)::value;
+        ev += fL.template at<k, J, 0>() * tp[J];
+        if constexpr (!mid) ov += fL.template at<k, J, 1>() * tm[J];
+      });
+      if constexpr (N1 % 2 == 1) ev += fL.template at<k, 0, 2>() * tp[HE - 1];
+      c0[b] = ev + ov;
+      c1[b] = ev - ov;
+    }
+    gauss_line(c0, w0);
+    if constexpr (!mid) gauss_line(c1, w1);
+#pragma unroll
+    for (int b = 0; b < N1; ++b) {
+      const T sp = mid ? c0[b] : c0[b] + c1[b], sm = c0[b] - c1[b];
+      static_for<0, HE>([&](auto ii) {
+        constexpr int I = decltype(ii)::value;
+        pe[b][I] += fLt.template at<I, k, mid ? 2 : 0>() * sp;
+        if constexpr (!mid && I < HO) po[b][I] += fLt.template at<I, k, 1>() * sm;
+      });
+    }
+  });
+  const auto put_plane = [&](T(&ve)[N1][HE], T(&vo)[N1][HO]) {
+#pragma unroll
+    for (int b = 0; b < N1; ++b) {
+      T y[N1];
+      pl_join<N1>(ve[b], vo[b], y);
+#pragma unroll
+      for (int a = 0; a < N1; ++a) pl[(a * N1 + b) * NS] = y[a];
+    }
+  };
+  put_plane(pe, po);
+  wave_lds_fence();
+  // z lines back: y = Lq^T p + E m
+  T ze[K3][HE], zo[K3][HO];
+#pragma unroll
+  for (int k = 0; k < K3; ++k) {
+    const uint32_t l = line_of(k);
+    T v[Q], vp[QE], vm[QO];
+#pragma unroll
+    for (int q = 0; q < Q; ++q) v[q] = lds[q * PS + l * NS + slot];
+    pl_split<Q>(v, vp, vm);
+    pl_halves<TLt, false>(fLt, vp, vm, ze[k], zo[k]);
+  }
+  if constexpr (KIN) {
+    // the sums are complete here, before E's coefficients take Lq's registers
+    if constexpr (sizeof(T) == 8) {
+#pragma unroll
+      for (int k = 0; k < K3; ++k) {
+#pragma unroll
+        for (int i = 0; i < HE; ++i) asm volatile("" : "+v"(ze[k][i]));
+#pragma unroll
+        for (int i = 0; i < HO; ++i) asm volatile("" : "+v"(zo[k][i]));
+      }
+    }
+    wave_lds_fence();
+    put_plane(me, mo);
+    wave_lds_fence();
+  }
+  const PlCoef<T, TE> fE(eo, ze[K3 - 1][0]);
+  double dotv = 0.0;
+  T* const yc = Yc + (size_t)e * NE * B + j;
+#pragma unroll
+  for (int k = 0; k < K3; ++k) {
+    const uint32_t l = line_of(k);
+    T xl[N1];
+    if constexpr (XN) {
+      // read again, not kept from the first phase: hidden from the compiler, which
+      // would hold all of this lane's input in registers meanwhile
+      uint32_t l2 = l;
+      asm("" : "+v"(l2));
+      if (dotp) load_line(l2, xl);
+    }
+    if constexpr (KIN) {
+      T v[Q], vp[QE], vm[QO];
+#pragma unroll
+      for (int q = 0; q < Q; ++q) v[q] = lds[q * PS + l * NS + slot];
+      pl_split<Q>(v, vp, vm);
+      T he[HE], ho[HO];
+      pl_halves<TE, false>(fE, vp, vm, he, ho);
+#pragma unroll
+      for (int i = 0; i < HE; ++i) ze[k][i] += hq * he[i];
+#pragma unroll
+      for (int i = 0; i < HO; ++i) zo[k][i] += hq * ho[i];
+    }
+    T y[N1];
+    pl_join<N1>(ze[k], zo[k], y);
+    if (live && r + Q * k < (uint32_t)N2) {
+#pragma unroll
+      for (int c = 0; c < N1; ++c) yc[(size_t)((c * N2 + l) * B)] = y[c];
+      if constexpr (XN) {
+        if (dotp) {
+#pragma unroll
+          for (int c = 0; c < N1; ++c) dotv += (double)xl[c] * (double)y[c];
+        }
+      }
+    }
+  }
+  if constexpr (XN) {
+    if (dotp) {
+      wave_lds_fence();
+      double* red = reinterpret_cast<double*>(lds);
+      red[lane] = dotv;
+      wave_lds_fence();
+      if (r == 0 && live) {
+        double t = 0.0;
+#pragma unroll
+        for (int q = 0; q < Q; ++q) t += red[q * NS + slot];
+        dotp[(size_t)j * (uint32_t)g.ncell + e] = t;
+      }
+    }
+  }
+}
+
+// Phase 2: every node sums its contributions from the (at most 8) cells that
+// share it -- found arithmetically on the structured mesh, so no atomics and
+// no colouring -- and combines them with up to three other blocks:
+//   Y = beta Y + alpha S[n] sum + a ca[j] xn[n] X + b cb[j] Z + c cc[j] W
+// (xn, the operator input's node scale, optional).  With `partial`, the
+// per-column block partials of V.Y (FP64) for the scaled operator input
+// V = xcol[j] xn[n] Xin, optionally stored.  Nodes are taken in their
+// linear order n = (iz N1 + iy) N1 + ix: block b covers R consecutive chunks
+// of per = 256 / (B / VW) nodes, [(b R + r) per, (b R + r + 1) per), so a
+// chunk may cross x rows and every lane has work; thread t owns column group
+// t % (B / VW) and position t / (B / VW) within each chunk.
 // VW consecutive elements of a node-major row (16-byte aligned for VW > 1).
 template <typename T, int VW>
 __device__ inline void vload(const T* __restrict__ p, T (&o)[VW]) {
@@ -2382,11 +2351,9 @@ void launch_build_hamiltonian(const Geo& g, const DevTables& t, double hh, const
   IDFT_HIP(hipGetLastError());
 }
 
-// Columns per work-group (CG) and per item (VC) of the sum-factorised
-// kernel built into the library: CG in {2, 4, 8} (its LDS holds 684 CG
-// values at p = 5, 636 CG in FP64: 40.7 KB at CG = 8), one column per item.  The kernel is
-// written for VC columns per item; wider items and 16-column groups measured
-// slower on every mesh tried and are not instantiated.
+// The sum-factorised kernel takes any block width in one way; its shape arguments
+// (columns per work-group 2, 4 or 8, one column per item) are accepted and change
+// nothing.
 bool sf_cols_supported(int cols, bool) { return cols == 2 || cols == 4 || cols == 8; }
 bool sf_vc_supported(int cols, int vc, bool fp64) {
   return sf_cols_supported(cols, fp64) && vc == 1;
@@ -2394,33 +2361,18 @@ bool sf_vc_supported(int cols, int vc, bool fp64) {
 
 static const double* sf_eo_table(int p);
 
-template <typename T, typename TV, int P, int CG>
-static void cell_sf_cg(const Geo& g, const CellOp<T>& op, const T* S, const TV* X,
-                       const double* xn, const double* xcol, T* Yc, int B, double* dotp,
+template <typename T, typename TV, int P, bool XN, bool KIN>
+static void cell_plane(const Geo& g, T hq, const T* W, uint32_t wstride, const T* S, const TV* X,
+                       int ldx, const double* xn, const double* xcol, T* Yc, int B, double* dotp,
                        hipStream_t s) {
-  check_u32(g.N * B);
+  constexpr int NS = PlaneLanes<P>::NS;
   check_u32(cell_scratch_elems(g, B));
-  const int64_t npair = g.ncell * ((B + CG - 1) / CG);
-  check_u32(8 * ((npair + 7) / 8));
-  dim3 grid((unsigned)(8 * ((npair + 7) / 8))), block(kThreads);
-  const T hq = (T)op.kin_scale;
-  const uint32_t nq = (P + 3) * (P + 3) * (P + 3);
-  const double* eo = sf_eo_table(P);
-  // per-cell dots only with node-scaled inputs (the MINRES steps)
-  if (dotp && !xn) throw Error(IDFT_EINVAL, "per-cell dots need a node-scaled input");
-  // node-scaled inputs (MINRES) come as FP64 vectors; FP32 vectors never
-  // carry a node scale
-  if constexpr (std::is_same<TV, double>::value) {
-    if (xn) {
-      k_cell_sf<T, TV, P, CG, 1, true, true><<<grid, block, 0, s>>>(
-          g, hq, op.W, nq, S, X, (uint32_t)B, xn, xcol, Yc, B, dotp, eo);
-      return;
-    }
-  } else {
-    if (xn) throw Error(IDFT_EINVAL, "node-scaled input needs FP64 vectors");
-  }
-  k_cell_sf<T, TV, P, CG, 1, false, true><<<grid, block, 0, s>>>(
-      g, hq, op.W, nq, S, X, (uint32_t)B, nullptr, xcol, Yc, B, nullptr, eo);
+  const uint32_t nslot = (uint32_t)(g.ncell * B);
+  const uint32_t nwave = (nslot + NS - 1) / NS;
+  const FastDiv divB = make_fastdiv((uint32_t)std::max(B, 2));
+  k_cell_plane<T, TV, P, XN, KIN><<<8 * ((nwave + 7) / 8), 64, 0, s>>>(
+      g, hq, W, wstride, S, X, (uint32_t)ldx, xn, xcol, Yc, (uint32_t)B, divB, nslot, dotp,
+      sf_eo_table(P));
 }
 
 template <typename T, typename TV, int P>
@@ -2430,12 +2382,22 @@ static void cell_sf_p(const Geo& g, const CellOp<T>& op, const T* S, const TV* X
   if (!op.W) throw Error(IDFT_ESTATE, "quadrature weights of the cell operator not set");
   if (!sf_vc_supported(cg, vc, std::is_same<T, double>::value))
     throw Error(IDFT_EINVAL, "shape not supported by the sum-factorised kernel");
-  switch (cg) {
-    case 2: cell_sf_cg<T, TV, P, 2>(g, op, S, X, xn, xcol, Yc, B, dotp, s); break;
-    case 4: cell_sf_cg<T, TV, P, 4>(g, op, S, X, xn, xcol, Yc, B, dotp, s); break;
-    case 8: cell_sf_cg<T, TV, P, 8>(g, op, S, X, xn, xcol, Yc, B, dotp, s); break;
-    default: throw Error(IDFT_EINVAL, "columns per work-group not supported by the sum-factorised kernel");
+  check_u32(g.N * B);
+  const T hq = (T)op.kin_scale;
+  constexpr uint32_t nq = (P + 3) * (P + 3) * (P + 3);
+  // per-cell dots only with node-scaled inputs (the MINRES steps)
+  if (dotp && !xn) throw Error(IDFT_EINVAL, "per-cell dots need a node-scaled input");
+  // node-scaled inputs (MINRES) come as FP64 vectors; FP32 vectors never
+  // carry a node scale
+  if constexpr (std::is_same<TV, double>::value) {
+    if (xn) {
+      cell_plane<T, TV, P, true, true>(g, hq, op.W, nq, S, X, B, xn, xcol, Yc, B, dotp, s);
+      return;
+    }
+  } else {
+    if (xn) throw Error(IDFT_EINVAL, "node-scaled input needs FP64 vectors");
   }
+  cell_plane<T, TV, P, false, true>(g, hq, op.W, nq, S, X, B, nullptr, xcol, Yc, B, nullptr, s);
 }
 
 template <typename T, typename TV, int P>
@@ -2619,22 +2581,6 @@ template int launch_cell_apply<float, double>(const Geo&, const CellOp<float>&, 
                                               const ApplyEpilogue<double>&, const GemmShape&,
                                               hipStream_t);
 
-template <int P>
-static void quad_cells_p(const Geo& g, const double* W, int64_t wstride, const double* X, int ldx,
-                         int wb, double* Yc, int cg, hipStream_t s) {
-  const int64_t npair = g.ncell * ((wb + cg - 1) / cg);
-  check_u32(8 * ((npair + 7) / 8));
-  const unsigned grid = (unsigned)(8 * ((npair + 7) / 8));
-  const double* eo = sf_eo_table(P);
-#define IDFT_QC(CG)                                                                            \
-  k_cell_sf<double, double, P, CG, 1, false, false><<<grid, kThreads, 0, s>>>(                 \
-      g, 0.0, W, (uint32_t)wstride, nullptr, X, (uint32_t)ldx, nullptr, nullptr, Yc, wb, nullptr, eo)
-  if (cg == 2) IDFT_QC(2);
-  else if (cg == 4) IDFT_QC(4);
-  else IDFT_QC(8);
-#undef IDFT_QC
-}
-
 int quad_gather_blocks(const Geo& g, int wb, int vw) {
   unsigned gx, gy;
   uint32_t R;
@@ -2650,8 +2596,6 @@ void launch_quad_pairs(const Geo& g, const double* W, int64_t wstride, const dou
     throw Error(IDFT_EINVAL, "block or pair count out of range");
   check_u32(g.N);
   check_u32(cell_scratch_elems(g, wb));
-  // columns per work-group: the narrowest group that holds a narrow block
-  const int cg = wb <= 2 ? 2 : 4;
   // two columns per 16-byte access where every row starts at an even column
   const int vw = wb % 2 == 0 && (np == 0 || lda % 2 == 0) && (!T2 || ldt % 2 == 0) ? 2 : 1;
   const int nblk = quad_gather_blocks(g, wb, vw);
@@ -2665,7 +2609,8 @@ void launch_quad_pairs(const Geo& g, const double* W, int64_t wstride, const dou
                                                   asc, T2, (uint32_t)ldt, pairs, (uint32_t)np,  \
                                                   partial.p)
 #define IDFT_QP(PP)                                                \
-  quad_cells_p<PP>(g, W, wstride, Bv, ldb, wb, Yc, cg, s);         \
+  cell_plane<double, double, PP, false, false>(g, 0.0, W, (uint32_t)wstride, nullptr, Bv, ldb, nullptr, \
+                                               nullptr, Yc, wb, nullptr, s);                    \
   IDFT_HIP(hipGetLastError());                                     \
   if (vw == 2) IDFT_QG(PP, 2);                                     \
   else IDFT_QG(PP, 1);

@@ -75,6 +75,9 @@ struct SfConst {
   double L[Q * N1];   // L[q][a] = l_a(g_q) at the p+3 Gauss points
   double M[N1 * N1];  // exact 1D mass on [-1, 1]
   double D[N1 * N1];  // exact 1D stiffness on [-1, 1]
+  // D from the Gauss points: E = D (L^T L)^-1 L^T, so that E L = D
+  double E[N1 * Q];
+  double w[Q];  // Gauss weights: L^T diag(w) L = M
 };
 
 template <int P>
@@ -118,6 +121,32 @@ __host__ __device__ constexpr SfConst<P> make_sf_const() {
         t.D[a * N1 + b] += w * lag_d(a, x) * lag_d(b, x);
       }
   }
+  for (int q = 0; q < Q; ++q) {
+    const double x = gq.x[q], d = legendre_c(Q, x).dP;
+    t.w[q] = 2.0 / ((1.0 - x * x) * d * d);
+  }
+  // Z = (L^T L)^-1 D by elimination (positive definite: no pivoting), E = Z^T L^T
+  double G[N1 * N1] = {}, Z[N1 * N1] = {};
+  for (int a = 0; a < N1; ++a)
+    for (int b = 0; b < N1; ++b) {
+      for (int q = 0; q < Q; ++q) G[a * N1 + b] += t.L[q * N1 + a] * t.L[q * N1 + b];
+      Z[a * N1 + b] = t.D[a * N1 + b];
+    }
+  for (int k = 0; k < N1; ++k)
+    for (int i = k + 1; i < N1; ++i) {
+      const double f = G[i * N1 + k] / G[k * N1 + k];
+      for (int j = k; j < N1; ++j) G[i * N1 + j] -= f * G[k * N1 + j];
+      for (int j = 0; j < N1; ++j) Z[i * N1 + j] -= f * Z[k * N1 + j];
+    }
+  for (int i = N1 - 1; i >= 0; --i)
+    for (int j = 0; j < N1; ++j) {
+      double v = Z[i * N1 + j];
+      for (int k = i + 1; k < N1; ++k) v -= G[i * N1 + k] * Z[k * N1 + j];
+      Z[i * N1 + j] = v / G[i * N1 + i];
+    }
+  for (int i = 0; i < N1; ++i)
+    for (int q = 0; q < Q; ++q)
+      for (int a = 0; a < N1; ++a) t.E[i * Q + q] += Z[a * N1 + i] * t.L[q * N1 + a];
   return t;
 }
 

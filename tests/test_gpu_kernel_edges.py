@@ -90,3 +90,17 @@ def test_poisson_tile_edges_match_oracle(glib, olib, n_cells, degree, with_bc):
     # in the residual's norm is below 1e3 here
     assert rel(pg, po) < 1e-9 and rel(ng, no) < 1e-9
     assert sg.rel_residual <= 1e-12 and abs(sg.charge - so.charge) < 1e-12 * abs(so.charge)
+
+
+# slots (cell, column) against the slots of a wave, 12, 10, 9 and 8 at p = 2 to 5: a
+# wave not filled, exactly filled (8, 40, 72 slots), and one slot more
+@pytest.mark.parametrize("p", [2, 3, 4, 5])
+@pytest.mark.parametrize("n_cells,ncols", [(2, 1), (2, 5), (2, 9), (3, 3)])
+def test_cell_product_wave_edges_match_oracle(glib, olib, p, n_cells, ncols):
+    _say("cell_product", n_cells, p, ncols)
+    g, o, s = bare_pair(glib, olib, n_cells, p, 4, precision=abi.MIXED)
+    x = np.random.default_rng(p + ncols).standard_normal((s.n_nodes, ncols))
+    want = o.apply_hamiltonian(x)
+    # sums of some 10^2 products per entry and axis: well below 1e3 roundings
+    assert rel(g.apply_hamiltonian(x, precision=abi.FP64), want) < 1e-13
+    assert rel(g.apply_hamiltonian(x, precision=abi.MIXED), want) < 2e-6
