@@ -156,6 +156,8 @@ struct ApplyEpilogue {
   const T* Z = nullptr; double b = 0.0; const double* cb = nullptr;
   const T* W = nullptr; double c = 0.0; const double* cc = nullptr;
   const double* xn = nullptr;    // node scale of the operator input and of X
+  const double* sxn = nullptr;   // with xn: the product Sg xn (launch_scale_product), which the
+                                 // sum-factorised kernel reads in place of both
   const double* xcol = nullptr;  // column scale of the operator input
   T* V = nullptr;                // stores the scaled input xcol xn Xin (needs dot_partial)
   double* dot_partial = nullptr;
@@ -235,6 +237,9 @@ void launch_lincomb_d2f(int64_t N, int B, float* Y, const double* X, double a, c
 void launch_lincomb_df2d(int64_t N, int B, double* Y, const double* X, double a,
                          const double* ca, const float* Z, double b, const double* cb,
                          hipStream_t s);
+// y = a b in FP64
+template <typename T>
+void launch_scale_product(int64_t n, double* y, const T* a, const double* b, hipStream_t s);
 void launch_convert_d2f(int64_t n, float* y, const double* x, hipStream_t s);
 void launch_convert_f2d(int64_t n, double* y, const float* x, hipStream_t s);
 int coldot_blocks(int64_t N, int B);
@@ -334,8 +339,8 @@ int launch_minres_start_dots(int64_t N, int B, const double* r, const double* D,
                              hipStream_t s);
 template <typename T, typename TV>
 void launch_cell_dot(const Geo& g, const CellOp<T>& op, const T* Sg, const TV* X, int B,
-                     const double* xn, const double* xcol, T* Yc, double* cell_dots,
-                     const GemmShape& shape, hipStream_t s);
+                     const double* xn, const double* sxn, const double* xcol, T* Yc,
+                     double* cell_dots, const GemmShape& shape, hipStream_t s);
 void launch_minres_alpha_cell(int B, int ncell, const double* cell_dots, double* st, hipStream_t s);
 template <typename TY>
 int launch_minres_gather(const Geo& g, const TY* Yc, const double* S, const double* D,

@@ -78,6 +78,7 @@ struct idft_ctx {
   bool verbose = false;  // IDFT_VERBOSE set: solver progress on stderr
   // static per-node / per-quadrature data
   DevBuf<double> S, sqrtM, invSqrtM, Djac, DjacSqrt, Mdiag, jxw;
+  DevBuf<double> SD, SD32;  // S Djac and S32 Djac: the node scales of a MINRES step's input
   DevBuf<float> S32;
   DevBuf<unsigned char> bnd, adjMask;
   DevBuf<double> potBase, rhoT, weight, veff, rho, u;
@@ -354,6 +355,7 @@ struct idft_ctx {
         ApplyEpilogue<double> ep;
         ep.Y = yd.p;
         ep.xn = Djac.p;
+        ep.sxn = f32 ? SD32.p : SD.p;
         ep.xcol = ones.p;
         if (f32) apply_f32op(xdp(), ncols, ep);
         else apply<double>(xdp(), ncols, ep);
@@ -1044,12 +1046,12 @@ struct idft_ctx {
       if (f32op) {
         st.applies_fp32++;
         st.apply_cols_fp32 += bc;
-        launch_cell_dot<float, double>(g, op32(), S32.p, r2, bc, Djac.p, cv, Yc32.p, mcell.p,
+        launch_cell_dot<float, double>(g, op32(), S32.p, r2, bc, Djac.p, SD32.p, cv, Yc32.p, mcell.p,
                                        shape32, s);
       } else {
         st.applies_fp64++;
         st.apply_cols_fp64 += bc;
-        launch_cell_dot<double, double>(g, op64(), S.p, r2, bc, Djac.p, cv, Yc64.p, mcell.p,
+        launch_cell_dot<double, double>(g, op64(), S.p, r2, bc, Djac.p, SD.p, cv, Yc64.p, mcell.p,
                                         shape64, s);
       }
       launch_minres_alpha_cell(bc, (int)t.ncell, mcell.p, mst.p, s);
@@ -1086,6 +1088,7 @@ struct idft_ctx {
       ep.X = r2; ep.a = 1.0; ep.ca = mst.p + (size_t)MS_CVN * bc;
       ep.Z = r1; ep.b = 1.0; ep.cb = mst.p + (size_t)MS_CR1 * bc;
       ep.xn = Djac.p;
+      ep.sxn = f32op ? SD32.p : SD.p;
       ep.xcol = mst.p + (size_t)MS_CV * bc;
       ep.dot_partial = partial.p;
       int nbk = f32op ? apply_f32op(r2, bc, ep) : apply<double>(r2, bc, ep);
@@ -1788,6 +1791,10 @@ idft_ctx* create_ctx(const idft_desc* d, const double* pot_base_q, const double*
     c->invSqrtM.upload(isq.data(), t.N, s);
     c->Djac.upload(Dj.data(), t.N, s);
     c->DjacSqrt.upload(Djs.data(), t.N, s);
+    c->SD.resize(t.N);
+    c->SD32.resize(t.N);
+    launch_scale_product<double>(t.N, c->SD.p, c->S.p, c->Djac.p, s);
+    launch_scale_product<float>(t.N, c->SD32.p, c->S32.p, c->Djac.p, s);
     c->bnd.upload(bnd.data(), t.N, s);
     c->adjMask.upload(am.data(), t.N, s);
     if (pot_base_q) {

@@ -807,6 +807,11 @@ struct PlaneStride {
   static constexpr int M = 256 / (int)sizeof(T);
   static constexpr int v = L + ((NS - L) % M + M) % M;
 };
+// The node scale of the input: S, or with a further node scale the product in FP64.
+template <typename T, bool XN>
+struct PlaneScale {
+  typedef typename std::conditional<XN, double, T>::type type;
+};
 // KIN = false: the potential chain alone on the unscaled input (S unused):
 // Yc = Lq^T diag(w_e) Lq X_e, the quadrature operator of a weight.  wstride: the
 // weights' step from cell to cell (0: the same weights in every cell); ldx: the row
@@ -814,10 +819,11 @@ struct PlaneStride {
 // dotp also each slot's x.(H_e x), dotp[column * ncell + cell].
 template <typename T, typename TV, int P, bool XN, bool KIN>
 __global__ __launch_bounds__(64, 2) void k_cell_plane(
-    Geo g, T hq, const T* __restrict__ W, uint32_t wstride, const T* __restrict__ S,
-    const TV* __restrict__ X, uint32_t ldx, const double* __restrict__ xn,
+    Geo g, T hq, const T* __restrict__ W, uint32_t wstride,
+    const typename PlaneScale<T, XN>::type* __restrict__ S, const TV* __restrict__ X, uint32_t ldx,
     const double* __restrict__ xcol, T* __restrict__ Yc, uint32_t B, FastDiv divB, uint32_t nslot,
     double* __restrict__ dotp, const double* __restrict__ eo) {
+  typedef typename PlaneScale<T, XN>::type SN;
   constexpr int N1 = P + 1, Q = P + 3, N2 = N1 * N1, NE = N2 * N1, Q2 = Q * Q;
   constexpr int NS = PlaneLanes<P>::NS, PS = PlaneStride<T, P>::v;
   constexpr int K3 = (N2 + Q - 1) / Q;  // lines per lane in the line phases
@@ -836,45 +842,41 @@ __global__ __launch_bounds__(64, 2) void k_cell_plane(
   if (kw >= nwave) return;
   const bool live = kw * NS + slot < nslot;
   const uint32_t sid = live ? kw * NS + slot : nslot - 1;
-  const uint32_t e = B == 1 ? sid : fast_div(sid, divB), j = sid - e * B;
-  const uint32_t nc = (uint32_t)g.nc, NN = (uint32_t)g.N1;
-  const uint32_t cx = e % nc, cyz = e / nc, cy = cyz % nc, cz = cyz / nc;
-  const uint32_t n00 = (cz * P * NN + cy * P) * NN + cx * P;
-  const uint32_t NNN = NN * NN;
+  const uint32_t nc = (uint32_t)g.nc, NN = (uint32_t)g.N1, NNN = NN * NN;
+  const auto cell_of = [&](uint32_t s) { return B == 1 ? s : fast_div(s, divB); };
+  const auto first_node = [&](uint32_t c) {
+    const uint32_t cx = c % nc, cyz = c / nc, cy = cyz % nc, cz = cyz / nc;
+    return (cz * P * NN + cy * P) * NN + cx * P;
+  };
+  const uint32_t e = cell_of(sid), j = sid - e * B, n00 = first_node(e);
   const T* we = W + (size_t)e * wstride + r * Q2;
   const double xc = xcol ? xcol[j] : 1.0;
   const T wg = KIN ? (T)eo[EoTable<P>::kWeights + r] : T(0);
   // the input of line l of this lane, scaled
-  const auto load_line = [&](uint32_t l, T(&v)[N1]) {
-    const uint32_t n0 = n00 + (l / N1) * NN + l % N1;
-    T sv[N1];
+  // (pointers stepped by uniform strides: a 64-bit product per entry would cost as
+  // much as the entry's arithmetic)
+  const size_t zx = (size_t)NNN * ldx;
+  const auto load_line = [&](uint32_t l, uint32_t n0, uint32_t jj, T(&v)[N1]) {
+    const uint32_t n = n0 + (l / N1) * NN + l % N1;
+    const TV* Xp = X + (size_t)n * ldx + jj;
+    const SN* Sp = KIN ? S + n : nullptr;
+    SN sv[N1];
     TV xv[N1];
-    double nv[N1];
 #pragma unroll
     for (int c = 0; c < N1; ++c) {
-      const uint32_t n = n0 + c * NNN;
-      xv[c] = X[(size_t)n * ldx + j];
-      if constexpr (KIN) sv[c] = S[n];
-      if constexpr (XN) nv[c] = xn[n];
+      xv[c] = Xp[c * zx];
+      if constexpr (KIN) sv[c] = Sp[(size_t)c * NNN];
     }
 #pragma unroll
     for (int c = 0; c < N1; ++c) {
-      if constexpr (!KIN) {
-        v[c] = (T)xv[c];
-      } else if constexpr (std::is_same<T, TV>::value) {
-        T x = sv[c] * xv[c];
-        if constexpr (XN) x *= (T)nv[c];
-        v[c] = x * (T)xc;
-      } else {
-        double x = (double)sv[c] * (double)xv[c];
-        if constexpr (XN) x *= nv[c];
-        v[c] = (T)(x * xc);
-      }
+      if constexpr (!KIN) v[c] = (T)xv[c];
+      else if constexpr (std::is_same<T, TV>::value) v[c] = sv[c] * xv[c] * (T)xc;
+      else v[c] = (T)((double)sv[c] * (double)xv[c] * xc);  // scaled in FP64, rounded once
     }
   };
   // line index of round k (rounds past the last line repeat it)
-  const auto line_of = [&](int k) -> uint32_t {
-    const uint32_t l = r + Q * k;
+  const auto line_of = [&](uint32_t rr, int k) -> uint32_t {
+    const uint32_t l = rr + Q * k;
     return l < (uint32_t)N2 ? l : (uint32_t)N2 - 1;
   };
   // z lines: u[q] = Lq x for the Q planes
@@ -882,9 +884,9 @@ __global__ __launch_bounds__(64, 2) void k_cell_plane(
   const PlCoef<T, TL> fL0(eo, T(0));
 #pragma unroll
   for (int k = 0; k < K3; ++k) {
-    const uint32_t l = line_of(k);
+    const uint32_t l = line_of(r, k);
     T v[N1], vp[HE], vm[HO], oe[QE], oo[QO], u[Q];
-    load_line(l, v);
+    load_line(l, n00, j, v);
     pl_split<N1>(v, vp, vm);
     pl_halves<TL, false>(fL0, vp, vm, oe, oo);
     pl_join<Q>(oe, oo, u);
@@ -1025,11 +1027,16 @@ __global__ __launch_bounds__(64, 2) void k_cell_plane(
   };
   put_plane(pe, po);
   wave_lds_fence();
+  // the lane's place found again (and with dotp its input read again), from numbers
+  // whose origin the compiler does not see: kept through the planes, they would cost
+  // registers that the planes need
+  uint32_t sid2 = sid, r2 = r;
+  if constexpr (XN) asm("" : "+v"(sid2), "+v"(r2));
   // z lines back: y = Lq^T p + E m
   T ze[K3][HE], zo[K3][HO];
 #pragma unroll
   for (int k = 0; k < K3; ++k) {
-    const uint32_t l = line_of(k);
+    const uint32_t l = line_of(r2, k);
     T v[Q], vp[QE], vm[QO];
 #pragma unroll
     for (int q = 0; q < Q; ++q) v[q] = lds[q * PS + l * NS + slot];
@@ -1053,17 +1060,15 @@ __global__ __launch_bounds__(64, 2) void k_cell_plane(
   }
   const PlCoef<T, TE> fE(eo, ze[K3 - 1][0]);
   double dotv = 0.0;
-  T* const yc = Yc + (size_t)e * NE * B + j;
+  const uint32_t e2 = cell_of(sid2), j2 = sid2 - e2 * B, n2 = XN ? first_node(e2) : 0;
+  T* const yc = Yc + (size_t)e2 * NE * B + j2;
+  const uint32_t zy = N2 * B;
 #pragma unroll
   for (int k = 0; k < K3; ++k) {
-    const uint32_t l = line_of(k);
+    const uint32_t l = line_of(r2, k);
     T xl[N1];
     if constexpr (XN) {
-      // read again, not kept from the first phase: hidden from the compiler, which
-      // would hold all of this lane's input in registers meanwhile
-      uint32_t l2 = l;
-      asm("" : "+v"(l2));
-      if (dotp) load_line(l2, xl);
+      if (dotp) load_line(l, n2, j2, xl);
     }
     if constexpr (KIN) {
       T v[Q], vp[QE], vm[QO];
@@ -1079,9 +1084,10 @@ __global__ __launch_bounds__(64, 2) void k_cell_plane(
     }
     T y[N1];
     pl_join<N1>(ze[k], zo[k], y);
-    if (live && r + Q * k < (uint32_t)N2) {
+    if (live && r2 + Q * k < (uint32_t)N2) {
+      T* const yl = yc + l * B;
 #pragma unroll
-      for (int c = 0; c < N1; ++c) yc[(size_t)((c * N2 + l) * B)] = y[c];
+      for (int c = 0; c < N1; ++c) yl[(size_t)c * zy] = y[c];
       if constexpr (XN) {
         if (dotp) {
 #pragma unroll
@@ -1100,7 +1106,7 @@ __global__ __launch_bounds__(64, 2) void k_cell_plane(
         double t = 0.0;
 #pragma unroll
         for (int q = 0; q < Q; ++q) t += red[q * NS + slot];
-        dotp[(size_t)j * (uint32_t)g.ncell + e] = t;
+        dotp[(size_t)j2 * (uint32_t)g.ncell + e2] = t;
       }
     }
   }
@@ -1739,6 +1745,12 @@ __global__ void k_lincomb_mixed(uint32_t NB, uint32_t B, TY* Y, const TX* X, dou
   }
 }
 
+template <typename T>
+__global__ void k_scale_product(int64_t n, double* __restrict__ y, const T* __restrict__ a,
+                                const double* __restrict__ b) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) y[i] = (double)a[i] * b[i];
+}
 __global__ void k_d2f(int64_t n, float* __restrict__ y, const double* __restrict__ x) {
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * blockDim.x)
@@ -2362,23 +2374,23 @@ bool sf_vc_supported(int cols, int vc, bool fp64) {
 static const double* sf_eo_table(int p);
 
 template <typename T, typename TV, int P, bool XN, bool KIN>
-static void cell_plane(const Geo& g, T hq, const T* W, uint32_t wstride, const T* S, const TV* X,
-                       int ldx, const double* xn, const double* xcol, T* Yc, int B, double* dotp,
-                       hipStream_t s) {
+static void cell_plane(const Geo& g, T hq, const T* W, uint32_t wstride,
+                       const typename PlaneScale<T, XN>::type* S, const TV* X, int ldx,
+                       const double* xcol, T* Yc, int B, double* dotp, hipStream_t s) {
   constexpr int NS = PlaneLanes<P>::NS;
   check_u32(cell_scratch_elems(g, B));
   const uint32_t nslot = (uint32_t)(g.ncell * B);
   const uint32_t nwave = (nslot + NS - 1) / NS;
   const FastDiv divB = make_fastdiv((uint32_t)std::max(B, 2));
   k_cell_plane<T, TV, P, XN, KIN><<<8 * ((nwave + 7) / 8), 64, 0, s>>>(
-      g, hq, W, wstride, S, X, (uint32_t)ldx, xn, xcol, Yc, (uint32_t)B, divB, nslot, dotp,
+      g, hq, W, wstride, S, X, (uint32_t)ldx, xcol, Yc, (uint32_t)B, divB, nslot, dotp,
       sf_eo_table(P));
 }
 
 template <typename T, typename TV, int P>
 static void cell_sf_p(const Geo& g, const CellOp<T>& op, const T* S, const TV* X,
-                      const double* xn, const double* xcol, T* Yc, int B, int cg, int vc,
-                      double* dotp, hipStream_t s) {
+                      const double* xn, const double* sxn, const double* xcol, T* Yc, int B,
+                      int cg, int vc, double* dotp, hipStream_t s) {
   if (!op.W) throw Error(IDFT_ESTATE, "quadrature weights of the cell operator not set");
   if (!sf_vc_supported(cg, vc, std::is_same<T, double>::value))
     throw Error(IDFT_EINVAL, "shape not supported by the sum-factorised kernel");
@@ -2391,21 +2403,22 @@ static void cell_sf_p(const Geo& g, const CellOp<T>& op, const T* S, const TV* X
   // carry a node scale
   if constexpr (std::is_same<TV, double>::value) {
     if (xn) {
-      cell_plane<T, TV, P, true, true>(g, hq, op.W, nq, S, X, B, xn, xcol, Yc, B, dotp, s);
+      if (!sxn) throw Error(IDFT_EINVAL, "node-scaled input without the product of its scales");
+      cell_plane<T, TV, P, true, true>(g, hq, op.W, nq, sxn, X, B, xcol, Yc, B, dotp, s);
       return;
     }
   } else {
     if (xn) throw Error(IDFT_EINVAL, "node-scaled input needs FP64 vectors");
   }
-  cell_plane<T, TV, P, false, true>(g, hq, op.W, nq, S, X, B, nullptr, xcol, Yc, B, nullptr, s);
+  cell_plane<T, TV, P, false, true>(g, hq, op.W, nq, S, X, B, xcol, Yc, B, nullptr, s);
 }
 
 template <typename T, typename TV, int P>
 static void cell_gemm_p(const Geo& g, const CellOp<T>& op, const T* S, const TV* X,
-                        const double* xn, const double* xcol, T* Yc, int B,
+                        const double* xn, const double* sxn, const double* xcol, T* Yc, int B,
                         const GemmShape& shape, hipStream_t s, double* dotp = nullptr) {
   if (shape.kernel == CK_SUM_FACTOR) {
-    cell_sf_p<T, TV, P>(g, op, S, X, xn, xcol, Yc, B, shape.vectors_per_tile,
+    cell_sf_p<T, TV, P>(g, op, S, X, xn, sxn, xcol, Yc, B, shape.vectors_per_tile,
                         shape.cells_per_wg, dotp, s);
     return;
   }
@@ -2511,10 +2524,10 @@ void launch_cell_gemm(const Geo& g, const CellOp<T>& op, const T* S, const T* X,
                       const double* xcol, T* Yc, int B, const GemmShape& shape, hipStream_t s) {
   if (B < 1 || B > kMaxCols) throw Error(IDFT_EINVAL, "block width out of range");
   switch (g.p) {
-    case 2: cell_gemm_p<T, T, 2>(g, op, S, X, nullptr, xcol, Yc, B, shape, s); break;
-    case 3: cell_gemm_p<T, T, 3>(g, op, S, X, nullptr, xcol, Yc, B, shape, s); break;
-    case 4: cell_gemm_p<T, T, 4>(g, op, S, X, nullptr, xcol, Yc, B, shape, s); break;
-    case 5: cell_gemm_p<T, T, 5>(g, op, S, X, nullptr, xcol, Yc, B, shape, s); break;
+    case 2: cell_gemm_p<T, T, 2>(g, op, S, X, nullptr, nullptr, xcol, Yc, B, shape, s); break;
+    case 3: cell_gemm_p<T, T, 3>(g, op, S, X, nullptr, nullptr, xcol, Yc, B, shape, s); break;
+    case 4: cell_gemm_p<T, T, 4>(g, op, S, X, nullptr, nullptr, xcol, Yc, B, shape, s); break;
+    case 5: cell_gemm_p<T, T, 5>(g, op, S, X, nullptr, nullptr, xcol, Yc, B, shape, s); break;
     default: throw Error(IDFT_EINVAL, "degree not supported by the HIP kernels (2..5)");
   }
   IDFT_HIP(hipGetLastError());
@@ -2532,10 +2545,10 @@ int launch_cell_apply(const Geo& g, const CellOp<T>& op, const T* Sg, const TV* 
                       hipStream_t s) {
   if (B < 1 || B > kMaxCols) throw Error(IDFT_EINVAL, "block width out of range");
   switch (g.p) {
-    case 2: cell_gemm_p<T, TV, 2>(g, op, Sg, X, ep.xn, ep.xcol, Yc, B, shape, s); break;
-    case 3: cell_gemm_p<T, TV, 3>(g, op, Sg, X, ep.xn, ep.xcol, Yc, B, shape, s); break;
-    case 4: cell_gemm_p<T, TV, 4>(g, op, Sg, X, ep.xn, ep.xcol, Yc, B, shape, s); break;
-    case 5: cell_gemm_p<T, TV, 5>(g, op, Sg, X, ep.xn, ep.xcol, Yc, B, shape, s); break;
+    case 2: cell_gemm_p<T, TV, 2>(g, op, Sg, X, ep.xn, ep.sxn, ep.xcol, Yc, B, shape, s); break;
+    case 3: cell_gemm_p<T, TV, 3>(g, op, Sg, X, ep.xn, ep.sxn, ep.xcol, Yc, B, shape, s); break;
+    case 4: cell_gemm_p<T, TV, 4>(g, op, Sg, X, ep.xn, ep.sxn, ep.xcol, Yc, B, shape, s); break;
+    case 5: cell_gemm_p<T, TV, 5>(g, op, Sg, X, ep.xn, ep.sxn, ep.xcol, Yc, B, shape, s); break;
     default: throw Error(IDFT_EINVAL, "degree not supported by the HIP kernels (2..5)");
   }
   IDFT_HIP(hipGetLastError());
@@ -2609,7 +2622,7 @@ void launch_quad_pairs(const Geo& g, const double* W, int64_t wstride, const dou
                                                   asc, T2, (uint32_t)ldt, pairs, (uint32_t)np,  \
                                                   partial.p)
 #define IDFT_QP(PP)                                                \
-  cell_plane<double, double, PP, false, false>(g, 0.0, W, (uint32_t)wstride, nullptr, Bv, ldb, nullptr, \
+  cell_plane<double, double, PP, false, false>(g, 0.0, W, (uint32_t)wstride, nullptr, Bv, ldb,  \
                                                nullptr, Yc, wb, nullptr, s);                    \
   IDFT_HIP(hipGetLastError());                                     \
   if (vw == 2) IDFT_QG(PP, 2);                                     \
@@ -2650,26 +2663,28 @@ void launch_pair_combine(int64_t N, int B, bool rhs, const double* T, const doub
 
 template <typename T, typename TV>
 void launch_cell_dot(const Geo& g, const CellOp<T>& op, const T* Sg, const TV* X, int B,
-                     const double* xn, const double* xcol, T* Yc, double* cell_dots,
-                     const GemmShape& shape, hipStream_t s) {
+                     const double* xn, const double* sxn, const double* xcol, T* Yc,
+                     double* cell_dots, const GemmShape& shape, hipStream_t s) {
   if (B < 1 || B > kMaxCols) throw Error(IDFT_EINVAL, "block width out of range");
   if (shape.kernel != CK_SUM_FACTOR || !cell_dots)
     throw Error(IDFT_EINVAL, "per-cell dots need the sum-factorised cell product");
   switch (g.p) {
-    case 2: cell_gemm_p<T, TV, 2>(g, op, Sg, X, xn, xcol, Yc, B, shape, s, cell_dots); break;
-    case 3: cell_gemm_p<T, TV, 3>(g, op, Sg, X, xn, xcol, Yc, B, shape, s, cell_dots); break;
-    case 4: cell_gemm_p<T, TV, 4>(g, op, Sg, X, xn, xcol, Yc, B, shape, s, cell_dots); break;
-    case 5: cell_gemm_p<T, TV, 5>(g, op, Sg, X, xn, xcol, Yc, B, shape, s, cell_dots); break;
+    case 2: cell_gemm_p<T, TV, 2>(g, op, Sg, X, xn, sxn, xcol, Yc, B, shape, s, cell_dots); break;
+    case 3: cell_gemm_p<T, TV, 3>(g, op, Sg, X, xn, sxn, xcol, Yc, B, shape, s, cell_dots); break;
+    case 4: cell_gemm_p<T, TV, 4>(g, op, Sg, X, xn, sxn, xcol, Yc, B, shape, s, cell_dots); break;
+    case 5: cell_gemm_p<T, TV, 5>(g, op, Sg, X, xn, sxn, xcol, Yc, B, shape, s, cell_dots); break;
     default: throw Error(IDFT_EINVAL, "degree not supported by the HIP kernels (2..5)");
   }
   IDFT_HIP(hipGetLastError());
 }
 template void launch_cell_dot<double, double>(const Geo&, const CellOp<double>&, const double*,
                                               const double*, int, const double*, const double*,
-                                              double*, double*, const GemmShape&, hipStream_t);
+                                              const double*, double*, double*, const GemmShape&,
+                                              hipStream_t);
 template void launch_cell_dot<float, double>(const Geo&, const CellOp<float>&, const float*,
                                              const double*, int, const double*, const double*,
-                                             float*, double*, const GemmShape&, hipStream_t);
+                                             const double*, float*, double*, const GemmShape&,
+                                             hipStream_t);
 
 template <typename TY>
 int launch_minres_gather(const Geo& g, const TY* Yc, const double* S, const double* D,
@@ -2762,6 +2777,15 @@ void launch_lincomb_df2d(int64_t N, int B, double* Y, const double* X, double a,
       (uint32_t)(N * B), (uint32_t)B, Y, X, a, ca, Z, b, cb);
   IDFT_HIP(hipGetLastError());
 }
+template <typename T>
+void launch_scale_product(int64_t n, double* y, const T* a, const double* b, hipStream_t s) {
+  k_scale_product<T><<<(unsigned)((n + 255) / 256), 256, 0, s>>>(n, y, a, b);
+  IDFT_HIP(hipGetLastError());
+}
+template void launch_scale_product<double>(int64_t, double*, const double*, const double*,
+                                           hipStream_t);
+template void launch_scale_product<float>(int64_t, double*, const float*, const double*,
+                                          hipStream_t);
 void launch_convert_d2f(int64_t n, float* y, const double* x, hipStream_t s) {
   k_d2f<<<grid_for(n), kThreads, 0, s>>>(n, y, x);
   IDFT_HIP(hipGetLastError());
