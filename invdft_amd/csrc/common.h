@@ -313,7 +313,7 @@ int launch_minres_lanczos(int64_t N, int B, const T* y, const T* r2, T* rnew, co
                           const double* st, double* partial, hipStream_t s);
 // nq = 3: partial also holds the Q2 and Q3 partials at row offsets nblk, 2 nblk
 void launch_minres_givens(int B, int nblk, const double* partial, const double* negEig,
-                          double* st, hipStream_t s, int nq = 1);
+                          double* st, hipStream_t s, int nq = 1, double* hist = nullptr);
 template <typename T>
 void launch_minres_update(int64_t N, int B, const T* r, const double* D, T* w1, const T* w, T* x,
                           const double* st, hipStream_t s);
@@ -322,19 +322,27 @@ void launch_copy_done(int B, const double* st, int* flags, hipStream_t s);
 // per CU (FP64 or FP32, unpacked), timed with HIP events on stream s
 double launch_fma_probe(bool fp64, int chains, hipStream_t s);
 // Fused MINRES step for sum-factorised cell products (shape.kernel ==
-// CK_SUM_FACTOR), four launches per step instead of five and four block
-// streams fewer (9 instead of 13, plus one update launch per run of steps):
+// CK_SUM_FACTOR): four launches per step instead of five and, with batches of 8
+// steps, 5.75 block streams instead of 13:
 //   start_dots   partials of r.D r and (D r)^2 of the right-hand side (2 x nblk
 //                rows), reduced by launch_minres_start(nq = 2) into beta and Q2
 //   cell_dot     cell product of v = cv D r2 (node scale D, column scale cv)
 //                with the per-cell dots x_e.(H_e x_e) (column-major, B x ncell)
 //   alpha_cell   alpha = sum of the cell dots + cv (cvn Q2 + cr1 Q3)
-//   gather       r1 <- S sum + (cvn D + ca2) r2 + cr1 r1 with the three next
-//                dots (3 x nblk rows), reduced by launch_minres_givens(nq = 3);
-//                with w != nullptr also the previous step's update
-//                w <- cwv D r1 + cww1 w + cww w1, x += cx w (read before r1 is
-//                overwritten), so that launch_minres_update runs only after the
-//                last step of a run of steps
+//   gather       r_new = S sum + (cvn D + ca2) r2 + cr1 r1 (r_new may be r1) with the
+//                three next dots (3 x nblk rows), reduced by
+//                launch_minres_givens(nq = 3), which also stores the step's
+//                direction coefficients in hist (4 x B)
+//   batch        the direction and solution updates of the last n steps at once
+//                (w holds the older direction, w1 the newer, before and after);
+//                place != nullptr receives a copy of the newest Lanczos vector `last`
+constexpr int kMinresBatch = 8;
+struct MinresVectors {
+  const double* r[kMinresBatch];
+};
+void launch_minres_batch(int64_t N, int B, int n, const MinresVectors& rs, const double* D,
+                         double* w, double* w1, double* x, const double* hist,
+                         const double* last, double* place, hipStream_t s);
 int launch_minres_start_dots(int64_t N, int B, const double* r, const double* D, double* partial,
                              hipStream_t s);
 template <typename T, typename TV>
@@ -344,9 +352,8 @@ void launch_cell_dot(const Geo& g, const CellOp<T>& op, const T* Sg, const TV* X
 void launch_minres_alpha_cell(int B, int ncell, const double* cell_dots, double* st, hipStream_t s);
 template <typename TY>
 int launch_minres_gather(const Geo& g, const TY* Yc, const double* S, const double* D,
-                         const double* r2, double* r1, int B, const double* st, double* partial,
-                         int gather_rows, hipStream_t s, double* w = nullptr,
-                         const double* w1 = nullptr, double* x = nullptr);
+                         const double* r2, const double* r1, double* rnew, int B,
+                         const double* st, double* partial, int gather_rows, hipStream_t s);
 
 // L-BFGS checkpoint settings of a context (idft_bfgs_set_checkpoint).
 struct BfgsCheckpoint {

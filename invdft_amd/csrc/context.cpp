@@ -58,6 +58,7 @@ struct AdjointState {
 template <typename T>
 struct MinresWork {
   DevBuf<T> r1, r2, y, w1, w, rhs;
+  DevBuf<T> q[kMinresBatch - 3];  // further Lanczos vectors of a batch of fused steps
   void ensure(size_t n) {
     r1.resize(n); r2.resize(n); y.resize(n); w1.resize(n); w.resize(n); rhs.resize(n);
   }
@@ -113,7 +114,7 @@ struct idft_ctx {
   idft_stats st{};
   AdjointState adj;
   MinresWork<double> mw64;
-  DevBuf<double> mst, mx, mtmp, mnegc, mcell, pairCoef;
+  DevBuf<double> mst, mx, mtmp, mnegc, mcell, mhist, pairCoef;
   DevBuf<int> mflags, msel, pairList;
   idft_mv mvPsi, mvX;
 
@@ -1015,6 +1016,27 @@ struct idft_ctx {
       const int nb = launch_coldot_partial<double>(N, b, r1, r1, Djac.p, partial.p, s);
       launch_minres_start(b, nb, partial.p, adj.dnegEig.p, mst.p, s);
     }
+    // Lanczos vectors that a batch of fused steps keeps: y (which fused steps do
+    // not use otherwise) and up to five more, taken only where they leave half of
+    // the free memory and not where memory is what the caller saves
+    // (psi_checkpoint)
+    std::vector<double*> vb;
+    if (fused) {
+      mhist.resize((size_t)kMinresBatch * 4 * b);
+      vb.push_back(W.y.p);
+      constexpr int nq = kMinresBatch - 3;
+      bool more = !d.psi_checkpoint;
+      if (more && W.q[nq - 1].n < NB(b)) {
+        size_t freeB = 0, totalB = 0;
+        IDFT_HIP(hipMemGetInfo(&freeB, &totalB));
+        more = nq * NB(b) * sizeof(double) <= freeB / 2;
+        if (more)
+          for (auto& q : W.q) q.resize(NB(b));
+      }
+      if (more)
+        for (auto& q : W.q) vb.push_back(q.p);
+    }
+    const int batch = (int)vb.size() + 2;
     // the compact block: bc columns, orig[k] the caller's column of column k
     int bc = b;
     std::vector<int> orig(b);
@@ -1034,54 +1056,72 @@ struct idft_ctx {
     // N*bc streams per step: 1 (cell product) + 3 (gather) + 3 (Lanczos) + 6
     // (update).  r2 = r_k (newest Lanczos residual), r1 = r_{k-1}; the step's
     // Lanczos vector v = cv D r2 is formed on the fly (not stored).
-    // Fused step: 4 launches and N*bc streams 1 (cell product) + 3 (gather:
-    // r2, r1 in, r1 out) + 5 (the previous step's update inside the gather:
-    // w, w1 and x in, w and x out; r1 is read anyway).  The last step's
-    // update of a run carries over into the next run's first gather; only
-    // before a compaction and at the end does finish_run() apply it on its own
-    // (6 streams), since those read x.
-    bool pending = false;  // a step whose update has not run yet
-    auto fused_step = [&] {
+    // Fused step: 4 launches and N*bc streams 1 (cell product) + 3 (gather: r2,
+    // r1 in, r_new out); the direction and solution updates of a batch of steps
+    // follow in one pass of n + 6 streams (launch_minres_batch), for which the
+    // batch keeps its Lanczos vectors: r1 and r2 at its start, then vb[0 .. n-3],
+    // and its last two in r1's place and in the spare buffer.
+    auto fused_step = [&](const double* ra, const double* rb, double* rnew, double* hist) {
       const double* cv = mst.p + (size_t)MS_CV * bc;
       if (f32op) {
         st.applies_fp32++;
         st.apply_cols_fp32 += bc;
-        launch_cell_dot<float, double>(g, op32(), S32.p, r2, bc, Djac.p, SD32.p, cv, Yc32.p, mcell.p,
-                                       shape32, s);
+        launch_cell_dot<float, double>(g, op32(), S32.p, rb, bc, Djac.p, SD32.p, cv, Yc32.p,
+                                       mcell.p, shape32, s);
       } else {
         st.applies_fp64++;
         st.apply_cols_fp64 += bc;
-        launch_cell_dot<double, double>(g, op64(), S.p, r2, bc, Djac.p, SD.p, cv, Yc64.p, mcell.p,
+        launch_cell_dot<double, double>(g, op64(), S.p, rb, bc, Djac.p, SD.p, cv, Yc64.p, mcell.p,
                                         shape64, s);
       }
       launch_minres_alpha_cell(bc, (int)t.ncell, mcell.p, mst.p, s);
-      // the previous step's update (w <- its new direction, x) if pending:
-      // after that step's swaps w holds its oldest direction and w1 the newer
-      double* wu = pending ? w : nullptr;
-      const double* w1u = pending ? w1 : nullptr;
-      double* xu = pending ? xc : nullptr;
       const int nbk =
-          f32op ? launch_minres_gather<float>(g, Yc32.p, S.p, Djac.p, r2, r1, bc, mst.p, partial.p,
-                                              shape32.gather_rows, s, wu, w1u, xu)
-                : launch_minres_gather<double>(g, Yc64.p, S.p, Djac.p, r2, r1, bc, mst.p,
-                                               partial.p, shape64.gather_rows, s, wu, w1u, xu);
-      launch_minres_givens(bc, nbk, partial.p, mnegc.p, mst.p, s, 3);
-      pending = true;
-      std::swap(r1, r2);
-      std::swap(w1, w);
+          f32op ? launch_minres_gather<float>(g, Yc32.p, S.p, Djac.p, rb, ra, rnew, bc, mst.p,
+                                              partial.p, shape32.gather_rows, s)
+                : launch_minres_gather<double>(g, Yc64.p, S.p, Djac.p, rb, ra, rnew, bc, mst.p,
+                                               partial.p, shape64.gather_rows, s);
+      launch_minres_givens(bc, nbk, partial.p, mnegc.p, mst.p, s, 3, hist);
     };
-    // the last step's update of a run of fused steps (r1 = its Lanczos
-    // residual after the swap, w its pending direction, w1 the newer one)
-    auto finish_run = [&] {
-      if (!pending) return;
-      launch_minres_update<double>(N, bc, r1, Djac.p, w, w1, xc, mst.p, s);
-      pending = false;
+    // the one buffer not holding a block vector (the buffers stay owned by
+    // their DevBufs; the block vectors are views that move between them)
+    double* spare = mtmp.p;
+    bool swapped = false;  // r2 and the spare buffer have changed places
+    // A small block copies the newest vector back into r2's place, 2 streams per
+    // batch, so that every run has the same arguments and one graph replays from the
+    // second run on; a large one exchanges the two buffers (and captures two graphs,
+    // from the fifth run on).  At 15625 nodes x 4 columns launching the first four
+    // runs directly cost 5 % of a force evaluation; from 32 MB per vector on, two
+    // streams take longer than a capture saves.
+    const bool copyBack = NB(b) < (size_t)4 << 20;
+    auto batch_steps = [&](int n) {
+      MinresVectors rs{};
+      const double *ra = r1, *rb = r2;
+      for (int i = 0; i < n; ++i) {
+        double* out = i == n - 1 ? spare : i == n - 2 ? r1 : vb[i];
+        fused_step(ra, rb, out, mhist.p + (size_t)4 * i * bc);
+        rs.r[i] = rb;
+        ra = rb;
+        rb = out;
+      }
+      launch_minres_batch(N, bc, n, rs, Djac.p, w, w1, xc, mhist.p, spare,
+                          copyBack && n > 1 ? r2 : nullptr, s);
+    };
+    auto batch_done = [&](int n) {
+      if (copyBack && n > 1) return;
+      if (n == 1) std::swap(r1, r2);  // the newer start vector is the older now
+      std::swap(r2, spare);
+      swapped = !swapped;
+    };
+    // n fused steps in batches of nearly equal length (at least 2 for n > 1)
+    auto fused_run = [&](int n, bool launch) {
+      const int nb = (n + batch - 1) / batch;
+      for (int i = 0; i < nb; ++i) {
+        const int len = n / nb + (i < n % nb ? 1 : 0);
+        if (launch) batch_steps(len);
+        batch_done(len);
+      }
     };
     auto step = [&] {
-      if (fused) {
-        fused_step();
-        return;
-      }
       // y <- H~ v - eps v + cr1 r1, v = cv D r2;  partial dots of v.y  (one apply)
       ApplyEpilogue<double> ep;
       ep.Y = W.y.p; ep.alpha = 1.0;
@@ -1106,7 +1146,7 @@ struct idft_ctx {
     const bool useGraph = d.minres_graph != 0 && check % 2 == 0;
     Yc64.resize(cell_scratch_elems(g, b));
     if (canRelax) Yc32.resize(cell_scratch_elems(g, b));
-    // graphs per (operator precision, update pending at the run's start)
+    // graphs per (operator precision, place of r2 at the run's start)
     hipGraphExec_t execs[4] = {nullptr, nullptr, nullptr, nullptr};
     struct ExecGuard {
       hipGraphExec_t* e;
@@ -1117,9 +1157,6 @@ struct idft_ctx {
       ~ExecGuard() { drop(); }
     } guard{execs};
     std::vector<double> hst;
-    // the one buffer not holding a block vector (the buffers stay owned by
-    // their DevBufs; the block vectors are views that move between them)
-    double* spare = mtmp.p;
     // Repack the compact block to the columns `keep` (positions in it): the
     // caller's x receives every current column first, then the vectors, the
     // per-column state and the shifts are gathered.
@@ -1153,7 +1190,7 @@ struct idft_ctx {
       guard.drop();
       sync();
     };
-    int k = 0;
+    int k = 0, runs = 0;  // steps, and runs of steps of this block
     for (;;) {
       launch_copy_done(bc, mst.p, mflags.p, s);
       IDFT_HIP(hipMemcpyAsync(flags.data(), mflags.p, bc * sizeof(int), hipMemcpyDeviceToHost, s));
@@ -1164,10 +1201,7 @@ struct idft_ctx {
       std::vector<int> open;
       for (int j = 0; j < bc; ++j)
         if (!flags[j]) open.push_back(j);
-      if (open.empty() || k >= maxit) {
-        finish_run();
-        break;
-      }
+      if (open.empty() || k >= maxit) break;
       // repack once enough columns have finished, keeping the width even
       // (one finished column rides along, inert: its coefficients are zero)
       // so that the block kernels move two columns per 16-byte access
@@ -1184,8 +1218,8 @@ struct idft_ctx {
           kflags[i] = flags[keep[i]];
           pb[i] = phibar[keep[i]];
         }
-        finish_run();  // x complete before it is copied out
         compact(keep);
+        runs = 0;
         st.minres_compactions++;
         if (verbose)
           std::fprintf(stderr, "[idft] minres: step %d, block compacted to %d columns\n", k, bc);
@@ -1205,16 +1239,16 @@ struct idft_ctx {
       }
       const int n = std::min(check, maxit - k);
       st.minres_column_steps += (int64_t)n * bc;
-      // a run of fused steps that starts without a pending update (the
-      // first after the start or a compaction) is launched directly; the
-      // runs after it, which all start with one, replay a graph
-      if (useGraph && n == check && (pending || !fused)) {
-        hipGraphExec_t& exec = execs[(f32op ? 1 : 0) + (pending ? 2 : 0)];
+      // the first runs of a block are launched directly, the ones after them replay
+      if (useGraph && n == check && (runs >= (copyBack ? 1 : 4) || !fused)) {
+        hipGraphExec_t& exec = execs[(f32op ? 1 : 0) + (swapped ? 2 : 0)];
         if (!exec) {
           hipGraph_t graph = nullptr;
           IDFT_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
           try {
-            for (int i = 0; i < n; ++i) step();
+            if (fused) fused_run(n, true);
+            else
+              for (int i = 0; i < n; ++i) step();
           } catch (...) {
             (void)hipStreamEndCapture(s, &graph);
             if (graph) (void)hipGraphDestroy(graph);
@@ -1225,9 +1259,8 @@ struct idft_ctx {
           (void)hipGraphDestroy(graph);
           IDFT_HIP(ie);
         } else {
-          // the capture counted its n steps; replays count theirs here (and,
-          // with fused steps, leave the last update pending as the capture
-          // did)
+          // the capture counted its n steps and moved the block's views;
+          // replays do so here
           if (f32op) {
             st.applies_fp32 += n;
             st.apply_cols_fp32 += (int64_t)n * bc;
@@ -1235,13 +1268,16 @@ struct idft_ctx {
             st.applies_fp64 += n;
             st.apply_cols_fp64 += (int64_t)n * bc;
           }
-          if (fused) pending = true;
+          if (fused) fused_run(n, false);
         }
         IDFT_HIP(hipGraphLaunch(exec, s));
+      } else if (fused) {
+        fused_run(n, true);
       } else {
         for (int i = 0; i < n; ++i) step();
       }
       k += n;
+      ++runs;
     }
     // the caller's x and the iteration counts of the columns still in the block
     if (bc > 0) compact({});
@@ -1529,6 +1565,7 @@ struct idft_ctx {
   void release_adjoint_work() {
     mw64.r1.release(); mw64.r2.release(); mw64.y.release(); mw64.w1.release();
     mw64.w.release(); mw64.rhs.release();
+    for (auto& q : mw64.q) q.release();
     mx.release(); mtmp.release(); rref.release(); xdelta.release(); T2buf.release();
     psiAll.release(); mvPsi.own.release(); mvX.own.release();
     Yc64.release(); Yc32.release();

@@ -1351,23 +1351,17 @@ __global__ __launch_bounds__(kThreads) void k_quad_gather(
 // MINRES step, phase 2 with the Lanczos recurrence fused in (sum-factorised
 // cell products, whose cell kernel has already produced v.Hv, so that the
 // step's alpha is known before this kernel runs):
-//   r_new = S sum + (cvn_j D r2 + ca2_j r2) + cr1_j r1     (over r1, in place)
+//   r_new = S sum + (cvn_j D r2 + ca2_j r2) + cr1_j r1
 // with cvn = -eps/beta, ca2 = -alpha/beta, cr1 = -beta/beta_old (per column,
 // from the state), and block partials of the three node dots the next step
 // needs: r_new.D r_new (beta^2), D^2 r_new^2 and D r_new.r2, at
-// partial[(k B + j) nblk + block] for k = 0, 1, 2.  Each thread reads and writes the same entries
-// of r1, so the update in place is safe.
-// UPD: also the previous step's direction and solution update, deferred to
-// here because this kernel reads r1 (that step's Lanczos residual) anyway:
-//   w <- cwv D r1 + cww1 w + cww w1,  x += cx w   (the previous step's
-// coefficients, which the state still holds: its Givens kernel wrote them
-// and this step's has not run yet)
-template <typename TY, typename T, int P, int VW, bool UPD>
+// partial[(k B + j) nblk + block] for k = 0, 1, 2.  r_new may be r1 (each
+// thread reads and writes the same entries).
+template <typename TY, typename T, int P, int VW>
 __global__ __launch_bounds__(kThreads) void k_minres_gather(
     Geo g, FastDiv divN1, uint32_t B, uint32_t R, const TY* __restrict__ Yc,
     const T* __restrict__ S, const double* __restrict__ D, const T* __restrict__ r2,
-    T* __restrict__ r1, const double* __restrict__ st, double* __restrict__ partial,
-    T* __restrict__ w, const T* __restrict__ w1, T* __restrict__ xs) {
+    const T* r1, T* rnew, const double* __restrict__ st, double* __restrict__ partial) {
   __shared__ double red[kThreads * VW];
   const uint32_t N1 = g.N1;
   const uint32_t nb = B / VW;
@@ -1377,18 +1371,12 @@ __global__ __launch_bounds__(kThreads) void k_minres_gather(
 #pragma unroll
   for (int v = 0; v < VW; ++v) q1[v] = q2[v] = q3[v] = 0.0;
   if (off < per) {
-    double cvn[VW], ca2[VW], cr1[VW], cwv[VW], cw1[VW], cww[VW], cx[VW];
+    double cvn[VW], ca2[VW], cr1[VW];
 #pragma unroll
     for (int v = 0; v < VW; ++v) {
       cvn[v] = st[MS_CVN * B + j0 + v];
       ca2[v] = st[MS_CA2 * B + j0 + v];
       cr1[v] = st[MS_CR1 * B + j0 + v];
-      if constexpr (UPD) {
-        cwv[v] = st[MS_CWV * B + j0 + v];
-        cw1[v] = st[MS_CWW1 * B + j0 + v];
-        cww[v] = st[MS_CWW * B + j0 + v];
-        cx[v] = st[MS_CX * B + j0 + v];
-      }
     }
     const uint32_t nn = N1 * N1 * N1;
     // groups of R consecutive chunks, strided over a grid of at most
@@ -1406,12 +1394,6 @@ __global__ __launch_bounds__(kThreads) void k_minres_gather(
       T xv[VW], zv[VW], ro[VW];
       vload<T, VW>(r2 + i, xv);
       vload<T, VW>(r1 + i, zv);
-      T wv[VW], w1v[VW], sv[VW];
-      if constexpr (UPD) {
-        vload<T, VW>(w + i, wv);
-        vload<T, VW>(w1 + i, w1v);
-        vload<T, VW>(xs + i, sv);
-      }
 #pragma unroll
       for (int v = 0; v < VW; ++v) {
         const double x = (double)xv[v];
@@ -1421,18 +1403,8 @@ __global__ __launch_bounds__(kThreads) void k_minres_gather(
         q1[v] += r * dr;
         q2[v] += dr * dr;
         q3[v] += dr * x;
-        if constexpr (UPD) {
-          const double wn = cwv[v] * (dn * (double)zv[v]) + cw1[v] * (double)wv[v] +
-                            cww[v] * (double)w1v[v];
-          wv[v] = (T)wn;
-          sv[v] = (T)((double)sv[v] + cx[v] * wn);
-        }
       }
-      vstore<T, VW>(r1 + i, ro);
-      if constexpr (UPD) {
-        vstore<T, VW>(w + i, wv);
-        vstore<T, VW>(xs + i, sv);
-      }
+      vstore<T, VW>(rnew + i, ro);
     }
   }
   // partials column-major, [k][column][block], so that each column's
@@ -2128,7 +2100,8 @@ __global__ __launch_bounds__(kThreads) void k_minres_lanczos(int64_t N, int B,
 __global__ __launch_bounds__(kRedThreads) void k_minres_givens(int B, int nblk,
                                                                 const double* __restrict__ partial,
                                                                 const double* __restrict__ negEig,
-                                                                double* __restrict__ st, int nq) {
+                                                                double* __restrict__ st, int nq,
+                                                                double* __restrict__ hist) {
   __shared__ double red[kRedThreads / 64];
   const int j = blockIdx.x;
   double s, q2 = 0.0, q3 = 0.0;
@@ -2149,6 +2122,8 @@ __global__ __launch_bounds__(kRedThreads) void k_minres_givens(int B, int nblk,
     S[MS_CWV * B + j] = 0.0; S[MS_CWW1 * B + j] = 0.0; S[MS_CWW * B + j] = 0.0;
     S[MS_CX * B + j] = 0.0; S[MS_CV * B + j] = 0.0; S[MS_CR1 * B + j] = 0.0;
     S[MS_CVN * B + j] = 0.0;
+    if (hist)
+      for (int k = 0; k < 4; ++k) hist[k * B + j] = 0.0;
     return;
   }
   const double oldb = S[MS_BETA * B + j];
@@ -2181,6 +2156,12 @@ __global__ __launch_bounds__(kRedThreads) void k_minres_givens(int B, int nblk,
   S[MS_CV * B + j] = done ? 0.0 : 1.0 / beta;
   S[MS_CVN * B + j] = S[MS_CV * B + j] * negEig[j];
   S[MS_CR1 * B + j] = done ? 0.0 : -beta / oldb;
+  if (hist) {  // this step's row for k_minres_batch
+    hist[j] = S[MS_CWV * B + j];
+    hist[B + j] = S[MS_CWW1 * B + j];
+    hist[2 * B + j] = S[MS_CWW * B + j];
+    hist[3 * B + j] = phi;
+  }
 }
 
 // w_new = cwv D r + cww1 w1 + cww w  (written over w1);  x += cx w_new,
@@ -2216,6 +2197,61 @@ __global__ void k_minres_update(uint32_t NB, uint32_t B, const T* __restrict__ r
     }
     vstore<T, VW>(w1 + i, wo);
     vstore<T, VW>(x + i, xo);
+  }
+}
+
+// The direction and solution updates of n <= kMinresBatch fused steps in one pass:
+// for each step, with its Lanczos vector r_i and its coefficients hist[(4 i + k) B + j],
+//   w_new = cwv D r_i + cww1 w + cww w1;  x += cx w_new;  (w, w1) <- (w1, w_new).
+// Bound by HBM: n + 6 streams where n updates of their own move 5 n (r is read by the
+// Lanczos recurrence anyway).  With them inside the gather a step moved 8 streams of
+// the block, with batches of 8 it moves 4.75, for 5 more vectors of storage.  All of a
+// thread's loads are issued before the first use; the coefficients come from LDS.
+// place != nullptr: the newest Lanczos vector `last` is copied there (2 more streams),
+// also where place is r_0, whose entry the thread has read by then.
+template <int VW>
+__global__ __launch_bounds__(kThreads) void k_minres_batch(uint32_t N, uint32_t B, int n,
+                                                           MinresVectors rs,
+                                                           const double* __restrict__ D,
+                                                           double* __restrict__ w,
+                                                           double* __restrict__ w1,
+                                                           double* __restrict__ x,
+                                                           const double* __restrict__ hist,
+                                                           const double* last, double* place) {
+  __shared__ double sh[kMinresBatch * 4 * kMaxCols];
+  const uint32_t tid = threadIdx.x, nb = B / VW, per = kThreads / nb;
+  for (uint32_t k = tid; k < 4u * n * B; k += kThreads) sh[k] = hist[k];
+  __syncthreads();
+  const uint32_t off = tid / nb, j0 = (tid % nb) * VW;
+  if (off >= per) return;
+  for (uint32_t node = blockIdx.x * per + off; node < N; node += gridDim.x * per) {
+    const uint32_t i = node * B + j0;
+    double a[VW], b[VW], xv[VW], r[kMinresBatch][VW];
+    vload<double, VW>(w + i, a);
+    vload<double, VW>(w1 + i, b);
+    vload<double, VW>(x + i, xv);
+#pragma unroll
+    for (int k = 0; k < kMinresBatch; ++k)
+      if (k < n) vload<double, VW>(rs.r[k] + i, r[k]);
+    double lv[VW];
+    if (place) vload<double, VW>(last + i, lv);
+    const double dn = D[node];
+#pragma unroll
+    for (int k = 0; k < kMinresBatch; ++k) {
+      if (k >= n) break;
+      const double* c = sh + 4 * k * B + j0;
+#pragma unroll
+      for (int v = 0; v < VW; ++v) {
+        const double wn = c[v] * (dn * r[k][v]) + c[B + v] * a[v] + c[2 * B + v] * b[v];
+        a[v] = b[v];
+        b[v] = wn;
+        xv[v] += c[3 * B + v] * wn;
+      }
+    }
+    vstore<double, VW>(w + i, a);
+    vstore<double, VW>(w1 + i, b);
+    vstore<double, VW>(x + i, xv);
+    if (place) vstore<double, VW>(place + i, lv);
   }
 }
 
@@ -2688,8 +2724,8 @@ template void launch_cell_dot<float, double>(const Geo&, const CellOp<float>&, c
 
 template <typename TY>
 int launch_minres_gather(const Geo& g, const TY* Yc, const double* S, const double* D,
-                         const double* r2, double* r1, int B, const double* st, double* partial,
-                         int gather_rows, hipStream_t s, double* w, const double* w1, double* x) {
+                         const double* r2, const double* r1, double* rnew, int B,
+                         const double* st, double* partial, int gather_rows, hipStream_t s) {
   if (B < 1 || B > kMaxCols) throw Error(IDFT_EINVAL, "block width out of range");
   check_u32(g.N * B);
   check_u32(cell_scratch_elems(g, B));
@@ -2699,15 +2735,9 @@ int launch_minres_gather(const Geo& g, const TY* Yc, const double* S, const doub
   const int vw = gather_vw(B, (int)sizeof(double));
   gather_grid(g, B, vw, gather_rows, gx, gy, R);
   gx = std::min<unsigned>(gx, (unsigned)kMinresGatherBlocks);
-#define IDFT_MG(PP, VW)                                                                   \
-  do {                                                                                     \
-    if (w)                                                                                 \
-      k_minres_gather<TY, double, PP, VW, true><<<dim3(gx), kThreads, 0, s>>>(             \
-          g, divN1, (uint32_t)B, R, Yc, S, D, r2, r1, st, partial, w, w1, x);              \
-    else                                                                                   \
-      k_minres_gather<TY, double, PP, VW, false><<<dim3(gx), kThreads, 0, s>>>(            \
-          g, divN1, (uint32_t)B, R, Yc, S, D, r2, r1, st, partial, nullptr, nullptr, nullptr); \
-  } while (0)
+#define IDFT_MG(PP, VW)                                                            \
+  k_minres_gather<TY, double, PP, VW><<<dim3(gx), kThreads, 0, s>>>(               \
+      g, divN1, (uint32_t)B, R, Yc, S, D, r2, r1, rnew, st, partial)
 #define IDFT_MG_P(PP)   \
   if (vw == 2) IDFT_MG(PP, 2); \
   else IDFT_MG(PP, 1);
@@ -2724,11 +2754,11 @@ int launch_minres_gather(const Geo& g, const TY* Yc, const double* S, const doub
   return (int)gx;
 }
 template int launch_minres_gather<double>(const Geo&, const double*, const double*, const double*,
-                                          const double*, double*, int, const double*, double*, int,
-                                          hipStream_t, double*, const double*, double*);
+                                          const double*, const double*, double*, int,
+                                          const double*, double*, int, hipStream_t);
 template int launch_minres_gather<float>(const Geo&, const float*, const double*, const double*,
-                                         const double*, double*, int, const double*, double*, int,
-                                         hipStream_t, double*, const double*, double*);
+                                         const double*, const double*, double*, int,
+                                         const double*, double*, int, hipStream_t);
 
 template <typename T>
 void launch_lincomb(int64_t N, int B, T* Y, double beta, const T* X, double a, const double* ca,
@@ -2973,8 +3003,26 @@ template int launch_minres_lanczos<float>(int64_t, int, const float*, const floa
 template int launch_minres_lanczos<double>(int64_t, int, const double*, const double*, double*,
                                            const double*, const double*, double*, hipStream_t);
 void launch_minres_givens(int B, int nblk, const double* partial, const double* negEig, double* st,
-                          hipStream_t s, int nq) {
-  k_minres_givens<<<B, kRedThreads, 0, s>>>(B, nblk, partial, negEig, st, nq);
+                          hipStream_t s, int nq, double* hist) {
+  k_minres_givens<<<B, kRedThreads, 0, s>>>(B, nblk, partial, negEig, st, nq, hist);
+  IDFT_HIP(hipGetLastError());
+}
+void launch_minres_batch(int64_t N, int B, int n, const MinresVectors& rs, const double* D,
+                         double* w, double* w1, double* x, const double* hist,
+                         const double* last, double* place, hipStream_t s) {
+  if (B < 1 || B > kMaxCols || n < 1 || n > kMinresBatch)
+    throw Error(IDFT_EINVAL, "block width or batch out of range");
+  check_u32(N * B);
+  const int vw = B % 2 == 0 ? 2 : 1, per = kThreads / (B / vw);
+  // a few work-groups per CU in flight, each over several chunks (its 20 KB of
+  // coefficients are loaded once)
+  const unsigned grid = (unsigned)std::min<int64_t>((N + per - 1) / per, 8192);
+  if (vw == 2)
+    k_minres_batch<2><<<grid, kThreads, 0, s>>>((uint32_t)N, (uint32_t)B, n, rs, D, w, w1, x, hist,
+                                            last, place);
+  else
+    k_minres_batch<1><<<grid, kThreads, 0, s>>>((uint32_t)N, (uint32_t)B, n, rs, D, w, w1, x, hist,
+                                            last, place);
   IDFT_HIP(hipGetLastError());
 }
 template <typename T>
