@@ -317,6 +317,15 @@ void launch_minres_givens(int B, int nblk, const double* partial, const double* 
 template <typename T>
 void launch_minres_update(int64_t N, int B, const T* r, const double* D, T* w1, const T* w, T* x,
                           const double* st, hipStream_t s);
+// Lanczos bound of the spectrum (see k_lan_start): lan has 2 k + 4 doubles, partial at
+// least 1024 and the operator's dot rows.  step: y = H v_j (v_j = r inv, inv at
+// lan[2 k]) with nalpha partials of v_j . y becomes r_{j+1}; rp (null at j = 0) = r_{j-1}.
+template <typename T>
+void launch_lan_start(int64_t N, uint64_t seed, const unsigned char* mask, T* r, double* partial,
+                      int k, double* lan, hipStream_t s);
+template <typename T>
+void launch_lan_step(int64_t N, T* y, const T* r, const T* rp, int nalpha, double* partial, int k,
+                     int j, double* lan, hipStream_t s);
 void launch_copy_done(int B, const double* st, int* flags, hipStream_t s);
 // TFLOP/s of `chains` independent FMA chains per thread over 32 work-groups
 // per CU (FP64 or FP32, unpacked), timed with HIP events on stream s

@@ -114,6 +114,7 @@ struct idft_ctx {
   idft_stats st{};
   AdjointState adj;
   MinresWork<double> mw64;
+  DevBuf<double> lanBuf, lanSt;  // Lanczos bound: three vectors, the scalars
   DevBuf<double> mst, mx, mtmp, mnegc, mcell, mhist, pairCoef;
   DevBuf<int> mflags, msel, pairList;
   idft_mv mvPsi, mvX;
@@ -441,37 +442,33 @@ struct idft_ctx {
   template <typename T>
   void lanczos_t(double& upper, double& lowest) {
     const int k = std::max(2, d.lanczos_steps);
-    std::vector<double> hv((size_t)t.N), hb;
-    std::vector<unsigned char> mask((size_t)t.N);
-    bnd.download(mask.data(), mask.size(), s);
-    sync();
-    uint64_t sd = d.seed ^ 0x5bd1e995ULL;
-    double nrm = 0.0;
-    for (int64_t n = 0; n < t.N; ++n) {
-      const double r = rand_pm1(sd);
-      hv[n] = mask[n] ? 0.0 : r;
-      nrm += hv[n] * hv[n];
-    }
-    nrm = std::sqrt(nrm);
-    for (auto& v : hv) v /= nrm;
-    DevBuf<double> v64(t.N);
-    v64.upload(hv.data(), hv.size(), s);
-    DevBuf<T> v(t.N), vp(t.N), w(t.N);
-    convert_to(v64.p, v.p, t.N);
-    launch_lincomb<T>(t.N, 1, vp.p, 0.0, nullptr, 0.0, nullptr, nullptr, 0.0, nullptr, nullptr, s);
-    std::vector<double> al, be;
-    double beta = 0.0;
+    lanBuf.resize(3 * (size_t)t.N);
+    lanSt.resize(2 * (size_t)k + 4);
+    T* base = reinterpret_cast<T*>(lanBuf.p);
+    T *rp = base, *r = base + t.N, *y = base + 2 * (size_t)t.N;
+    const int rows = gather_blocks(
+        g, 1, std::is_same<T, double>::value ? shape64.gather_rows : shape32.gather_rows,
+        (int)sizeof(T));
+    partial.resize(std::max(1024, rows));
+    launch_lan_start<T>(t.N, d.seed ^ 0x5bd1e995ULL, bnd.p, r, partial.p, k, lanSt.p, s);
     for (int j = 0; j < k; ++j) {
-      happly<T>(v.p, w.p, 1, 1.0);
-      const double a = coldot_t<T>(v.p, w.p, 1)[0];
-      launch_lincomb<T>(t.N, 1, w.p, 1.0, v.p, -a, nullptr, vp.p, -beta, nullptr, nullptr, s);
-      const double b2 = std::sqrt(std::max(coldot_t<T>(w.p, w.p, 1)[0], 0.0));
-      al.push_back(a);
-      be.push_back(b2);
-      beta = b2;
-      if (b2 == 0.0) break;
-      std::swap(vp.p, v.p);
-      launch_lincomb<T>(t.N, 1, v.p, 0.0, w.p, 1.0 / b2, nullptr, nullptr, 0.0, nullptr, nullptr, s);
+      ApplyEpilogue<T> ep;  // y = H v with the partials of v.y, v = inv r
+      ep.Y = y;
+      ep.xcol = lanSt.p + 2 * k;
+      ep.dot_partial = partial.p;
+      const int na = apply<T>(r, 1, ep);
+      launch_lan_step<T>(t.N, y, r, j ? rp : nullptr, na, partial.p, k, j, lanSt.p, s);
+      T* o = rp;
+      rp = r; r = y; y = o;
+    }
+    std::vector<double> ab(2 * (size_t)k);
+    lanSt.download(ab.data(), ab.size(), s);
+    sync();
+    std::vector<double> al, be;
+    for (int j = 0; j < k; ++j) {
+      al.push_back(ab[j]);
+      be.push_back(ab[k + j]);
+      if (ab[k + j] == 0.0) break;
     }
     const int kk = (int)al.size();
     std::vector<double> T3((size_t)kk * kk, 0.0), ev, V;
@@ -483,22 +480,6 @@ struct idft_ctx {
     upper = ev[kk - 1] + std::fabs(be[kk - 1]);
     lowest = ev[0];
   }
-
-  template <typename T>
-  std::vector<double> coldot_t(const T* a, const T* b2, int b) {
-    partial.resize((size_t)1024 * std::max(b, 1));
-    small.resize(std::max(b, 16));
-    const int nb = launch_coldot_partial<T>(t.N, b, a, b2, nullptr, partial.p, s);
-    launch_sum_partials(nb, b, partial.p, small.p, s);
-    std::vector<double> out(b);
-    small.download(out.data(), b, s);
-    sync();
-    return out;
-  }
-  void convert_to(const double* a, double* o, int64_t n) {
-    IDFT_HIP(hipMemcpyAsync(o, a, n * sizeof(double), hipMemcpyDeviceToDevice, s));
-  }
-  void convert_to(const double* a, float* o, int64_t n) { launch_convert_d2f(n, o, a, s); }
 
   // Scaled Chebyshev filter (Zhou-Saad) of X in place, FP64 or FP32.
   template <typename T>
@@ -1560,6 +1541,7 @@ struct idft_ctx {
   void release_eigen_work() {
     X2.release(); HX.release(); Xtmp.release();
     F0.release(); F1.release(); F2.release(); Rf.release();
+    lanBuf.release();
     haveHX = false;
   }
   void release_adjoint_work() {

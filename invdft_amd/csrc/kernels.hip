@@ -2030,6 +2030,75 @@ __global__ __launch_bounds__(kRedThreads) void k_minres_alpha_cell(int B, int nc
   st[MS_CA2 * B + j] = done ? 0.0 : -a / st[MS_BETA * B + j];
 }
 
+// Lanczos bound of the spectrum with its scalars on the device (one host round trip
+// for the k steps where dots read by the host took two per step: about 25 us each, a
+// tenth of a small problem's evaluation).  r_j are the unscaled vectors, v_j = r_j inv_j;
+// lan holds [k] alphas, [k] betas, then inv_j, inv_{j-1}, ca = -alpha inv_j and
+// cb = -beta_{j-1} inv_{j-1}.
+// r_0: the n-th number in (-1, 1) of the splitmix64 sequence from `seed`, 0 on the
+// boundary, with the block partials of r_0 . r_0.
+template <typename T>
+__global__ __launch_bounds__(kThreads) void k_lan_start(uint32_t N, uint64_t seed,
+                                                        const unsigned char* __restrict__ mask,
+                                                        T* __restrict__ r,
+                                                        double* __restrict__ partial) {
+  __shared__ double red[kThreads / 64];
+  double t = 0.0;
+  for (uint32_t n = blockIdx.x * kThreads + threadIdx.x; n < N; n += gridDim.x * kThreads) {
+    uint64_t z = seed + 0x9e3779b97f4a7c15ULL * ((uint64_t)n + 1);
+    z = (z ^ (z >> 30)) * 0xbf58476d1ce4e5b9ULL;
+    z = (z ^ (z >> 27)) * 0x94d049bb133111ebULL;
+    z ^= z >> 31;
+    const T v = (T)(mask[n] ? 0.0 : 2.0 * ((double)(z >> 11) * 0x1.0p-53) - 1.0);
+    r[n] = v;
+    t += (double)v * (double)v;
+  }
+  t = block_total<kThreads>(t, red);
+  if (threadIdx.x == 0) partial[blockIdx.x] = t;
+}
+// j < 0: the norm of r_0; else beta_j = |r_{j+1}|.  A vanishing vector gets inv = 0: the
+// steps after it are zero and the host cuts them off.
+__global__ __launch_bounds__(kRedThreads) void k_lan_beta(int nblk, const double* __restrict__ partial,
+                                                          int k, int j, double* __restrict__ lan) {
+  __shared__ double red[kRedThreads / 64];
+  const double b = sqrt(fmax(block_sum_contig<kRedThreads>(partial, nblk, red), 0.0));
+  if (threadIdx.x != 0) return;
+  double* c = lan + 2 * k;
+  const double inv = c[0];
+  if (j >= 0) lan[k + j] = b;
+  c[0] = b > 0.0 ? 1.0 / b : 0.0;
+  c[1] = inv;
+  c[3] = j >= 0 ? -b * inv : 0.0;
+}
+__global__ __launch_bounds__(kRedThreads) void k_lan_alpha(int nblk, const double* __restrict__ partial,
+                                                           int k, int j, double* __restrict__ lan) {
+  __shared__ double red[kRedThreads / 64];
+  const double a = block_sum_contig<kRedThreads>(partial, nblk, red);
+  if (threadIdx.x != 0) return;
+  lan[j] = a;
+  lan[2 * k + 2] = -a * lan[2 * k];
+}
+// y <- y + ca r + cb rp, with the block partials of y . y
+template <typename T>
+__global__ __launch_bounds__(kThreads) void k_lan_update(uint32_t N, T* __restrict__ y,
+                                                         const T* __restrict__ r,
+                                                         const T* __restrict__ rp,
+                                                         const double* __restrict__ c,
+                                                         double* __restrict__ partial) {
+  __shared__ double red[kThreads / 64];
+  const double ca = c[2], cb = c[3];
+  double t = 0.0;
+  for (uint32_t n = blockIdx.x * kThreads + threadIdx.x; n < N; n += gridDim.x * kThreads) {
+    double v = (double)y[n] + ca * (double)r[n];
+    if (rp) v += cb * (double)rp[n];
+    const T o = (T)v;
+    y[n] = o;
+    t += (double)o * (double)o;
+  }
+  t = block_total<kThreads>(t, red);
+  if (threadIdx.x == 0) partial[blockIdx.x] = t;
+}
+
 // Partials of r.D r and (D r).(D r) per column (rows [0, nblk) and
 // [nblk, 2 nblk) of partial): the start of a fused MINRES solve.
 __global__ __launch_bounds__(kThreads) void k_minres_start_dots(int64_t N, int B,
@@ -2841,8 +2910,6 @@ int launch_coldot_partial(int64_t N, int B, const T* X, const T* Y, const double
   IDFT_HIP(hipGetLastError());
   return nb;
 }
-template int launch_coldot_partial<float>(int64_t, int, const float*, const float*, const double*,
-                                          double*, hipStream_t);
 template int launch_coldot_partial<double>(int64_t, int, const double*, const double*,
                                            const double*, double*, hipStream_t);
 
@@ -3041,6 +3108,33 @@ template void launch_minres_update<float>(int64_t, int, const float*, const doub
                                           const float*, float*, const double*, hipStream_t);
 template void launch_minres_update<double>(int64_t, int, const double*, const double*, double*,
                                            const double*, double*, const double*, hipStream_t);
+static int lan_blocks(int64_t N) { return (int)std::min<int64_t>((N + kThreads - 1) / kThreads, 1024); }
+template <typename T>
+void launch_lan_start(int64_t N, uint64_t seed, const unsigned char* mask, T* r, double* partial,
+                      int k, double* lan, hipStream_t s) {
+  check_u32(N);
+  const int nb = lan_blocks(N);
+  k_lan_start<T><<<nb, kThreads, 0, s>>>((uint32_t)N, seed, mask, r, partial);
+  k_lan_beta<<<1, kRedThreads, 0, s>>>(nb, partial, k, -1, lan);
+  IDFT_HIP(hipGetLastError());
+}
+template <typename T>
+void launch_lan_step(int64_t N, T* y, const T* r, const T* rp, int nalpha, double* partial, int k,
+                     int j, double* lan, hipStream_t s) {
+  const int nb = lan_blocks(N);
+  k_lan_alpha<<<1, kRedThreads, 0, s>>>(nalpha, partial, k, j, lan);
+  k_lan_update<T><<<nb, kThreads, 0, s>>>((uint32_t)N, y, r, rp, lan + 2 * k, partial);
+  k_lan_beta<<<1, kRedThreads, 0, s>>>(nb, partial, k, j, lan);
+  IDFT_HIP(hipGetLastError());
+}
+#define IDFT_LAN(T)                                                                            \
+  template void launch_lan_start<T>(int64_t, uint64_t, const unsigned char*, T*, double*, int, \
+                                    double*, hipStream_t);                                     \
+  template void launch_lan_step<T>(int64_t, T*, const T*, const T*, int, double*, int, int,    \
+                                   double*, hipStream_t);
+IDFT_LAN(float)
+IDFT_LAN(double)
+#undef IDFT_LAN
 void launch_copy_done(int B, const double* st, int* flags, hipStream_t s) {
   k_copy_done<<<(B + 63) / 64, 64, 0, s>>>(B, st, flags);
   IDFT_HIP(hipGetLastError());
