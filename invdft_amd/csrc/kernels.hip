@@ -83,6 +83,29 @@ __device__ inline void tree_cols(double* red, int per, int B, int tid, int off) 
     n = h;
   }
 }
+// The same for NQ sums of VW columns per thread at once: thread tid = k nb + g holds
+// q[n][v] of column g VW + v (threads past per nb hold nothing), and the sums over k < per
+// arrive in red[n][g VW + v].  A tree: one thread per column adding `per` values in turn
+// took half of the gather's time at 2 columns (per = 256).
+template <int NQ, int VW>
+__device__ inline void tree_groups(double (&red)[NQ][kThreads * VW], const double (&q)[NQ][VW],
+                                   uint32_t per, uint32_t nb, uint32_t tid, uint32_t off) {
+#pragma unroll
+  for (int n = 0; n < NQ; ++n)
+#pragma unroll
+    for (int v = 0; v < VW; ++v) red[n][tid * VW + v] = q[n][v];
+  for (uint32_t n = per; n > 1;) {
+    __syncthreads();
+    const uint32_t h = (n + 1) / 2;
+    if (off < n - h)
+#pragma unroll
+      for (int k = 0; k < NQ; ++k)
+#pragma unroll
+        for (int v = 0; v < VW; ++v) red[k][tid * VW + v] += red[k][(tid + h * nb) * VW + v];
+    n = h;
+  }
+  __syncthreads();
+}
 
 // Work-group size of the per-column reductions of long partial rows (cell
 // dots, gather partials, Gram partials): 16 waves, about 12 values per thread
@@ -1216,14 +1239,14 @@ __global__ __launch_bounds__(kThreads) void k_cell_gather(
     const double* __restrict__ cb, const T* __restrict__ W, double c,
     const double* __restrict__ cc, const T* __restrict__ Xin, const double* __restrict__ xn,
     const double* __restrict__ xcol, T* __restrict__ V, double* __restrict__ partial) {
-  __shared__ double red[kThreads * VW];
+  __shared__ double red[1][kThreads * VW];
   const uint32_t N1 = g.N1;
   const uint32_t nb = B / VW;  // column groups of a node
   const uint32_t tid = threadIdx.x, per = kThreads / nb;
   const uint32_t jg = tid % nb, off = tid / nb, j0 = jg * VW;
-  double dot[VW];
+  double dot[1][VW];
 #pragma unroll
-  for (int v = 0; v < VW; ++v) dot[v] = 0.0;
+  for (int v = 0; v < VW; ++v) dot[0][v] = 0.0;
   if (off < per) {
     double caj[VW], cbj[VW], ccj[VW], xs[VW];
 #pragma unroll
@@ -1263,7 +1286,7 @@ __global__ __launch_bounds__(kThreads) void k_cell_gather(
 #pragma unroll
         for (int v = 0; v < VW; ++v) {
           vv[v] = (T)(xs[v] * (sn * (double)xin[v]));
-          dot[v] += (double)vv[v] * (double)yo[v];
+          dot[0][v] += (double)vv[v] * (double)yo[v];
         }
         if (V) vstore<T, VW>(V + i, vv);
       }
@@ -1271,15 +1294,8 @@ __global__ __launch_bounds__(kThreads) void k_cell_gather(
     }
   }
   if (partial) {
-#pragma unroll
-    for (int v = 0; v < VW; ++v) red[tid * VW + v] = dot[v];
-    __syncthreads();
-    if (tid < B) {
-      const uint32_t g2 = tid / VW, v = tid % VW;
-      double t = 0.0;
-      for (uint32_t k = 0; k < per; ++k) t += red[(k * nb + g2) * VW + v];
-      partial[((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * B + tid] = t;
-    }
+    tree_groups<1, VW>(red, dot, per, nb, tid, off);
+    if (tid < B) partial[((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * B + tid] = red[0][tid];
   }
 }
 
@@ -1362,14 +1378,14 @@ __global__ __launch_bounds__(kThreads) void k_minres_gather(
     Geo g, FastDiv divN1, uint32_t B, uint32_t R, const TY* __restrict__ Yc,
     const T* __restrict__ S, const double* __restrict__ D, const T* __restrict__ r2,
     const T* r1, T* rnew, const double* __restrict__ st, double* __restrict__ partial) {
-  __shared__ double red[kThreads * VW];
+  __shared__ double red[3][kThreads * VW];
   const uint32_t N1 = g.N1;
   const uint32_t nb = B / VW;
   const uint32_t tid = threadIdx.x, per = kThreads / nb;
   const uint32_t jg = tid % nb, off = tid / nb, j0 = jg * VW;
-  double q1[VW], q2[VW], q3[VW];
+  double q[3][VW];
 #pragma unroll
-  for (int v = 0; v < VW; ++v) q1[v] = q2[v] = q3[v] = 0.0;
+  for (int v = 0; v < VW; ++v) q[0][v] = q[1][v] = q[2][v] = 0.0;
   if (off < per) {
     double cvn[VW], ca2[VW], cr1[VW];
 #pragma unroll
@@ -1400,9 +1416,9 @@ __global__ __launch_bounds__(kThreads) void k_minres_gather(
         const double t = sn * sum[v] + (cvn[v] * dn + ca2[v]) * x + cr1[v] * (double)zv[v];
         ro[v] = (T)t;
         const double r = (double)ro[v], dr = dn * r;
-        q1[v] += r * dr;
-        q2[v] += dr * dr;
-        q3[v] += dr * x;
+        q[0][v] += r * dr;
+        q[1][v] += dr * dr;
+        q[2][v] += dr * x;
       }
       vstore<T, VW>(rnew + i, ro);
     }
@@ -1410,21 +1426,9 @@ __global__ __launch_bounds__(kThreads) void k_minres_gather(
   // partials column-major, [k][column][block], so that each column's
   // reduction reads contiguous memory
   const int64_t nblk = (int64_t)gridDim.x;
-  auto emit = [&](int k, const double (&q)[VW]) {
-#pragma unroll
-    for (int v = 0; v < VW; ++v) red[tid * VW + v] = q[v];
-    __syncthreads();
-    if (tid < B) {
-      const uint32_t g2 = tid / VW, v = tid % VW;
-      double t = 0.0;
-      for (uint32_t m = 0; m < per; ++m) t += red[(m * nb + g2) * VW + v];
-      partial[((int64_t)k * B + tid) * nblk + blockIdx.x] = t;
-    }
-    __syncthreads();
-  };
-  emit(0, q1);
-  emit(1, q2);
-  emit(2, q3);
+  tree_groups<3, VW>(red, q, per, nb, tid, off);
+  for (uint32_t c = tid; c < 3 * B; c += kThreads)
+    partial[(int64_t)c * nblk + blockIdx.x] = red[c / B][c % B];
 }
 
 // ------------------------------------------------------ Hamiltonian build
@@ -2171,15 +2175,39 @@ __global__ __launch_bounds__(kRedThreads) void k_minres_givens(int B, int nblk,
                                                                 const double* __restrict__ negEig,
                                                                 double* __restrict__ st, int nq,
                                                                 double* __restrict__ hist) {
-  __shared__ double red[kRedThreads / 64];
+  __shared__ double red[3 * (kRedThreads / 64)];
   const int j = blockIdx.x;
   double s, q2 = 0.0, q3 = 0.0;
-  if (nq >= 3) {  // fused steps: [k][column][block] partials
-    s = block_sum_contig<kRedThreads>(partial + (int64_t)j * nblk, nblk, red);
+  if (nq >= 3) {  // fused steps: [k][column][block] partials, the three sums in one pass
+    const double* p = partial + (int64_t)j * nblk;
+    const int64_t row = (int64_t)B * nblk;
+    s = 0.0;
+    for (int b = threadIdx.x; b < nblk; b += kRedThreads) {
+      s += p[b];
+      q2 += p[row + b];
+      q3 += p[2 * row + b];
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      s += __shfl_xor(s, o, 64);
+      q2 += __shfl_xor(q2, o, 64);
+      q3 += __shfl_xor(q3, o, 64);
+    }
+    constexpr int kW = kRedThreads / 64;
+    const int wave = threadIdx.x >> 6;
+    if ((threadIdx.x & 63) == 0) {
+      red[wave] = s;
+      red[kW + wave] = q2;
+      red[2 * kW + wave] = q3;
+    }
     __syncthreads();
-    q2 = block_sum_contig<kRedThreads>(partial + ((int64_t)B + j) * nblk, nblk, red);
-    __syncthreads();
-    q3 = block_sum_contig<kRedThreads>(partial + ((int64_t)2 * B + j) * nblk, nblk, red);
+    s = q2 = q3 = 0.0;
+#pragma unroll
+    for (int w = 0; w < kW; ++w) {
+      s += red[w];
+      q2 += red[kW + w];
+      q3 += red[2 * kW + w];
+    }
   } else {
     s = block_sum_col<kRedThreads>(partial, nblk, B, j, red);
   }
