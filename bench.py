@@ -69,14 +69,13 @@ def sf_flops_per_cell_column(p):
 # HBM bytes per launch of the cell-product kernels from two rocprofv3 --pmc runs
 # (FETCH_SIZE, WRITE_SIZE) of `bench.py --kernels-only --shape ...`, FETCH_SIZE
 # scaled by the copy calibration (x1.926), WRITE_SIZE as read; the summaries
-# with the commands are profiles/cell_sf_inverse_24c_p5_pmc.md (shape 1 4 4 2),
-# profiles/cell_sf_batched_40c_p4_pmc.md (1 8 8 2) and
+# with the commands are profiles/cell_plane_pmc.md (shape 1 4 4 2) and
 # profiles/cell_gemm_inverse_24c_p5_pmc.md (2 16 4 0 and 1 16 0 1).
 MEASURED_TRAFFIC = {
-    ("inverse_24c_p5", "k_cell_sf<float,float,5,4,1,false>"): 276.3e6,
-    ("inverse_24c_p5", "k_cell_sf<double,double,5,4,1,false>"): 552.5e6,
-    ("batched_40c_p4", "k_cell_sf<float,float,4,8,1,false>"): 4245.0e6,
-    ("batched_40c_p4", "k_cell_sf<double,double,4,8,1,false>"): 9262.7e6,
+    ("inverse_24c_p5", "k_cell_plane<float,float,5,false,true>"): 276.7e6,
+    ("inverse_24c_p5", "k_cell_plane<double,double,5,false,true>"): 554.4e6,
+    ("batched_40c_p4", "k_cell_plane<float,float,4,false,true>"): 4263.6e6,
+    ("batched_40c_p4", "k_cell_plane<double,double,4,false,true>"): 9255.1e6,
     ("inverse_24c_p5", "k_cell_gemm<float,float,5,1>"): 2613e6,
     ("inverse_24c_p5", "k_cell_symm<float,float,5,1>"): 1691e6,
 }
@@ -273,7 +272,7 @@ def c3_leg(lib, cheb_tol):
         nbytes = 8 * (cells * (p + 3) ** 3 + N * (B + 1) + cells * (p + 1) ** 3 * B)
         ms = out["fp64"]["fp64_cell_product_ms"]
         ach = flops / (ms * 1e-3) / 1e12
-        kname = f"k_cell_sf<double,double,{p},{sh['vectors_per_tile']},1,false>"
+        kname = f"k_cell_plane<double,double,{p},false,true>"
         roof = {"bound": "valu", "kernel": kname,
                 "achieved": round(ach, 2), "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
                 "frac": round(ach / FP64_PEAK_TFLOPS, 4),
@@ -538,7 +537,7 @@ def main():
     #    algorithmic bytes per launch are the symmetric H_e (ne(ne+1)/2 entries
     #    per cell) read once, the block X and node scale S read once and the
     #    per-cell products written once (the gather kernel reads them back);
-    #  - the sum-factorised kernel (k_cell_sf) is bound by the vector ALUs; its
+    #  - the sum-factorised kernel (k_cell_plane) is bound by the vector ALUs; its
     #    algorithmic work per launch is the 1D contractions, sf_flops(p) per
     #    cell and column, and it moves w_e + X + S + the per-cell products.
     # The timed launches are plain applications (no node scale on the input).
@@ -559,8 +558,7 @@ def main():
         sz, tn = (4, "float") if fp32 else (8, "double")
         kern = shape["kernel"]
         if kern == abi.KERNEL_SUM_FACTOR:
-            kname = (f"k_cell_sf<{tn},{tn},{p},{shape['vectors_per_tile']},"
-                     f"{shape['cells_per_wg']},false>")
+            kname = f"k_cell_plane<{tn},{tn},{p},false,true>"
             fl = s.n_cells * B * sf_flops_per_cell_column(p)
             peak = FP32_PEAK_TFLOPS if fp32 else FP64_PEAK_TFLOPS
             tf = fl / (ms_cell * 1e-3) / 1e12

@@ -274,6 +274,18 @@ struct idft_ctx {
     }
     launch_right_mult(t.N, b, a, small2.p, out, ns, beta, s);
   }
+  // the node scales of a MINRES step's input, formed by the first solve (a caller with
+  // its own solver has no use for them)
+  void ensure_step_scales() {
+    if (!SD.p) {
+      SD.resize(t.N);
+      launch_scale_product<double>(t.N, SD.p, S.p, Djac.p, s);
+    }
+    if (mixed && !SD32.p) {
+      SD32.resize(t.N);
+      launch_scale_product<float>(t.N, SD32.p, S32.p, Djac.p, s);
+    }
+  }
   void zero_boundary(double* v, int b) { launch_zero_boundary(g, b, v, s); }
 
   // ------------------------------------------------------ Hamiltonian
@@ -346,6 +358,7 @@ struct idft_ctx {
       profYf.resize(n);
       launch_convert_d2f((int64_t)(n * kProfBlocks), profXf.p, profX.p, s);
     }
+    ensure_step_scales();
     int blk = 0;  // input block of the next application
     auto xdp = [&] { return profX.p + n * (blk++ % kProfBlocks); };
     auto xfp = [&] { return profXf.p + n * (blk++ % kProfBlocks); };
@@ -977,6 +990,7 @@ struct idft_ctx {
     // any step is captured into a graph
     (void)op64();
     if (canRelax) (void)op32();
+    ensure_step_scales();
     // dot partials of every block width the compaction may reach
     int nblk = 1024;
     for (int bw = 1; bw <= b; ++bw) {
@@ -1810,10 +1824,6 @@ idft_ctx* create_ctx(const idft_desc* d, const double* pot_base_q, const double*
     c->invSqrtM.upload(isq.data(), t.N, s);
     c->Djac.upload(Dj.data(), t.N, s);
     c->DjacSqrt.upload(Djs.data(), t.N, s);
-    c->SD.resize(t.N);
-    c->SD32.resize(t.N);
-    launch_scale_product<double>(t.N, c->SD.p, c->S.p, c->Djac.p, s);
-    launch_scale_product<float>(t.N, c->SD32.p, c->S32.p, c->Djac.p, s);
     c->bnd.upload(bnd.data(), t.N, s);
     c->adjMask.upload(am.data(), t.N, s);
     if (pot_base_q) {

@@ -1299,7 +1299,7 @@ __global__ __launch_bounds__(kThreads) void k_cell_gather(
   }
 }
 
-// Node sums of the quadrature operator's cell products (k_cell_sf without the
+// Node sums of the quadrature operator's cell products (k_cell_plane without the
 // kinetic chain) and, while a node's row is at hand, the pair sums
 //   partial[k gridDim.x + block] = sum over the block's nodes of
 //                                  asc[n] A[n][i_k] T[n][j_k],  k < np <= 256,
