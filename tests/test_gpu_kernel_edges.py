@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 
 from invdft_amd import abi
-from tests.helpers import bare_pair, rel
+from tests.helpers import bare_pair, random_veff, rel
 from tests.setup_abi import poisson
 
 pytestmark = pytest.mark.gpu
@@ -104,3 +104,30 @@ def test_cell_product_wave_edges_match_oracle(glib, olib, p, n_cells, ncols):
     # sums of some 10^2 products per entry and axis: well below 1e3 roundings
     assert rel(g.apply_hamiltonian(x, precision=abi.FP64), want) < 1e-13
     assert rel(g.apply_hamiltonian(x, precision=abi.MIXED), want) < 2e-6
+
+
+# runs of 1, 2, 3, 8 and 9 steps (batches of 1, 2, 3, 8, and 5 + 4; with the checkpoint
+# option at most 3), the last run of a solve cut short by its step limit
+@pytest.mark.parametrize("check_every,steps,ckpt", [(1, 3, 0), (2, 5, 0), (3, 7, 1), (8, 8, 1),
+                                                    (8, 19, 0), (9, 20, 0)])
+def test_batched_minres_updates_match_separate_steps(glib, olib, check_every, steps, ckpt):
+    _say("minres_batch", check_every, steps, ckpt)
+    b, rng = 3, np.random.default_rng(steps)
+    out = []
+    for fused in (1, 0):
+        d = abi.default_desc(olib, n_cells=3, degree=3, half_width=4.0, n_eig=b, n_electrons=2.0,
+                             check_every=check_every, minres_fused=fused, psi_checkpoint=ckpt)
+        s = abi.geometry(olib, d)
+        zq = np.zeros(s.n_cells * s.quad_per_cell)
+        g = abi.Context(glib, d, zq, zq, np.ones(zq.size), np.ones(s.n_nodes))
+        g.set_veff_quad(random_veff(olib, d, 0))
+        if not out:
+            psi = np.linalg.qr(rng.standard_normal((s.n_nodes, b)))[0]
+            u = rng.standard_normal(s.n_cells * s.quad_per_cell)
+        mp, x = g.mv(b, psi), g.mv(b)
+        g.adj_update_input_psi(mp, np.full(b, 0.5), u, [(i, i) for i in range(b)], -0.5,
+                               np.array([-1.5, -1.2, -0.7]))
+        g.minres_solve(x, None, 1e-30, steps, distribute=False)
+        out.append(x.get())
+    # at most 20 steps from the same start: rounding grows by the condition number, < 1e4
+    assert rel(out[0], out[1]) < 1e-10
