@@ -43,13 +43,15 @@ int idft_profile_apply(idft_ctx* ctx, int32_t ncols, int32_t precision, int32_t 
  *     partial sums of all block rows per wave and applies to 16-column tiles
  *     (and 32 in FP32), wider tiles run the row pass.  The stored H_e is
  *     built on first use.
- *   IDFT_KERNEL_SUM_FACTOR: vectors_per_tile 2, 4 or 8 and cells_per_wg 1; the
- *     kernel fills its waves at any block width and has no shape to choose. */
+ *   IDFT_KERNEL_SUM_FACTOR: vectors_per_tile = columns per work-group of the
+ *     FP64 MINRES steps, 2, 4 or 8 (the other products fill their waves at any
+ *     block width and have no shape to choose); cells_per_wg must be 1. */
 int idft_set_apply_shape(idft_ctx* ctx, int32_t precision, int32_t cells_per_wg,
                          int32_t vectors_per_tile, int32_t kernel, int32_t gather_rows);
 
-/* Autotuner of the cell operator: times the sum-factorised kernel, then every
- * stored-H shape
+/* Autotuner of the cell operator: times the sum-factorised kernels (in FP64 at
+ * every column count per work-group; 2 only for blocks narrower than 8
+ * columns), then every stored-H shape
  * cells-per-work-group in {1,2,4,8} x vectors-per-tile in {16,32,64} (tiles
  * wider than the block collapse to one pass) x {row pass, tile pass} where
  * it applies, then node chunks per gather work-group in {default,1,2,4,8} with

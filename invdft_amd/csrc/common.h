@@ -157,7 +157,7 @@ struct ApplyEpilogue {
   const T* W = nullptr; double c = 0.0; const double* cc = nullptr;
   const double* xn = nullptr;    // node scale of the operator input and of X
   const double* sxn = nullptr;   // with xn: the product Sg xn (launch_scale_product), which the
-                                 // sum-factorised kernel reads in place of both
+                                 // sum-factorised FP32 kernel reads in place of both
   const double* xcol = nullptr;  // column scale of the operator input
   T* V = nullptr;                // stores the scaled input xcol xn Xin (needs dot_partial)
   double* dot_partial = nullptr;
@@ -177,9 +177,10 @@ enum CellKernel {
 // Launch shape of the cell product (chosen by the autotuner).
 struct GemmShape {
   int cells_per_wg = 1;       // stored-H kernels: cells processed in sequence by one work-group;
-                              // sum-factorised kernel: 1
+                              // sum-factorised kernels: 1
   int vectors_per_tile = 80;  // stored-H kernels: columns per tile (rounded to 16; >= B: one
-                              // pass); sum-factorised kernel: 2, 4 or 8, without effect
+                              // pass); sum-factorised: columns per work-group of the FP64
+                              // MINRES steps' kernel, 2, 4 or 8
   int gather_rows = 0;        // node chunks (256 / (B / VW) nodes each) per gather work-group
                               // (0: about kGatherBlocks groups)
   int kernel = CK_ROW_PASS;   // CellKernel; the tile pass applies to 16-column tiles (FP32 also 32)
@@ -238,8 +239,7 @@ void launch_lincomb_df2d(int64_t N, int B, double* Y, const double* X, double a,
                          const double* ca, const float* Z, double b, const double* cb,
                          hipStream_t s);
 // y = a b in FP64
-template <typename T>
-void launch_scale_product(int64_t n, double* y, const T* a, const double* b, hipStream_t s);
+void launch_scale_product(int64_t n, double* y, const float* a, const double* b, hipStream_t s);
 void launch_convert_d2f(int64_t n, float* y, const double* x, hipStream_t s);
 void launch_convert_f2d(int64_t n, double* y, const float* x, hipStream_t s);
 int coldot_blocks(int64_t N, int B);
@@ -276,6 +276,9 @@ void launch_quad_pairs(const Geo& g, const double* W, int64_t wstride, const dou
                        int wb, double* Yc, const double* A, int lda, const double* asc, double* T2,
                        int ldt, const int* pairs, int np, DevBuf<double>& partial, double* out,
                        hipStream_t s);
+// Y += N^T diag(wq) N X over the cells of one colour
+void launch_quad_operator(const Geo& g, const DevTables& t, const double* X, int B,
+                          const double* wq, double* Y, int colour, hipStream_t s);
 // Y = S T (+ column scale cc, and psi's node scale q, with rhs) + psi C for a C
 // with few entries: coef[e] of column i at e in [list[i], list[i + 1]), its row
 // (psi's column) list[B + 1 + e].

@@ -79,7 +79,7 @@ struct idft_ctx {
   bool verbose = false;  // IDFT_VERBOSE set: solver progress on stderr
   // static per-node / per-quadrature data
   DevBuf<double> S, sqrtM, invSqrtM, Djac, DjacSqrt, Mdiag, jxw;
-  DevBuf<double> SD, SD32;  // S Djac and S32 Djac: the node scales of a MINRES step's input
+  DevBuf<double> SD32;  // S32 Djac: the node scale of an FP32 MINRES step's input
   DevBuf<float> S32;
   DevBuf<unsigned char> bnd, adjMask;
   DevBuf<double> potBase, rhoT, weight, veff, rho, u;
@@ -274,16 +274,12 @@ struct idft_ctx {
     }
     launch_right_mult(t.N, b, a, small2.p, out, ns, beta, s);
   }
-  // the node scales of a MINRES step's input, formed by the first solve (a caller with
-  // its own solver has no use for them)
-  void ensure_step_scales() {
-    if (!SD.p) {
-      SD.resize(t.N);
-      launch_scale_product<double>(t.N, SD.p, S.p, Djac.p, s);
-    }
+  // the node scale of an FP32 MINRES step's input, formed by the first solve (a caller
+  // with its own solver has no use for it)
+  void ensure_step_scale() {
     if (mixed && !SD32.p) {
       SD32.resize(t.N);
-      launch_scale_product<float>(t.N, SD32.p, S32.p, Djac.p, s);
+      launch_scale_product(t.N, SD32.p, S32.p, Djac.p, s);
     }
   }
   void zero_boundary(double* v, int b) { launch_zero_boundary(g, b, v, s); }
@@ -358,7 +354,7 @@ struct idft_ctx {
       profYf.resize(n);
       launch_convert_d2f((int64_t)(n * kProfBlocks), profXf.p, profX.p, s);
     }
-    ensure_step_scales();
+    ensure_step_scale();
     int blk = 0;  // input block of the next application
     auto xdp = [&] { return profX.p + n * (blk++ % kProfBlocks); };
     auto xfp = [&] { return profXf.p + n * (blk++ % kProfBlocks); };
@@ -370,7 +366,7 @@ struct idft_ctx {
         ApplyEpilogue<double> ep;
         ep.Y = yd.p;
         ep.xn = Djac.p;
-        ep.sxn = f32 ? SD32.p : SD.p;
+        ep.sxn = f32 ? SD32.p : nullptr;
         ep.xcol = ones.p;
         if (f32) apply_f32op(xdp(), ncols, ep);
         else apply<double>(xdp(), ncols, ep);
@@ -735,17 +731,24 @@ struct idft_ctx {
       launch_quad_pairs(g, wq, wstride, Bv + j, b, wj, Yc64.p, A, b, asc, T2 ? T2 + j : nullptr, b,
                         adj.dpairs.p, fused ? np : 0, partial, small.p, s);
     }
-    if (!fused)  // pairs in runs of the node-dot kernel's 256
-      for (int k = 0; k < np; k += 256) {
-        const int m = std::min(256, np - k);
-        partial.resize((size_t)1024 * m);
-        const int nb = launch_pairdot_partial(t.N, b, A, T2, asc, adj.dpairs.p + 2 * k, m, partial.p, s);
-        launch_sum_partials(nb, m, partial.p, small.p + k, s);
-      }
+    if (!fused) node_pairs(A, asc, T2, b);
     std::vector<double> out(np);
     if (np) small.download(out.data(), np, s);
     sync();
     return out;
+  }
+
+  // small[k] = sum_n asc[n] A[n][i_k] T[n][j_k], the pairs in runs of the node-dot
+  // kernel's 256
+  void node_pairs(const double* A, const double* asc, const double* T, int b) {
+    const int np = (int)adj.pairs.size() / 2;
+    small.resize(std::max(np, 16));
+    for (int k = 0; k < np; k += 256) {
+      const int m = std::min(256, np - k);
+      partial.resize((size_t)1024 * m);
+      const int nb = launch_pairdot_partial(t.N, b, A, T, asc, adj.dpairs.p + 2 * k, m, partial.p, s);
+      launch_sum_partials(nb, m, partial.p, small.p + k, s);
+    }
   }
 
   void compute_mu(const std::vector<double>& occv) {
@@ -823,7 +826,8 @@ struct idft_ctx {
     A.ready = true;
   }
 
-  void compute_rhs(idft_mv* x, double* rhs) {
+  // ordered: in the order of sums that a MINRES solve keeps (see k_cell_line)
+  void compute_rhs(idft_mv* x, double* rhs, bool ordered = false) {
     AdjointState& A = adj;
     if (!A.ready) throw Error(IDFT_ESTATE, "computeRhs before updateInputPsi");
     const int b = A.B;
@@ -834,13 +838,23 @@ struct idft_ctx {
     // sum_q u JxW psi_i psi_j = psi_i . (R psi)_j
     T2buf.resize(NB(b));
     double* T2 = T2buf.p;
-    A.pairQ = quad_pairs(psi, nullptr, psi, b, A.uJxW.p, t.nq, T2);
+    if (ordered) {
+      launch_lincomb<double>(t.N, b, T2, 0.0, nullptr, 0.0, nullptr, nullptr, 0.0, nullptr, nullptr, s);
+      for (int colour = 0; colour < 8; ++colour)
+        launch_quad_operator(g, dt, psi, b, A.uJxW.p, T2, colour, s);
+      node_pairs(psi, nullptr, T2, b);
+      A.pairQ.resize(A.pairs.size() / 2);
+      if (!A.pairQ.empty()) small.download(A.pairQ.data(), A.pairQ.size(), s);
+      sync();
+    } else {
+      A.pairQ = quad_pairs(psi, nullptr, psi, b, A.uJxW.p, t.nq, T2);
+    }
     A.havePairQ = true;
     compute_mu(A.occ);
     // rhs = 4 f M^{-1/2} R psi - 2 sqrt(M) psi Mu   (column i: sum_k Mu[k][i] psi_k)
     std::vector<double> C((size_t)b * b);
     for (size_t k = 0; k < C.size(); ++k) C[k] = -2.0 * A.Mu[k];
-    const int nnz = pair_lists(C, b);
+    const int nnz = ordered ? -1 : pair_lists(C, b);
     if (nnz >= 0) {
       launch_pair_combine(t.N, b, true, T2, S.p, sqrtM.p, psi, A.docc4.p, pairCoef.p, pairList.p,
                           nnz, rhs, s);
@@ -990,7 +1004,7 @@ struct idft_ctx {
     // any step is captured into a graph
     (void)op64();
     if (canRelax) (void)op32();
-    ensure_step_scales();
+    ensure_step_scale();
     // dot partials of every block width the compaction may reach
     int nblk = 1024;
     for (int bw = 1; bw <= b; ++bw) {
@@ -1066,8 +1080,8 @@ struct idft_ctx {
       } else {
         st.applies_fp64++;
         st.apply_cols_fp64 += bc;
-        launch_cell_dot<double, double>(g, op64(), S.p, rb, bc, Djac.p, SD.p, cv, Yc64.p, mcell.p,
-                                        shape64, s);
+        launch_cell_dot<double, double>(g, op64(), S.p, rb, bc, Djac.p, nullptr, cv, Yc64.p,
+                                        mcell.p, shape64, s);
       }
       launch_minres_alpha_cell(bc, (int)t.ncell, mcell.p, mst.p, s);
       const int nbk =
@@ -1123,7 +1137,7 @@ struct idft_ctx {
       ep.X = r2; ep.a = 1.0; ep.ca = mst.p + (size_t)MS_CVN * bc;
       ep.Z = r1; ep.b = 1.0; ep.cb = mst.p + (size_t)MS_CR1 * bc;
       ep.xn = Djac.p;
-      ep.sxn = f32op ? SD32.p : SD.p;
+      ep.sxn = f32op ? SD32.p : nullptr;
       ep.xcol = mst.p + (size_t)MS_CV * bc;
       ep.dot_partial = partial.p;
       int nbk = f32op ? apply_f32op(r2, bc, ep) : apply<double>(r2, bc, ep);
@@ -1286,7 +1300,7 @@ struct idft_ctx {
     if (x->ncols != b) throw Error(IDFT_EINVAL, "block size mismatch");
     DevBuf<double>& rhs = mw64.rhs;
     rhs.resize(NB(b));
-    compute_rhs(x, rhs.p);
+    compute_rhs(x, rhs.p, true);
     {
       std::vector<double> nr = coldot(rhs.p, rhs.p, b);
       for (double v : nr)
@@ -2262,9 +2276,18 @@ int idft_autotune_apply(idft_ctx* c, int32_t ncols, int32_t prec, int32_t reps,
     };
     target.gather_rows = 0;
     target.kernel = CK_SUM_FACTOR;
-    target.vectors_per_tile = 4;
     target.cells_per_wg = 1;
-    trial();
+    for (int cg : {2, 4, 8}) {
+      if (f32 && cg != 4) continue;           // without effect in FP32
+      if (!f32 && cg > 2 && cg / 2 >= ncols) continue;  // mostly empty column groups
+      // 2 columns per work-group gather each node row of the block once per
+      // 2 columns.  Between the solvers' other vector kernels this measured
+      // 1.3x slower than 4 columns at B = 12 (FP64 MINRES, kernel trace), a
+      // cost that a timing loop of back-to-back applications does not show.
+      if (cg == 2 && ncols >= 8) continue;
+      target.vectors_per_tile = cg;
+      trial();
+    }
     const int tpMax = f32 ? 32 : 16;  // widest tile of the tile-pass kernel
     for (int vt : widths) {
       for (int k = CK_ROW_PASS; k <= (vt <= tpMax ? CK_TILE_PASS : CK_ROW_PASS); ++k) {

@@ -107,6 +107,28 @@ __device__ inline void tree_groups(double (&red)[NQ][kThreads * VW], const doubl
   __syncthreads();
 }
 
+// The same sums in the order of the positions k = 0, 1, .. per - 1, all NQ VW nb <= 256
+// of them at once: returns sum c (column c % (VW nb) of quantity c / (VW nb)) to the
+// thread that asks for it.  For the dots of a MINRES step, whose order is fixed (see
+// k_cell_line).
+template <int NQ, int VW>
+__device__ inline double ordered_groups(double (&red)[NQ][kThreads * VW],
+                                        const double (&q)[NQ][VW], uint32_t per, uint32_t nb,
+                                        uint32_t tid, uint32_t c) {
+#pragma unroll
+  for (int n = 0; n < NQ; ++n)
+#pragma unroll
+    for (int v = 0; v < VW; ++v) red[n][tid * VW + v] = q[n][v];
+  __syncthreads();
+  const uint32_t B = nb * VW;
+  double t = 0.0;
+  if (c < NQ * B) {
+    const double* row = red[c / B] + c % B;
+    for (uint32_t k = 0; k < per; ++k) t += row[k * B];
+  }
+  return t;
+}
+
 // Work-group size of the per-column reductions of long partial rows (cell
 // dots, gather partials, Gram partials): 16 waves, about 12 values per thread
 // for the 12-16 k values of a column.
@@ -596,6 +618,8 @@ __global__ __launch_bounds__(kSymmThreads) void k_cell_symm(Geo g, const T* __re
 // barrier each) moved 4850 and left a quarter of its lanes idle in most stages.
 // Slots are numbered cell B + column over the whole mesh, so that a wave is full at
 // every block width.
+// It takes every FP32 product and the FP64 ones of the operator, the filter and the
+// quadrature operator; the FP64 steps of MINRES keep the line-by-line kernel below.
 // Bound by VALU issue: about 60 % of it in FP64, 80 % in FP32 (2 to 5 waves per
 // SIMD; FP64 at p = 5 takes 246 registers).  Measured against the line-by-line
 // kernel, us of the cell product alone: FP64 27 cells p = 3 B = 12 135 -> 96,
@@ -839,7 +863,7 @@ struct PlaneScale {
 // Yc = Lq^T diag(w_e) Lq X_e, the quadrature operator of a weight.  wstride: the
 // weights' step from cell to cell (0: the same weights in every cell); ldx: the row
 // length of X (B, or more for a block of columns).  XN: node-scaled input, and with
-// dotp also each slot's x.(H_e x), dotp[column * ncell + cell].
+// dotp also each slot's x.(H_e x), dotp[column * ncell + cell] (FP32 products alone).
 template <typename T, typename TV, int P, bool XN, bool KIN>
 __global__ __launch_bounds__(64, 2) void k_cell_plane(
     Geo g, T hq, const T* __restrict__ W, uint32_t wstride,
@@ -1135,6 +1159,366 @@ __global__ __launch_bounds__(64, 2) void k_cell_plane(
   }
 }
 
+// ---------------------------------------- cell product line by line (MINRES, FP64)
+// The FP64 product of the MINRES steps: the same chain as k_cell_plane, but each
+// contraction of the tensor along a line of the cell, with the input scaled on the
+// fly and the cell's dots x.(H_e x).  An iterate that a step limit stops is not
+// determined by its inputs in 64 bits: once a Ritz value has converged the Lanczos
+// vectors amplify rounding (two orders of the same sums gave iterates 1e-8 to 1e-2
+// apart after 30 to 64 steps on meshes of 17 to 63 nodes per axis, and 1e-14 apart
+// on 100).  So the steps keep one order of arithmetic, this one, and an iterate
+// stopped after k steps stays what it has been; its price is the plane kernel's
+// gain in FP64 solves (24 cells p = 5 B = 12: 261 against 233 us, 30 p = 4 B = 64:
+// 1383 against 1139).  Do not regroup a sum here.
+//
+// One work-group handles one cell and CG columns; an item is one line of the cell's
+// tensor along one axis for one column.  Intermediates live in LDS as [entry][CG],
+// with padded line strides (N1 and Q rounded up to odd: 5, 7 at p = 4; 7, 9 at
+// p = 5) so that the 64 lanes of a wave spread over the banks.  The exception is
+// region D at p = 5 (Q = 8): unpadded lines, entry x of line (c, y) at slot x ^ y,
+// which spreads the lanes as the stride 9 does and puts the lines that one stage-6
+// item reads 512 B apart, so that the compiler pairs those accesses.  The kinetic
+// chain runs first and the x-line input stays in registers for the potential chain;
+// the y and z stages overwrite their input in place.  Region Bk is dead once stage
+// 3 has run, so D shares its memory:
+//   1  x lines (c,b):  ka = M x -> A,  kb = D x -> Bk      (x gathered from HBM)
+//   2  y lines (c,a):  k1 = M ka -> A,  k2 = D ka + M kb -> Bk
+//   3  z lines (b,a):  yk = D k1 + M k2 -> A
+//   4  x lines (c,b):  t1[c][b][qx] = Lq x -> D             (x from registers)
+//   5  y lines (c,qx): t2[c][qy][qx] = Lq t1 -> D
+//   6  z lines (qy,qx): s2 = Lq^T (w .* (Lq t2)) -> D
+//   7  y lines (c,qx): s1[c][b][qx] = Lq^T s2 -> D
+//   8  x lines (c,b):  Yc[e][(c,b,a)][j] = (Lq^T s1)[a] + (h/4) yk[a]
+__host__ __device__ constexpr int cmax(int a, int b) { return a > b ? a : b; }
+
+// Coefficient W (0 even, 1 odd, 2 middle) of row I, column J of operator A: a scalar
+// load from the table eo (EoTable<P>::v).
+template <class A, int I, int J, int W>
+__device__ inline double eo_coef(const double* __restrict__ eo) {
+  using E = EoTable<A::kP>;
+  constexpr int c = E::C(A::kK);
+  constexpr int idx = E::base(A::kK) + I * E::stride(A::kK) +
+                      (W == 0 ? J : W == 1 ? c / 2 + J : 2 * (c / 2));
+  return eo[idx];
+}
+// Adds row I's even and odd sums of A applied to the split input (xp, xm).
+template <class A, int I>
+__device__ inline void eo_row(const double (&xp)[(A::C + 1) / 2], const double (&xm)[A::C / 2],
+                              double& e, double& o, const double* __restrict__ eo) {
+  static_for<0, A::C / 2>([&](auto j) {
+    constexpr int J = decltype(j)::value;
+    e += eo_coef<A, I, J, 0>(eo) * xp[J];
+    if constexpr (2 * I + 1 != A::R) o += eo_coef<A, I, J, 1>(eo) * xm[J];
+  });
+  if constexpr (A::C % 2 == 1) e += eo_coef<A, I, 0, 2>(eo) * xp[A::C / 2];
+}
+// The R outputs of one or more even-odd contractions: rows(i, e, o) adds the
+// sums of row i, put(i, y) receives output i (i an integral constant).
+template <int R, typename Rows, typename Put>
+__device__ inline void eo_out(Rows&& rows, Put&& put) {
+  static_for<0, (R + 1) / 2>([&](auto i) {
+    constexpr int I = decltype(i)::value;
+    double e = 0.0, o = 0.0;
+    rows(i, e, o);
+    if constexpr (2 * I + 1 == R) {
+      put(i, e);
+    } else {
+      put(i, e + o);
+      put(ic<R - 1 - I>{}, e - o);
+    }
+  });
+}
+#define IDFT_IC(x) decltype(x)::value
+// Entry A of a line from its even-odd split (pl_split): the inverse of the
+// split, to rounding.
+template <int C, int A>
+__device__ inline double eo_unsplit(const double (&xp)[(C + 1) / 2], const double (&xm)[C / 2]) {
+  if constexpr (2 * A + 1 == C) {
+    return xp[A];
+  } else if constexpr (A < C / 2) {
+    return 0.5 * (xp[A] + xm[A]);
+  } else {
+    constexpr int J = C - 1 - A;
+    return 0.5 * (xp[J] - xm[J]);
+  }
+}
+
+template <int P, int CG>
+__global__ __launch_bounds__(kThreads) void k_cell_line(
+    Geo g, double hq, const double* __restrict__ W, const double* __restrict__ S,
+    const double* __restrict__ X, const double* __restrict__ xn, const double* __restrict__ xcol,
+    double* __restrict__ Yc, int B, double* __restrict__ dotp, const double* __restrict__ eo) {
+  constexpr int N1 = P + 1, Q = P + 3, N2 = N1 * N1, NE = N2 * N1, Q2 = Q * Q;
+  constexpr int QP = Q | 1, N1P = N1 | 1, NV = CG;
+  constexpr int HE = (N1 + 1) / 2, HO = N1 / 2, QE = (Q + 1) / 2, QO = Q / 2;
+  // x-line items per thread (lines x columns over the work-group)
+  constexpr int KI = (N2 * NV + kThreads - 1) / kThreads;
+  typedef SfTab<P, 0> TL;
+  typedef SfTab<P, 1> TLt;
+  typedef SfTab<P, 2> TM;
+  typedef SfTab<P, 3> TD;
+  // regions, each [entry][NV]:
+  //   A  [(c,b)][N1P]      ka -> k1 -> yk            (kinetic chain, in place)
+  //   Bk [(c,b)][N1P]      kb -> k2                  (stages 1-3)
+  //   D  [c][Q][QS]        t1 -> t2 -> s2 -> s1      (stages 4-8, over Bk)
+  // SWZ: D unpadded (QS = Q = 8), entry (c, y, x) at slot x ^ y of its line
+  constexpr bool SWZ = Q == 8;
+  constexpr int QS = SWZ ? Q : QP;
+  __shared__ __align__(16) double rA[N2 * N1P * NV];
+  __shared__ __align__(16) double rBD[cmax(N2 * N1P, N1 * Q * QS) * NV];
+  double* const rB = rBD;
+  // Byte offsets into D of entry (c, y, x), column jv, from a per-item base and the
+  // one index that is a compile-time constant at the access (so that the rest folds
+  // into the LDS instruction's offset field):
+  //   dy(c, x, jv) then at_y(base, y);  dx(c, y, jv) then at_x(base, x);
+  //   dc(y, x, jv) then at_c(base, c).
+  // With SWZ the slot x ^ y is an XOR of the offset's slot bits (the slot
+  // field, NV sizeof(double) bytes per slot and 8 slots, holds no other bits).
+  constexpr uint32_t SB = NV * sizeof(double);
+  const auto dy = [](uint32_t c, uint32_t x, uint32_t jv) -> uint32_t {
+    return (c * Q * QS + x) * SB + jv * (uint32_t)sizeof(double);
+  };
+  const auto at_y = [](uint32_t base, uint32_t y) -> uint32_t {
+    return SWZ ? (base ^ (y * SB)) + y * QS * SB : base + y * QS * SB;
+  };
+  const auto dx = [](uint32_t c, uint32_t y, uint32_t jv) -> uint32_t {
+    return ((c * Q + y) * QS + (SWZ ? y : 0u)) * SB + jv * (uint32_t)sizeof(double);
+  };
+  const auto at_x = [](uint32_t base, uint32_t x) -> uint32_t {
+    return SWZ ? base ^ (x * SB) : base + x * SB;
+  };
+  const auto dc = [](uint32_t y, uint32_t x, uint32_t jv) -> uint32_t {
+    return (y * QS + (SWZ ? (x ^ y) : x)) * SB + jv * (uint32_t)sizeof(double);
+  };
+  const auto at_c = [](uint32_t base, uint32_t c) -> uint32_t { return base + c * Q * QS * SB; };
+  char* const rDb = reinterpret_cast<char*>(rBD);
+  const auto dref = [rDb](uint32_t off) -> double& { return *reinterpret_cast<double*>(rDb + off); };
+  // (cell, column group) pairs dealt to the 8 XCDs in contiguous runs, the
+  // groups of one cell at consecutive slots of one XCD, so that they share
+  // that XCD's L2 for the cell's rows of X and of the cell scratch (each group
+  // holds CG of the B columns of a row).  Every index below fits in 32 bits
+  // (the host checks N B and cells n_e B against 2^32).
+  const uint32_t ncell = (uint32_t)g.ncell, nc = (uint32_t)g.nc, np = (uint32_t)g.p;
+  const uint32_t NN = (uint32_t)g.N1, ub = (uint32_t)B;
+  const uint32_t ngrp = (ub + CG - 1) / CG, npair = ncell * ngrp;
+  const uint32_t per = (npair + 7) / 8;
+  const uint32_t k = (blockIdx.x % 8) * per + blockIdx.x / 8;
+  if (k >= npair) return;
+  const uint32_t e = k / ngrp;
+  const int c0 = (int)(k % ngrp) * CG;
+  const int bw = min(CG, B - c0);
+  const int tid = threadIdx.x;
+  const uint32_t cx = e % nc, cy = (e / nc) % nc, cz = e / (nc * nc);
+  const double* we = W + e * (uint32_t)(Q2 * Q);
+  // this thread's column (every item of a thread has column tid % NV, since kThreads
+  // is a multiple of NV) and its scale, loaded first: a later load would make its
+  // first use wait for the weights too
+  const int jv = tid % NV;
+  const double xc = xcol ? xcol[c0 + min(jv, bw - 1)] : 1.0;
+  // the quadrature weights of this thread's stage-6 items, loaded now so that
+  // their latency hides behind stages 1-5 (item it6 = tid + k6 kThreads takes
+  // w_e[qz][ln6] for its line ln6 = it6 / NV)
+  constexpr int K6 = (Q2 * NV + kThreads - 1) / kThreads;
+  double wpre[K6][Q];
+#pragma unroll
+  for (int k6 = 0; k6 < K6; ++k6) {
+    const int it6 = tid + k6 * kThreads;
+    const int ln6 = it6 < Q2 * NV ? it6 / NV : 0;
+#pragma unroll
+    for (int qz = 0; qz < Q; ++qz) wpre[k6][qz] = we[qz * Q2 + ln6];
+  }
+  // the input lines stay in registers from stage 1 to stage 8 (even-odd split)
+  double keep_p[KI][HE], keep_m[KI][HO];
+  // stage 1: x lines ln = c*N1 + b of the gathered input -> ka = M x, kb = D x
+#pragma unroll
+  for (int ki = 0; ki < KI; ++ki) {
+    const int it = tid + ki * kThreads;
+    if (it >= N2 * NV) break;
+    const int ln = it / NV;
+    double v[N1];
+    const uint32_t b = ln % N1, c = ln / N1;
+    const uint32_t n0 = ((cz * np + c) * NN + (cy * np + b)) * NN + cx * np;
+    // the line's N1 nodes are consecutive: one base pointer per array, the nodes at
+    // immediate offsets (the X rows B apart), all loads issued before the first product
+    const double* Sp = S + n0;
+    if (jv < bw) {
+      const double* Xp = X + (size_t)n0 * ub + (uint32_t)(c0 + jv);
+      double sv[N1], xv[N1], nv[N1];
+#pragma unroll
+      for (int a = 0; a < N1; ++a) {
+        sv[a] = Sp[a];
+        xv[a] = Xp[(size_t)a * ub];
+        nv[a] = xn[n0 + a];
+      }
+#pragma unroll
+      for (int a = 0; a < N1; ++a) {
+        double x = sv[a] * xv[a];
+        x *= nv[a];
+        if (xcol) x *= xc;
+        v[a] = x;
+      }
+    } else {
+#pragma unroll
+      for (int a = 0; a < N1; ++a) v[a] = 0.0;
+    }
+    pl_split<N1>(v, keep_p[ki], keep_m[ki]);
+    eo_out<N1>(
+        [&](auto i, double& s, double& d) { eo_row<TM, IDFT_IC(i)>(keep_p[ki], keep_m[ki], s, d, eo); },
+        [&](auto a2, double r) { rA[(ln * N1P + IDFT_IC(a2)) * NV + jv] = r; });
+    eo_out<N1>(
+        [&](auto i, double& s, double& d) { eo_row<TD, IDFT_IC(i)>(keep_p[ki], keep_m[ki], s, d, eo); },
+        [&](auto a2, double r) { rB[(ln * N1P + IDFT_IC(a2)) * NV + jv] = r; });
+  }
+  __syncthreads();
+  // stage 2: y lines (c, a) of the kinetic chain, in place:
+  // k1 = M ka (over ka), k2 = D ka + M kb (over kb)
+  for (int it = tid; it < N2 * NV; it += kThreads) {
+    const int l2 = it / NV;
+    const int a = l2 % N1, c = l2 / N1;
+    double va[N1], vb[N1], ap[HE], am[HO], bp[HE], bm[HO];
+#pragma unroll
+    for (int b = 0; b < N1; ++b) {
+      va[b] = rA[((c * N1 + b) * N1P + a) * NV + jv];
+      vb[b] = rB[((c * N1 + b) * N1P + a) * NV + jv];
+    }
+    pl_split<N1>(va, ap, am);
+    pl_split<N1>(vb, bp, bm);
+    eo_out<N1>([&](auto i, double& s, double& d) { eo_row<TM, IDFT_IC(i)>(ap, am, s, d, eo); },
+               [&](auto b2, double r) { rA[((c * N1 + IDFT_IC(b2)) * N1P + a) * NV + jv] = r; });
+    eo_out<N1>(
+        [&](auto i, double& s, double& d) {
+          eo_row<TD, IDFT_IC(i)>(ap, am, s, d, eo);
+          eo_row<TM, IDFT_IC(i)>(bp, bm, s, d, eo);
+        },
+        [&](auto b2, double r) { rB[((c * N1 + IDFT_IC(b2)) * N1P + a) * NV + jv] = r; });
+  }
+  __syncthreads();
+  // stage 3: z lines (b, a) of the kinetic chain: yk = D k1 + M k2 (over k1)
+  for (int it = tid; it < N2 * NV; it += kThreads) {
+    const int l2 = it / NV;  // l2 = b * N1 + a
+    const int a = l2 % N1, b = l2 / N1;
+    double v1[N1], v2[N1], p1[HE], m1[HO], p2[HE], m2[HO];
+#pragma unroll
+    for (int c = 0; c < N1; ++c) {
+      v1[c] = rA[((c * N1 + b) * N1P + a) * NV + jv];
+      v2[c] = rB[((c * N1 + b) * N1P + a) * NV + jv];
+    }
+    pl_split<N1>(v1, p1, m1);
+    pl_split<N1>(v2, p2, m2);
+    eo_out<N1>(
+        [&](auto i, double& s, double& d) {
+          eo_row<TD, IDFT_IC(i)>(p1, m1, s, d, eo);
+          eo_row<TM, IDFT_IC(i)>(p2, m2, s, d, eo);
+        },
+        [&](auto c2, double r) { rA[((IDFT_IC(c2) * N1 + b) * N1P + a) * NV + jv] = r; });
+  }
+  __syncthreads();
+  // stage 4: x lines of the potential chain from the kept input:
+  // t1[c][b][qx] = Lq x (over k2, which stage 3 has consumed)
+#pragma unroll
+  for (int ki = 0; ki < KI; ++ki) {
+    const int it = tid + ki * kThreads;
+    if (it >= N2 * NV) break;
+    const int ln = it / NV;
+    const int b = ln % N1, c = ln / N1;
+    const uint32_t base = dx(c, b, jv);
+    eo_out<Q>(
+        [&](auto i, double& s, double& d) { eo_row<TL, IDFT_IC(i)>(keep_p[ki], keep_m[ki], s, d, eo); },
+        [&](auto q, double r) { dref(at_x(base, IDFT_IC(q))) = r; });
+  }
+  __syncthreads();
+  // stage 5: y lines (c, qx): t2[c][qy][qx] = Lq t1, in place (over t1)
+  for (int it = tid; it < N1 * Q * NV; it += kThreads) {
+    const int ln = it / NV;
+    const int qx = ln % Q, c = ln / Q;
+    const uint32_t base = dy(c, qx, jv);
+    double v[N1], vp[HE], vm[HO];
+#pragma unroll
+    for (int b = 0; b < N1; ++b) v[b] = dref(at_y(base, b));
+    pl_split<N1>(v, vp, vm);
+    eo_out<Q>([&](auto i, double& s, double& d) { eo_row<TL, IDFT_IC(i)>(vp, vm, s, d, eo); },
+              [&](auto qy, double r) { dref(at_y(base, IDFT_IC(qy))) = r; });
+  }
+  __syncthreads();
+  // stage 6: z lines (qy, qx) through the quadrature weights, in place:
+  // s2 = Lq^T (w .* (Lq t2)) (over t2)
+#pragma unroll
+  for (int k6 = 0; k6 < K6; ++k6) {
+    const int it = tid + k6 * kThreads;
+    if (it >= Q2 * NV) break;
+    const int ln = it / NV;  // ln = qy * Q + qx
+    const int qx = ln % Q, qy = ln / Q;
+    const uint32_t base = dc(qy, qx, jv);
+    double v[N1], vp[HE], vm[HO];
+#pragma unroll
+    for (int c = 0; c < N1; ++c) v[c] = dref(at_c(base, c));
+    pl_split<N1>(v, vp, vm);
+    double u[Q], up[QE], um[QO];
+    eo_out<Q>([&](auto i, double& s, double& d) { eo_row<TL, IDFT_IC(i)>(vp, vm, s, d, eo); },
+              [&](auto qz, double r) { u[IDFT_IC(qz)] = r * wpre[k6][IDFT_IC(qz)]; });
+    pl_split<Q>(u, up, um);
+    eo_out<N1>([&](auto i, double& s, double& d) { eo_row<TLt, IDFT_IC(i)>(up, um, s, d, eo); },
+               [&](auto c, double r) { dref(at_c(base, IDFT_IC(c))) = r; });
+  }
+  __syncthreads();
+  // stage 7: y lines back (c, qx), in place: s1[c][b][qx] = Lq^T s2 (over s2)
+  for (int it = tid; it < N1 * Q * NV; it += kThreads) {
+    const int ln = it / NV;
+    const int qx = ln % Q, c = ln / Q;
+    const uint32_t base = dy(c, qx, jv);
+    double v[Q], vp[QE], vm[QO];
+#pragma unroll
+    for (int qy = 0; qy < Q; ++qy) v[qy] = dref(at_y(base, qy));
+    pl_split<Q>(v, vp, vm);
+    eo_out<N1>([&](auto i, double& s, double& d) { eo_row<TLt, IDFT_IC(i)>(vp, vm, s, d, eo); },
+               [&](auto b, double r) { dref(at_y(base, IDFT_IC(b))) = r; });
+  }
+  __syncthreads();
+  // stage 8: x lines back (c, b) plus the kinetic part, into the cell scratch; with
+  // dotp also the cell's x.(H_e x) per column, into dotp[column * ncell + cell] (x
+  // from the kept input lines: each item holds the same line as in stage 1)
+  double dotv = 0.0;
+#pragma unroll
+  for (int ki = 0; ki < KI; ++ki) {
+    const int it = tid + ki * kThreads;
+    if (it >= N2 * NV) break;
+    const int ln = it / NV;
+    if (jv >= bw) continue;
+    const int b = ln % N1, c = ln / N1;
+    const uint32_t base = dx(c, b, jv);
+    double v[Q], vp[QE], vm[QO];
+#pragma unroll
+    for (int qx = 0; qx < Q; ++qx) v[qx] = dref(at_x(base, qx));
+    pl_split<Q>(v, vp, vm);
+    double* yp = Yc + (size_t)((e * NE + ln * N1) * ub + c0 + jv);
+    eo_out<N1>([&](auto i, double& s, double& d) { eo_row<TLt, IDFT_IC(i)>(vp, vm, s, d, eo); },
+               [&](auto a, double r) {
+                 constexpr int A = IDFT_IC(a);
+                 const double y = hq * rA[(ln * N1P + A) * NV + jv] + r;
+                 yp[(size_t)A * ub] = y;
+                 if (dotp) dotv += eo_unsplit<N1, A>(keep_p[ki], keep_m[ki]) * y;
+               });
+  }
+  if (dotp) {
+    // per column jv: the threads tid = jv (mod NV) (kThreads and 64 are
+    // multiples of NV), summed over each wave, then over the 4 waves
+    __syncthreads();  // stage 8 has read rA
+    const int lane = tid & 63, wave = tid >> 6;
+    double t = dotv;
+#pragma unroll
+    for (int o = 32; o >= NV; o >>= 1) t += __shfl_xor(t, o, 64);
+    if (lane < NV) rA[wave * NV + lane] = t;
+    __syncthreads();
+    if (tid < bw) {
+      double d = 0.0;
+#pragma unroll
+      for (int w = 0; w < kThreads / 64; ++w) d += rA[w * NV + tid];
+      dotp[(size_t)(uint32_t)(c0 + tid) * ncell + e] = d;
+    }
+  }
+}
+#undef IDFT_IC
+
 // Phase 2: every node sums its contributions from the (at most 8) cells that
 // share it -- found arithmetically on the structured mesh, so no atomics and
 // no colouring -- and combines them with up to three other blocks:
@@ -1294,8 +1678,14 @@ __global__ __launch_bounds__(kThreads) void k_cell_gather(
     }
   }
   if (partial) {
-    tree_groups<1, VW>(red, dot, per, nb, tid, off);
-    if (tid < B) partial[((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * B + tid] = red[0][tid];
+    double t;
+    if (xn) {  // a MINRES step: its fixed order of sums
+      t = ordered_groups<1, VW>(red, dot, per, nb, tid, tid);
+    } else {
+      tree_groups<1, VW>(red, dot, per, nb, tid, off);
+      t = red[0][tid];
+    }
+    if (tid < B) partial[((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * B + tid] = t;
   }
 }
 
@@ -1426,9 +1816,8 @@ __global__ __launch_bounds__(kThreads) void k_minres_gather(
   // partials column-major, [k][column][block], so that each column's
   // reduction reads contiguous memory
   const int64_t nblk = (int64_t)gridDim.x;
-  tree_groups<3, VW>(red, q, per, nb, tid, off);
-  for (uint32_t c = tid; c < 3 * B; c += kThreads)
-    partial[(int64_t)c * nblk + blockIdx.x] = red[c / B][c % B];
+  const double t = ordered_groups<3, VW>(red, q, per, nb, tid, tid);
+  if (tid < 3 * B) partial[(int64_t)tid * nblk + blockIdx.x] = t;
 }
 
 // ------------------------------------------------------ Hamiltonian build
@@ -1533,6 +1922,40 @@ __device__ void tp_eval(const double* A, const double* in, double* t1, double* t
   __syncthreads();
 }
 
+// Transpose: in [Q][Q][Q][NC] -> out [N1][N1][N1][NC] (integration against N).
+template <int N1, int Q, int NC>
+__device__ void tp_integrate(const double* A, const double* in, double* t1, double* t2,
+                             double* out) {
+  const int tid = threadIdx.x;
+  for (int i = tid; i < Q * Q * N1 * NC; i += kThreads) {  // t1[qz][qy][a][col]
+    const int col = i % NC, a = (i / NC) % N1, qzy = i / (NC * N1);
+    const double* src = in + qzy * Q * NC + col;
+    double s = 0.0;
+#pragma unroll
+    for (int qx = 0; qx < Q; ++qx) s += A[qx * N1 + a] * src[qx * NC];
+    t1[i] = s;
+  }
+  __syncthreads();
+  for (int i = tid; i < Q * N1 * N1 * NC; i += kThreads) {  // t2[qz][b][a][col]
+    const int col = i % NC, a = (i / NC) % N1, b = (i / (NC * N1)) % N1, qz = i / (NC * N1 * N1);
+    const double* src = t1 + (qz * Q * N1 + a) * NC + col;
+    double s = 0.0;
+#pragma unroll
+    for (int qy = 0; qy < Q; ++qy) s += A[qy * N1 + b] * src[qy * N1 * NC];
+    t2[i] = s;
+  }
+  __syncthreads();
+  for (int i = tid; i < N1 * N1 * N1 * NC; i += kThreads) {  // out[c][b][a][col]
+    const int col = i % NC, ba = (i / NC) % (N1 * N1), c = i / (NC * N1 * N1);
+    const double* src = t2 + ba * NC + col;
+    double s = 0.0;
+#pragma unroll
+    for (int qz = 0; qz < Q; ++qz) s += A[qz * N1 + c] * src[qz * N1 * N1 * NC];
+    out[i] = s;
+  }
+  __syncthreads();
+}
+
 template <int N1, int Q, int NC>
 struct TpScratch {
   static constexpr int kIn = (N1 * N1 * N1 > Q * Q * Q ? N1 * N1 * N1 : Q * Q * Q) * NC;
@@ -1580,6 +2003,47 @@ __global__ __launch_bounds__(kThreads) void k_density(Geo g, const double* __res
     __syncthreads();
   }
   for (int q = tid; q < NQ; q += kThreads) rho[e * NQ + q] = acc[q];
+}
+
+// --------------------------------------------- quadrature cell operator
+// Y += N^T diag(wq) N X on the cells of one colour (no write conflicts): the
+// quadrature operator of an adjoint solve's right-hand side, whose order of sums is
+// fixed as that of the solve's steps is (see k_cell_line).  8 launches, 2.18 ms at
+// 121^3 nodes x 12 columns, once per solve; launch_quad_pairs takes 0.3 ms there.
+template <int P, int NC>
+__global__ __launch_bounds__(kThreads) void k_quad_operator(Geo g, const double* __restrict__ Lq,
+                                                            const double* __restrict__ X, int B,
+                                                            const double* __restrict__ wq,
+                                                            double* __restrict__ Y, int colour,
+                                                            int64_t nw) {
+  constexpr int N1 = P + 1, Q = P + 3, NE = ne_of(P), NQ = Q * Q * Q;
+  typedef TpScratch<N1, Q, NC> Sz;
+  __shared__ double A[Q * N1];
+  __shared__ double sin_[Sz::kIn], t1[Sz::kT1], t2[Sz::kT2], sout[Sz::kOut];
+  __shared__ int64_t nodes[NE];
+  const int64_t e = colour_cell(g, colour, blockIdx.x, nw);
+  if (e < 0) return;
+  const int64_t cx = e % g.nc, cy = (e / g.nc) % g.nc, cz = e / ((int64_t)g.nc * g.nc);
+  const int tid = threadIdx.x;
+  for (int i = tid; i < Q * N1; i += kThreads) A[i] = Lq[i];
+  for (int l = tid; l < NE; l += kThreads) nodes[l] = cell_node(g, cx, cy, cz, l);
+  __syncthreads();
+  for (int j0 = 0; j0 < B; j0 += NC) {
+    for (int i = tid; i < NE * NC; i += kThreads) {
+      const int l = i / NC, j = j0 + i % NC;
+      sin_[i] = j < B ? X[nodes[l] * B + j] : 0.0;
+    }
+    __syncthreads();
+    tp_eval<N1, Q, NC>(A, sin_, t1, t2, sout);
+    for (int i = tid; i < NQ * NC; i += kThreads) sout[i] *= wq[e * NQ + i / NC];
+    __syncthreads();
+    tp_integrate<N1, Q, NC>(A, sout, t1, t2, sin_);
+    for (int i = tid; i < NE * NC; i += kThreads) {
+      const int l = i / NC, j = j0 + i % NC;
+      if (j < B) Y[nodes[l] * B + j] += sin_[i];
+    }
+    __syncthreads();
+  }
 }
 
 // ------------------------------------------------------------ v_xc -> quad
@@ -1721,8 +2185,7 @@ __global__ void k_lincomb_mixed(uint32_t NB, uint32_t B, TY* Y, const TX* X, dou
   }
 }
 
-template <typename T>
-__global__ void k_scale_product(int64_t n, double* __restrict__ y, const T* __restrict__ a,
+__global__ void k_scale_product(int64_t n, double* __restrict__ y, const float* __restrict__ a,
                                 const double* __restrict__ b) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) y[i] = (double)a[i] * b[i];
@@ -2181,12 +2644,19 @@ __global__ __launch_bounds__(kRedThreads) void k_minres_givens(int B, int nblk,
   if (nq >= 3) {  // fused steps: [k][column][block] partials, the three sums in one pass
     const double* p = partial + (int64_t)j * nblk;
     const int64_t row = (int64_t)B * nblk;
-    s = 0.0;
-    for (int b = threadIdx.x; b < nblk; b += kRedThreads) {
-      s += p[b];
-      q2 += p[row + b];
-      q3 += p[2 * row + b];
-    }
+    double a[3][4] = {};  // in block_sum_contig's order
+    int b = threadIdx.x;
+    for (; b + 3 * kRedThreads < nblk; b += 4 * kRedThreads)
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) a[k][u] += p[k * row + b + u * kRedThreads];
+    for (; b < nblk; b += kRedThreads)
+#pragma unroll
+      for (int k = 0; k < 3; ++k) a[k][0] += p[k * row + b];
+    s = (a[0][0] + a[0][1]) + (a[0][2] + a[0][3]);
+    q2 = (a[1][0] + a[1][1]) + (a[1][2] + a[1][3]);
+    q3 = (a[2][0] + a[2][1]) + (a[2][2] + a[2][3]);
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
       s += __shfl_xor(s, o, 64);
@@ -2496,9 +2966,9 @@ void launch_build_hamiltonian(const Geo& g, const DevTables& t, double hh, const
   IDFT_HIP(hipGetLastError());
 }
 
-// The sum-factorised kernel takes any block width in one way; its shape arguments
-// (columns per work-group 2, 4 or 8, one column per item) are accepted and change
-// nothing.
+// Columns per work-group (2, 4 or 8: 40.7 KB of LDS at 8, p = 5) of the line-by-line
+// kernel of the FP64 MINRES steps, one column per item; the plane kernel takes any
+// block width in one way.
 bool sf_cols_supported(int cols, bool) { return cols == 2 || cols == 4 || cols == 8; }
 bool sf_vc_supported(int cols, int vc, bool fp64) {
   return sf_cols_supported(cols, fp64) && vc == 1;
@@ -2520,6 +2990,17 @@ static void cell_plane(const Geo& g, T hq, const T* W, uint32_t wstride,
       sf_eo_table(P));
 }
 
+template <int P, int CG>
+static void cell_line(const Geo& g, const CellOp<double>& op, const double* S, const double* X,
+                      const double* xn, const double* xcol, double* Yc, int B, double* dotp,
+                      hipStream_t s) {
+  check_u32(cell_scratch_elems(g, B));
+  const int64_t npair = g.ncell * ((B + CG - 1) / CG);
+  check_u32(8 * ((npair + 7) / 8));
+  k_cell_line<P, CG><<<(unsigned)(8 * ((npair + 7) / 8)), kThreads, 0, s>>>(
+      g, op.kin_scale, op.W, S, X, xn, xcol, Yc, B, dotp, sf_eo_table(P));
+}
+
 template <typename T, typename TV, int P>
 static void cell_sf_p(const Geo& g, const CellOp<T>& op, const T* S, const TV* X,
                       const double* xn, const double* sxn, const double* xcol, T* Yc, int B,
@@ -2533,8 +3014,19 @@ static void cell_sf_p(const Geo& g, const CellOp<T>& op, const T* S, const TV* X
   // per-cell dots only with node-scaled inputs (the MINRES steps)
   if (dotp && !xn) throw Error(IDFT_EINVAL, "per-cell dots need a node-scaled input");
   // node-scaled inputs (MINRES) come as FP64 vectors; FP32 vectors never
-  // carry a node scale
-  if constexpr (std::is_same<TV, double>::value) {
+  // carry a node scale.  In FP64 they take the line-by-line kernel, whose order of
+  // sums a solve keeps; FP32 products decide no iterate to 64-bit rounding (the
+  // sweeps that refine it do), and the plane kernel is 1.1 to 4 times faster there.
+  if constexpr (std::is_same<T, double>::value) {
+    if (xn) {
+      switch (cg) {
+        case 2: cell_line<P, 2>(g, op, S, X, xn, xcol, Yc, B, dotp, s); break;
+        case 4: cell_line<P, 4>(g, op, S, X, xn, xcol, Yc, B, dotp, s); break;
+        default: cell_line<P, 8>(g, op, S, X, xn, xcol, Yc, B, dotp, s); break;
+      }
+      return;
+    }
+  } else if constexpr (std::is_same<TV, double>::value) {
     if (xn) {
       if (!sxn) throw Error(IDFT_EINVAL, "node-scaled input without the product of its scales");
       cell_plane<T, TV, P, true, true>(g, hq, op.W, nq, sxn, X, B, xcol, Yc, B, dotp, s);
@@ -2904,15 +3396,10 @@ void launch_lincomb_df2d(int64_t N, int B, double* Y, const double* X, double a,
       (uint32_t)(N * B), (uint32_t)B, Y, X, a, ca, Z, b, cb);
   IDFT_HIP(hipGetLastError());
 }
-template <typename T>
-void launch_scale_product(int64_t n, double* y, const T* a, const double* b, hipStream_t s) {
-  k_scale_product<T><<<(unsigned)((n + 255) / 256), 256, 0, s>>>(n, y, a, b);
+void launch_scale_product(int64_t n, double* y, const float* a, const double* b, hipStream_t s) {
+  k_scale_product<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(n, y, a, b);
   IDFT_HIP(hipGetLastError());
 }
-template void launch_scale_product<double>(int64_t, double*, const double*, const double*,
-                                           hipStream_t);
-template void launch_scale_product<float>(int64_t, double*, const float*, const double*,
-                                          hipStream_t);
 void launch_convert_d2f(int64_t n, float* y, const double* x, hipStream_t s) {
   k_d2f<<<grid_for(n), kThreads, 0, s>>>(n, y, x);
   IDFT_HIP(hipGetLastError());
@@ -3021,6 +3508,21 @@ void launch_loss(int64_t nQ, int nq, const double* rho, const double* rhoT, cons
                  const double* veff, const double* jxw, double* u, double* partial,
                  hipStream_t s) {
   k_loss<<<256, kThreads, 0, s>>>(nQ, nq, rho, rhoT, w, veff, jxw, u, partial);
+  IDFT_HIP(hipGetLastError());
+}
+
+void launch_quad_operator(const Geo& g, const DevTables& t, const double* X, int B,
+                          const double* wq, double* Y, int colour, hipStream_t s) {
+  const int64_t nw = colour_count(g, colour);
+  if (nw == 0) return;
+  dim3 grid(colour_grid(nw)), block(kThreads);
+  switch (g.p) {
+    case 2: k_quad_operator<2, 8><<<grid, block, 0, s>>>(g, t.Lq.p, X, B, wq, Y, colour, nw); break;
+    case 3: k_quad_operator<3, 8><<<grid, block, 0, s>>>(g, t.Lq.p, X, B, wq, Y, colour, nw); break;
+    case 4: k_quad_operator<4, 8><<<grid, block, 0, s>>>(g, t.Lq.p, X, B, wq, Y, colour, nw); break;
+    case 5: k_quad_operator<5, 8><<<grid, block, 0, s>>>(g, t.Lq.p, X, B, wq, Y, colour, nw); break;
+    default: throw Error(IDFT_EINVAL, "degree not supported");
+  }
   IDFT_HIP(hipGetLastError());
 }
 
