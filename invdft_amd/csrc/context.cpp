@@ -17,6 +17,7 @@
 #include <rocblas/rocblas.h>
 
 #include "common.h"
+#include "host_rules.h"
 #include "setup.h"
 #include "sf_tables.h"
 
@@ -967,6 +968,31 @@ struct idft_ctx {
   }
 
   // ------------------------------------------------------------ MINRES
+  // The five further Lanczos vectors of n elements of a batch of steps, or none of
+  // them: not where memory is what the caller saves (psi_checkpoint), nor where they
+  // would take more than an eighth of the free memory (other contexts may need it by
+  // the time that this solve ends), nor where an allocation fails all the same.
+  static constexpr size_t kKeptBatchBytes = (size_t)64 << 20;
+  bool take_batch_vectors(size_t n) {
+    constexpr int nq = kMinresBatch - 3;
+    if (!d.psi_checkpoint && mw64.q[nq - 1].n >= n) return true;
+    for (auto& q : mw64.q) q.release();  // those of a smaller block
+    if (d.psi_checkpoint) return false;
+    size_t freeB = 0, totalB = 0;
+    IDFT_HIP(hipMemGetInfo(&freeB, &totalB));
+    if (nq * n * sizeof(double) > freeB / 8) return false;
+    if (resize_all_or_none<Error>(mw64.q, nq, n)) return true;
+    (void)hipGetLastError();  // the failed allocation's, which the next launch would report
+    return false;
+  }
+  // Given back after a solve unless they are few: allocating and freeing 567 MB (24
+  // cells p = 5, 8 columns) or 10.7 GB (40 cells p = 4, 64 columns) in each solve is
+  // within the runs' differences (281 and 360 ms); of a solve of 1 ms it would show.
+  void drop_batch_vectors() {
+    if ((kMinresBatch - 3) * mw64.q[0].n * sizeof(double) > kKeptBatchBytes)
+      for (auto& q : mw64.q) q.release();
+  }
+
   // Preconditioned MINRES (FP64 recurrence) from x = 0 (x accumulates), per-
   // column tolerance.  relax > 0 (MIXED): the FP64 cell operator is applied
   // until every open column's residual estimate phibar is below relax times
@@ -1025,24 +1051,16 @@ struct idft_ctx {
       const int nb = launch_coldot_partial<double>(N, b, r1, r1, Djac.p, partial.p, s);
       launch_minres_start(b, nb, partial.p, adj.dnegEig.p, mst.p, s);
     }
+    Yc64.resize(cell_scratch_elems(g, b));
+    if (canRelax) Yc32.resize(cell_scratch_elems(g, b));
     // Lanczos vectors that a batch of fused steps keeps: y (which fused steps do
-    // not use otherwise) and up to five more, taken only where they leave half of
-    // the free memory and not where memory is what the caller saves
-    // (psi_checkpoint)
+    // not use otherwise) and five more if they are to be had, after everything
+    // that the solve cannot do without
     std::vector<double*> vb;
     if (fused) {
       mhist.resize((size_t)kMinresBatch * 4 * b);
       vb.push_back(W.y.p);
-      constexpr int nq = kMinresBatch - 3;
-      bool more = !d.psi_checkpoint;
-      if (more && W.q[nq - 1].n < NB(b)) {
-        size_t freeB = 0, totalB = 0;
-        IDFT_HIP(hipMemGetInfo(&freeB, &totalB));
-        more = nq * NB(b) * sizeof(double) <= freeB / 2;
-        if (more)
-          for (auto& q : W.q) q.resize(NB(b));
-      }
-      if (more)
+      if (take_batch_vectors(NB(b)))
         for (auto& q : W.q) vb.push_back(q.p);
     }
     const int batch = (int)vb.size() + 2;
@@ -1153,8 +1171,6 @@ struct idft_ctx {
     // (kernels only: no memset or copy nodes); the apply scratch is sized
     // before capture.
     const bool useGraph = d.minres_graph != 0 && check % 2 == 0;
-    Yc64.resize(cell_scratch_elems(g, b));
-    if (canRelax) Yc32.resize(cell_scratch_elems(g, b));
     // graphs per (operator precision, place of r2 at the run's start)
     hipGraphExec_t execs[4] = {nullptr, nullptr, nullptr, nullptr};
     struct ExecGuard {
@@ -1368,6 +1384,7 @@ struct idft_ctx {
     }
     st.minres_iters_max = std::max(st.minres_iters_max, mx);
     st.minres_iters_total += tot;
+    drop_batch_vectors();
     if (distribute) distribute_x();
     sync();
   }
