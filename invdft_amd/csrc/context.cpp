@@ -972,7 +972,7 @@ struct idft_ctx {
   // them: not where memory is what the caller saves (psi_checkpoint), nor where they
   // would take more than an eighth of the free memory (other contexts may need it by
   // the time that this solve ends), nor where an allocation fails all the same.
-  static constexpr size_t kKeptBatchBytes = (size_t)64 << 20;
+  static constexpr size_t kKeptBatchBytes = (size_t)1 << 30;
   bool take_batch_vectors(size_t n) {
     constexpr int nq = kMinresBatch - 3;
     if (!d.psi_checkpoint && mw64.q[nq - 1].n >= n) return true;
@@ -985,9 +985,9 @@ struct idft_ctx {
     (void)hipGetLastError();  // the failed allocation's, which the next launch would report
     return false;
   }
-  // Given back after a solve unless they are few: allocating and freeing 567 MB (24
-  // cells p = 5, 8 columns) or 10.7 GB (40 cells p = 4, 64 columns) in each solve is
-  // within the runs' differences (281 and 360 ms); of a solve of 1 ms it would show.
+  // Given back after a solve above 1 GiB: allocating 10.7 GB in each solve does not show
+  // (40 cells p = 4, 64 columns: 360 ms), but 567 MB in each force evaluation of 24 cells
+  // p = 5, 8 columns, took 2.4 of 277 ms.
   void drop_batch_vectors() {
     if ((kMinresBatch - 3) * mw64.q[0].n * sizeof(double) > kKeptBatchBytes)
       for (auto& q : mw64.q) q.release();
