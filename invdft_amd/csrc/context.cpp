@@ -716,10 +716,8 @@ struct idft_ctx {
                                  const double* wq, int64_t wstride, double* T2) {
     const int np = (int)adj.pairs.size() / 2;
     if (np == 0 && !T2) return {};
-    // columns per pass: all, unless the cell kernel's width or the 32-bit index
-    // of the cell scratch bounds them
     const int64_t fit = ((int64_t)0xffffffffLL - 1) / cell_scratch_elems(g, 1);
-    const int w = (int)std::min<int64_t>(std::min(b, kMaxCols), std::max<int64_t>(fit, 1));
+    const int w = quad_slice(b, kMaxCols, fit);
     const bool fused = w == b && np <= 256;
     if (!fused && !T2 && np) {
       T2buf.resize(NB(b));

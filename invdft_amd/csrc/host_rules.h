@@ -1,6 +1,8 @@
 // Rules of the host code that need no device: tested on the CPU.
 #pragma once
+#include <algorithm>
 #include <cstddef>
+#include <cstdint>
 
 namespace idft {
 
@@ -16,6 +18,14 @@ bool resize_all_or_none(Buf* bufs, int n, size_t count) {
     for (int i = 0; i < n; ++i) bufs[i].release();
     return false;
   }
+}
+
+// Columns per pass over a block of b columns where the cell kernel takes at most
+// `cols` and the 32-bit index of the cell scratch `fit`: b if it fits, otherwise even
+// (the gather stores two columns at a time where a row starts at an even column), or 1.
+inline int quad_slice(int b, int cols, int64_t fit) {
+  const int w = (int)std::min<int64_t>(std::min(b, cols), std::max<int64_t>(fit, 1));
+  return w < b && w > 1 ? w - w % 2 : w;
 }
 
 }  // namespace idft

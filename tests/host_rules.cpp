@@ -30,5 +30,8 @@ int main() {
     for (const Buf& x : b) std::printf(" %zu", x.n);
     std::printf("\n");
   }
+  for (int b = 1; b <= 80; ++b)
+    for (int fit : {0, 1, 2, 3, 7, 16, 33, 79, 80, 1000})
+      std::printf("slice %d %d %d\n", b, fit, idft::quad_slice(b, 80, fit));
   return 0;
 }

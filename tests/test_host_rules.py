@@ -30,3 +30,20 @@ def test_optional_workspace_is_whole_or_absent(rules):
             assert not ok and sizes == [0] * 5
         else:
             assert ok and sizes == [64, 64, 64, 70, 64]
+
+
+def test_column_slices_start_at_even_columns(rules):
+    """Slices of an even block start at even columns, so that 16-byte accesses stay
+    aligned, and fit the scratch; a block that fits is one slice."""
+    n = 0
+    for f in rules:
+        if f[0] != "slice":
+            continue
+        b, fit, w = (int(v) for v in f[1:])
+        n += 1
+        assert 1 <= w <= min(b, max(fit, 1))
+        if b <= fit:
+            assert w == b
+        elif b % 2 == 0 and w > 1:
+            assert all(j % 2 == 0 for j in range(0, b, w)), (b, fit, w)
+    assert n == 800
