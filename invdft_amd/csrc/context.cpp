@@ -118,6 +118,8 @@ struct idft_ctx {
   DevBuf<double> lanBuf, lanSt;  // Lanczos bound: three vectors, the scalars
   DevBuf<double> mst, mx, mtmp, mnegc, mcell, mhist, pairCoef;
   DevBuf<int> mflags, msel, pairList;
+  std::vector<double> pairCoefHost;  // sources of pairCoef's and pairList's uploads, which
+  std::vector<int> pairListHost;     // the callers of pair_lists wait for
   idft_mv mvPsi, mvX;
 
   // rocBLAS handle on s (created on first use), for the Gram and X Q products
@@ -767,7 +769,7 @@ struct idft_ctx {
   // k with C[k][i]) that is zero outside the adjoint's pairs, either way round;
   // uploaded for k_pair_combine.  Returns the entry count, or -1 if a dense
   // product is the better one: more than kSparsePairs entries per column on
-  // average.
+  // average.  The uploads read the host lists until the caller's next sync().
   static constexpr int kSparsePairs = 8;
   int pair_lists(const std::vector<double>& C, int b) {
     std::vector<char> used((size_t)b * b, 0);
@@ -778,8 +780,11 @@ struct idft_ctx {
         if (!used[e] && C[e] != 0.0) { used[e] = 1; ++nnz; }
     }
     if (nnz > kSparsePairs * b || b > 2 * kMaxCols) return -1;
-    std::vector<double> coef;
-    std::vector<int> list((size_t)b + 1, 0), rows;
+    std::vector<double>& coef = pairCoefHost;
+    std::vector<int>& list = pairListHost;
+    std::vector<int> rows;
+    coef.clear();
+    list.assign((size_t)b + 1, 0);
     for (int i = 0; i < b; ++i) {
       for (int k = 0; k < b; ++k)
         if (used[(size_t)k * b + i]) {
