@@ -769,7 +769,9 @@ struct idft_ctx {
   // k with C[k][i]) that is zero outside the adjoint's pairs, either way round;
   // uploaded for k_pair_combine.  Returns the entry count, or -1 if a dense
   // product is the better one: more than kSparsePairs entries per column on
-  // average.  The uploads read the host lists until the caller's next sync().
+  // average.  computeRhs, sparse and dense, us: 24 cells p = 5 B = 12, 7 entries per
+  // column 487 and 537, 12 entries 548 and 540; B = 32, 7 entries 1188 and 1459, 15
+  // entries 1392 and 1454, 23 entries 2616 and 2615.  The uploads read the host lists until the caller's next sync().
   static constexpr int kSparsePairs = 8;
   int pair_lists(const std::vector<double>& C, int b) {
     std::vector<char> used((size_t)b * b, 0);
@@ -1118,10 +1120,10 @@ struct idft_ctx {
     bool swapped = false;  // r2 and the spare buffer have changed places
     // A small block copies the newest vector back into r2's place, 2 streams per
     // batch, so that every run has the same arguments and one graph replays from the
-    // second run on; a large one exchanges the two buffers (and captures two graphs,
-    // from the fifth run on).  At 15625 nodes x 4 columns launching the first four
-    // runs directly cost 5 % of a force evaluation; from 32 MB per vector on, two
-    // streams take longer than a capture saves.
+    // second run on; a large one exchanges the two buffers and captures two graphs.
+    // Copying against exchanging, us for 96 steps: 2640 and 2808 at 0.06 M entries,
+    // 6937 and 6967 at 1.65 M, 7493 and 7584 at 2.13 M; 11666 and 11561 at 4.25 M,
+    // 19826 and 19639 at 7.1 M, 53199 and 52331 at 21 M.
     const bool copyBack = NB(b) < (size_t)4 << 20;
     auto batch_steps = [&](int n) {
       MinresVectors rs{};
@@ -1267,8 +1269,8 @@ struct idft_ctx {
       }
       const int n = std::min(check, maxit - k);
       st.minres_column_steps += (int64_t)n * bc;
-      // the first runs of a block are launched directly, the ones after them replay
-      if (useGraph && n == check && (runs >= (copyBack ? 1 : 4) || !fused)) {
+      // the first run of a block is launched directly, the ones after it replay
+      if (useGraph && n == check && (runs >= 1 || !fused)) {
         hipGraphExec_t& exec = execs[(f32op ? 1 : 0) + (swapped ? 2 : 0)];
         if (!exec) {
           hipGraph_t graph = nullptr;

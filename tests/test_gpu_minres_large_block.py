@@ -37,8 +37,7 @@ def _solve(glib, inputs, b, steps, **kw):
 
 
 # runs of check_every steps, more than six of them so that both graphs are captured
-# (fifth and sixth run) and replayed, then a shorter run: one batch of 2, 6 and 7 + 7
-# steps; with at most 3 steps a batch (psi_checkpoint) 3 + 3 + 2 and 2 + 2, an odd and
+# and replayed, then a shorter run: one batch of 2, 6 and 7 + 7 steps; with at most 3 steps a batch (psi_checkpoint) 3 + 3 + 2 and 2 + 2, an odd and
 # an even number of exchanges; the last run of the first case is one step long
 @pytest.mark.parametrize("b,check_every,steps,ckpt", [(5, 2, 17, 0), (6, 6, 50, 0), (5, 14, 114, 0),
                                                       (6, 8, 67, 1), (5, 4, 33, 1)])
