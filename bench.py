@@ -581,8 +581,8 @@ def main():
 
     # The dominant kernel of the mixed iteration is the FP32 cell product of
     # the Chebyshev filter (the largest share of kernel time in the iteration
-    # trace); the FP64 cell product of the MINRES steps and Rayleigh-Ritz is
-    # reported beside it.
+    # trace in single precision); the FP64 one of Rayleigh-Ritz is reported
+    # beside it.  The FP64 MINRES steps run another kernel (k_cell_line).
     ms_op32, ms_cell32 = cm.profile_apply(B, abi.MIXED, reps=20)
     roof = roofline(mixed["tuned"]["fp32"], True, ms_cell32, ms_op32)
     ms_op64, ms_cell64 = cm.profile_apply(B, abi.FP64, reps=20)

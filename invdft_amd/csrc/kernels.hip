@@ -1164,9 +1164,9 @@ __global__ __launch_bounds__(64, 2) void k_cell_plane(
 // contraction of the tensor along a line of the cell, with the input scaled on the
 // fly and the cell's dots x.(H_e x).  An iterate that a step limit stops is not
 // determined by its inputs in 64 bits: once a Ritz value has converged the Lanczos
-// vectors amplify rounding (two orders of the same sums gave iterates 1e-8 to 1e-2
-// apart after 30 to 64 steps on meshes of 17 to 63 nodes per axis, and 1e-14 apart
-// on 100).  So the steps keep one order of arithmetic, this one, and an iterate
+// vectors amplify rounding (two orders of the same sums gave iterates 1e-8 to 3e-2
+// apart after 32 to 64 steps on meshes of 25 to 63 nodes per axis, 1e-15 to 1e-10 on
+// 91 to 115).  So the steps keep one order of arithmetic, this one, and an iterate
 // stopped after k steps stays what it has been; its price is the plane kernel's
 // gain in FP64 solves (24 cells p = 5 B = 12: 261 against 233 us, 30 p = 4 B = 64:
 // 1383 against 1139).  Do not regroup a sum here.

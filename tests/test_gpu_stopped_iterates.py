@@ -1,7 +1,7 @@
 """MINRES iterates that a step limit stops, against fixed values (gfx950 only).
 
 Once a Ritz value has converged, rounding decides such an iterate: two orders of the
-same sums give solutions 1e-8 to 1e-2 apart here, so no other arithmetic can be the
+same sums give solutions 6e-9 to 1e-5 apart here, so no other arithmetic can be the
 reference.  The FP64 steps and their right-hand side keep one order of sums instead,
 and tests/golden/stopped_iterates.npz holds its values (golden/make_stopped_iterates.py).
 """
